@@ -360,6 +360,20 @@ def alg_bytes(physics, n, halo, e, nts, S, variant=(0, 0)):
         else:
             # CD: r p^n, p^n-1, fact; w p^n+1 (4e); + w D (5e).  Adjoint with
             # the fused correlation: + r D, grad read-modify-write (7e).
+            if physics == "cd2d" and len(variant) > 1 and variant[1] > 22:
+                # n levels per launch: a launch reads p^n, p^n-1 and fact once
+                # (3e), writes the two last levels (2e) and the D of every
+                # stored level (1e); an adjoint launch also reads and writes
+                # the gradient (2e) and reads one history level per level.
+                # Launches end at multiples of S.
+                n = variant[1] % 10
+                lf = sum(-(-(min((k + 1) * S, nt) - k * S) // n) for k in range(kl + 1))
+                lr = kl * -(-S // n)
+                fwd_b += (lf + lr) * (5 * e * N + strip) + (last + rep) * e * N
+                fwd_n += lf + lr
+                adj_b += lf * (7 * e * N + strip) + nt * e * N
+                adj_n += lf
+                continue
             if physics == "cd2d" and len(variant) > 1 and variant[1] % 10 == 2:
                 # two levels per forward / replay launch: r p^n, p^n-1, fact
                 # once per launch (3e), w each level (1e) and its D (1e);
@@ -446,7 +460,12 @@ def kernel_names(physics, variant):
         else:
             k = f"cd3d_step_kernel<float, {v}, 0>"
         return f"{k} (forward)", f"{k} (adjoint)"
-    # [rows per thread, levels per launch: 10 x adjoint + forward / replay]
+    # [rows per thread or window shapes, levels per launch; each but the rows
+    # 10 x adjoint + forward / replay]
+    if len(variant) > 1 and variant[1] > 22:
+        shape = {0: "8, 8", 1: "4, 16", 2: "2, 16"}
+        return (f"cd2d_stepn_kernel<float, {shape[variant[0] % 10]}, false> (forward)",
+                f"cd2d_stepn_kernel<float, {shape[variant[0] // 10]}, true> (adjoint)")
     k = f"cd2d_step_kernel<float, {variant[0] or 2}>"
     two = variant[1] if len(variant) > 1 else 0
     fwd = "cd2d_step2_kernel<float, false>" if two % 10 == 2 else k

@@ -159,7 +159,8 @@ typedef struct {
    * 308/316/332 one launch, 102/104 z-marching strips; + 1000 k: shots in
    * groups of 2^k in the block order); elastic [forward, adjoint] variant
    * codes (0/1 stress and displacement launches, 2 one fused launch); CD 2D
-   * [rows per thread, 10 x adjoint + forward levels per launch]; CD 3D
+   * [window shapes (or, with one level per launch, rows per thread), most
+   * levels per launch], each 10 x adjoint + forward; CD 3D
    * [launch shape 8/4/2/108/104/102/208/204/202, planes per z chunk]; 0
    * where there is one shape. */
   int32_t kernel_variant[2];

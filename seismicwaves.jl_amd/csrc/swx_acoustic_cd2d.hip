@@ -9,11 +9,11 @@
 //   correlate  src/models/acoustic/backends/shared/correlate_gradient_xPU.jl:1-10
 //
 // Device layout (x fastest, exactly the Julia layout), one slab per shot:
-//   p      [4][ns][nx*nz]  time levels, p^k lives in slot k mod 4 (the
-//                          reference swaps pold/pcur/pnew, :122-124; a
-//                          fourth slot lets a launch step two levels)
-//   psi_x  [3][ns][2h*nz]  level k in buffer k mod 3, so a cell can
-//   psi_z  [3][ns][nx*2h]  recompute its left neighbour's new value
+//   p      [4][ns][nx*nz]  the two last time levels and the slots of the
+//                          next two (the reference swaps pold/pcur/pnew,
+//                          :122-124)
+//   psi_x  [3][ns][2h*nz]  the last level and free buffers for the next, so a
+//   psi_z  [3][ns][nx*2h]  cell can recompute its left neighbour's new value
 //   xi_x   [3][ns][(2h+2)*nz], xi_z [3][ns][nx*(2h+2)]
 //   (the adjoint state is laid out the same way)
 //   D      [S][ns][nx*nz]  p^{it-2} - 2 p^{it-1} + p^{it} of the segment
@@ -286,357 +286,476 @@ __global__ __launch_bounds__(TX *TZ) void cd2d_step_kernel(Cd2dStepArgs<T> a) {
 }
 
 // ---------------------------------------------------------------------------
-// Two forward / replay levels per launch (cd2d_step2_kernel).
+// Up to SN_MAX levels per launch (cd2d_stepn_kernel).
 //
-// A launch at it steps the levels it and it+1.  A block owns a TX x H tile
-// (H = TZ * 2 rows) and computes level it on the tile plus a one-cell ring
-// (its "region", kept in LDS with the level-it C-PML memory variables),
-// then level it+1 on the tile from the region.  The ring cells belong to
-// the neighbouring tiles, whose blocks compute them as well; only the
-// owning block writes a cell.  Because a block reads levels it-1 and it-2
-// of the ring while its neighbours write levels it and it+1, the forward
-// state keeps four pressure levels (slot k mod 4) and three levels of the
-// C-PML memory variables (buffer k mod 3).  Every cell update is the
-// expression of cd2d_cell / cd2d_lean_cells in the same operand order, so
-// the results are bitwise those of two one-level launches.
+// A block of NW waves loads a 64 x (NW R) window of the two last levels
+// into registers (lane = column, R rows per wave) and steps it n times; the
+// window's valid part shrinks by one cell per level and side, so the block
+// owns, and writes, the cells at least n from the window's sides (all cells
+// up to a side that is the grid's).  x neighbours come from the adjacent
+// lanes, z neighbours from the thread's own rows; only the first and last row
+// of each wave pass through LDS, with one barrier per level.  The C-PML
+// memory variables of the window's strip cells step along in registers, and
+// in the adjoint the gradient of the owned cells, with the forward history
+// loaded two levels ahead.  Point values of the n levels are staged in LDS
+// once.  Every cell update is spelled as in cd2d_cell, so the results are
+// bitwise those of n one-level launches.
+//
+// Bound by latency at small sizes (a launch of 8 levels of one 201 x 151 shot
+// takes 17 us: 5-7 us of loads, stores and launch, 1.3 us per level of barrier,
+// LDS round trip and the strip updates' chain) and by instruction issue at
+// large ones (about 20 vector instructions per cell and level, 1.5-1.8 times
+// the grid's cells).  us per level against the two-level LDS tiles this
+// replaces (one level per launch where that was faster):
+//   f32 201 x 151:        forward 5.1 -> 2.2, adjoint + replay   8.9 -> 3.7
+//   f32 1000 x 1000:      forward 7.9 -> 3.9, adjoint + replay  15.9 -> 7.2
+//   f64 12 x 397 x 253:   forward  15 -> 6.2, adjoint + replay    33 -> 13
 
-constexpr int S2H = TZ * 2;          // tile rows
-constexpr int S2W = TX + 2;          // region columns (tile + ring)
-constexpr int S2R = S2H + 2;         // region rows
-constexpr int S2N = S2W * S2R;       // region cells
-constexpr int S2Q = (S2N + TX * TZ - 1) / (TX * TZ);   // region cells per thread
+constexpr int SN_MAX = 8;        // most levels per launch
+constexpr int SN_SLOTS = 126;    // staged point values per level
+constexpr int SN_RECS = 254;     // receivers whose traces are kept
 
-// Replay-history slot of level itl for shot s (or -1).
 template <typename T>
-__device__ __forceinline__ int cd2d_dslot(const Cd2dStepArgs<T> &a, int nts, int itl) {
-  if (a.dmode == 1) {
-    const int seg0 = ((nts - 1) / a.S) * a.S;
-    return itl > seg0 ? itl - seg0 - 1 : -1;
-  }
-  return a.dmode == 2 ? itl - a.cbase - 1 : -1;
-}
-
-// Results of one cell update (cd2d_cell's, without the stores).
-template <typename T>
-struct Cd2dCell {
-  T pnv, dval, psx, psz, xix, xiz;
-  int kx, kz;
-  bool xup, zup;   // xi_x / xi_z updated
+struct Cd2dStepNArgs {
+  Cd2dStepArgs<T> a;   // a.it: first level; a.pnew: the last level stepped
+  T *pnew0;            // the level before it (n >= 2)
+  int n;               // levels
 };
 
-// cd2d_cell's update of cell (i, j) at level itl (forward: sources;
-// ADJ: the prescaled residuals),
-// reading the current level through pc(di, dj), the old C-PML memory
-// variables through psxo(cell i, strip k) / pszo(cell j, strip k) and
-// xixo() / xizo() (the cell's own xi).
-template <typename T, bool ADJ, typename PC, typename PSX, typename PSZ, typename XIX, typename XIZ>
-__device__ __forceinline__ Cd2dCell<T> cd2d_cell_eval(const Cd2dStepArgs<T> &a, int s, int nts, int itl, int i,
-                                                      int j, PC pc_at, T pov, T fa, PSX psxo, PSZ pszo, XIX xixo,
-                                                      XIZ xizo) {
-  const int nx = a.nx, nz = a.nz, h = a.h;
-  const int64_t c = (int64_t)j * nx + i;
-  const bool interior = (i >= 1 && i <= nx - 2 && j >= 1 && j <= nz - 2);
-  const T pc = pc_at(0, 0);
-  const T pl = interior ? pc_at(-1, 0) : T(0), pr = interior ? pc_at(1, 0) : T(0);
-  const T pd = interior ? pc_at(0, -1) : T(0), pu = interior ? pc_at(0, 1) : T(0);
-  const T *cb = a.cpml + (int64_t)s * a.cstride;
-  const AxisCoef<T> cx = axis_coef(cb, h, 0);
-  const AxisCoef<T> cz = axis_coef(cb, h, 1);
-  Cd2dCell<T> o;
-  o.kx = -1;
-  if (i < h) o.kx = i;
-  else if (i >= nx - h - 1 && i <= nx - 2) o.kx = i + 1 - nx + 2 * h;
-  o.psx = 0;
-  if (o.kx >= 0) {
-    const T d = (pc_at(1, 0) - pc) * a.idx;
-    o.psx = cx.bh(o.kx) * psxo(i, o.kx) + cx.ah(o.kx) * d;
+// Value of the lane before / after (0 beyond the wave's ends).
+template <int CTRL>
+__device__ __forceinline__ float lane_shift(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true));
+}
+template <int CTRL>
+__device__ __forceinline__ double lane_shift(double x) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+template <typename T>
+__device__ __forceinline__ T lane_before(T x) { return lane_shift<0x138>(x); }   // wave_shr:1
+template <typename T>
+__device__ __forceinline__ T lane_after(T x) { return lane_shift<0x130>(x); }    // wave_shl:1
+
+template <typename T, int R, int NW>
+struct Cd2dNLds {
+  T first[2][NW][TX], last[2][NW][TX], lastz[2][NW][TX];   // rows 0 and R-1 of p, row R-1 of psi_z
+  T cz[NW * R + 1][4];         // z C-PML coefficients b_h, a_h, b, a of the rows, from the one before
+  short inj[NW * R][TX];       // staged values of a cell's points: slot + 1 and, above bit 7, their number;
+                               // 0: no point, -1: not staged
+  short rec[NW * R][TX];       // a cell's entries of col: first + 1 and, above bit 8, their number; 0, -1 alike
+  T val[SN_MAX][SN_SLOTS];
+  int col[SN_RECS];            // traces of the window's receivers
+  int used, rused;             // slots and entries taken
+};
+
+// Registers of one thread: R cells of a column.
+template <typename T, int R>
+struct Cd2dNRegs {
+  T pc[R], po[R], fa[R];
+  T psx[R], xix[R], psz[R], xiz[R];
+};
+
+// Window of a block and what its threads own.
+struct Cd2dNWin {
+  int i, j0, w, lane;
+  bool own;            // column owned
+  int rows;            // rows of this wave owned (bit r: row r)
+  int jin, kzr, xzr;   // rows inside the grid's z edges, with a psi_z / a xi_z
+  int imask, rmask;    // rows that hold injected points / receivers
+};
+
+// Injection of the level with index m (of the nl staged ones) and number l at
+// row r: p += value (times the factor in the adjoint), in list order.
+template <typename T, int R, int NW, bool ADJ>
+__device__ __forceinline__ void cd2d_n_inject(const Cd2dStepArgs<T> &a, const Cd2dNLds<T, R, NW> &L,
+                                              const Cd2dNWin &W, int s, int nts, int r, int m, int l, T f, T &pnv,
+                                              T &inj) {
+  const int e = L.inj[W.w * R + r][W.lane];
+  if (e == 0) return;
+  auto add = [&](T v) {
+    if (ADJ) {
+      pnv += v * f;
+    } else {
+      pnv += v;
+      inj += v;
+    }
+  };
+  if (e > 0) {
+    const T *v = L.val[m] + (e & 127) - 1;
+#pragma clang loop unroll(disable)
+    for (int k = 0; k < e >> 7; k++) add(v[k]);
+    return;
   }
-  o.kz = -1;
-  if (j < h) o.kz = j;
-  else if (j >= nz - h - 1 && j <= nz - 2) o.kz = j + 1 - nz + 2 * h;
-  o.psz = 0;
-  if (o.kz >= 0) {
-    const T d = (pc_at(0, 1) - pc) * a.idz;
-    o.psz = cz.bh(o.kz) * pszo(j, o.kz) + cz.ah(o.kz) * d;
-  }
-  o.xup = o.zup = false;
-  o.xix = o.xiz = 0;
-  T pnv = 0, flap = 0, inj = 0;
-  if (interior) {
+  const int *ptr = ADJ ? a.pt.urec_ptr : a.pt.usrc_ptr, *list = ADJ ? a.pt.urec_list : a.pt.usrc_list;
+  const T *tf = (ADJ ? a.res + a.pt.off_tr[s] : a.srctf + a.pt.off_tf[s]) + (l - 1);
+  const int j = W.j0 + r;
+  const int u = find_point(ADJ ? a.pt.rrow : a.pt.srow, ADJ ? a.pt.urec_cell : a.pt.usrc_cell, a.pt.nrows, s, j,
+                           (int64_t)j * a.nx + W.i);
+#pragma clang loop unroll(disable)
+  for (int k = ptr[u]; k < ptr[u + 1]; k++) add(tf[(int64_t)nts * list[k]]);
+}
+
+// One level on a thread's R cells.  XS: the window reaches an x strip or x
+// edge; ZS: the wave's rows reach a z strip or z edge.  up / dn: values of
+// the row before the first / after the last, zup: old psi_z of the row
+// before.  dv receives what the history keeps of a forward level (before the
+// injection).
+template <typename T, int R, int NW, bool ADJ, bool XS, bool ZS>
+__device__ __forceinline__ void cd2d_n_level(const Cd2dStepArgs<T> &a, const Cd2dNLds<T, R, NW> &L,
+                                             const Cd2dNWin &W, int kx, const T *xc, T up, T dn, T zup,
+                                             Cd2dNRegs<T, R> &G, T *dv) {
+  const int nx = a.nx, h = a.h, i = W.i;
+  const bool xin = !XS || (i >= 1 && i <= nx - 2);
+  const bool xst = XS && (i < h || i >= nx - h);
+  T prev = up, pszp = 0;
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    const bool interior = xin && (!ZS || (W.jin >> r & 1));
+    const T pc = G.pc[r], pov = G.po[r];
+    const T pl = lane_before(pc), pr = lane_after(pc);
+    const T pd = prev, pu = r + 1 < R ? G.pc[r + 1 < R ? r + 1 : r] : dn;
     const T d2x = (pl - T(2) * pc + pr) * a.idx2;
     const T d2z = (pd - T(2) * pc + pu) * a.idz2;
     T lx = d2x, lz = d2z;
-    if (i < h || i >= nx - h) {
-      const int kn = o.kx - 1;
-      const T psn = cx.bh(kn) * psxo(i - 1, kn) + cx.ah(kn) * ((pc - pl) * a.idx);
-      const T dpsi = (o.psx - psn) * a.idx;
-      const T xi = cx.b(o.kx) * xixo() + cx.a(o.kx) * (d2x + dpsi);
-      o.xix = xi;
-      o.xup = true;
-      lx = d2x + dpsi + xi;
-    }
-    if (j < h || j >= nz - h) {
-      const int kn = o.kz - 1;
-      const T psn = cz.bh(kn) * pszo(j - 1, kn) + cz.ah(kn) * ((pc - pd) * a.idz);
-      const T dpsi = (o.psz - psn) * a.idz;
-      const T xi = cz.b(o.kz) * xizo() + cz.a(o.kz) * (d2z + dpsi);
-      o.xiz = xi;
-      o.zup = true;
-      lz = d2z + dpsi + xi;
-    }
-    flap = fa * (lx + lz);
-    pnv = T(2) * pc - pov + flap;
-  }
-  if (!interior) pnv = pov;
-  if (!ADJ) {
-    const int u = find_point(a.pt.srow, a.pt.usrc_cell, a.pt.nrows, s, j, c);
-    if (u >= 0) {
-      const T *tf = a.srctf + a.pt.off_tf[s] + (itl - 1);
-      for (int k = a.pt.usrc_ptr[u]; k < a.pt.usrc_ptr[u + 1]; k++) {
-        const T v = tf[(int64_t)nts * a.pt.usrc_list[k]];
-        pnv += v;
-        inj += v;
+    if (XS) {
+      // psi_x of the cell's own strip entry; the left neighbour's is its lane's
+      const T d = (pr - pc) * a.idx;
+      const T psx = kx >= 0 ? xc[0] * G.psx[r] + xc[1] * d : T(0);
+      const T psn = lane_before(psx);
+      G.psx[r] = psx;
+      if (xst && interior) {
+        const T dpsi = (psx - psn) * a.idx;
+        const T xi = xc[2] * G.xix[r] + xc[3] * (d2x + dpsi);
+        G.xix[r] = xi;
+        lx = d2x + dpsi + xi;
       }
     }
-  } else {
-    const int u = find_point(a.pt.rrow, a.pt.urec_cell, a.pt.nrows, s, j, c);
-    if (u >= 0) {
-      const T *rs = a.res + a.pt.off_tr[s] + (itl - 1);
-      const T f = fa;
-      for (int k = a.pt.urec_ptr[u]; k < a.pt.urec_ptr[u + 1]; k++) pnv += rs[(int64_t)nts * a.pt.urec_list[k]] * f;
+    if (ZS) {
+      T psz = 0;
+      if (W.kzr >> r & 1) {
+        const T *cz = L.cz[W.w * R + r + 1];
+        const T d = (pu - pc) * a.idz;
+        psz = cz[0] * G.psz[r] + cz[1] * d;
+        if (W.xzr >> r & 1) {
+          // psi_z of the row before: stepped already, or (first row of the
+          // wave) recomputed from its old value
+          T psn = pszp;
+          if (r == 0) {
+            const T dp = (pc - pd) * a.idz;
+            psn = cz[-4] * zup + cz[-3] * dp;
+          }
+          if (interior) {
+            const T dpsi = (psz - psn) * a.idz;
+            const T xi = cz[2] * G.xiz[r] + cz[3] * (d2z + dpsi);
+            G.xiz[r] = xi;
+            lz = d2z + dpsi + xi;
+          }
+        }
+      }
+      G.psz[r] = psz;
+      pszp = psz;
+    }
+    const T flap = G.fa[r] * (lx + lz);
+    T pnv = T(2) * pc - pov + flap;
+    T dval = flap;
+    if (XS || ZS) {
+      if (!interior) {
+        pnv = pov;
+        dval = (pov - T(2) * pc) + pnv;
+      }
+    }
+    prev = pc;
+    G.po[r] = pc;
+    G.pc[r] = pnv;
+    if (!ADJ) dv[r] = dval;
+  }
+}
+
+// Makes x opaque: the compiler otherwise keeps what follows from it for every
+// row (tests, addresses) in scalar registers over the levels, spills them and
+// pays a lane read for each use, more than computing it again.
+// (x is the same in all lanes of the wave.)
+__device__ __forceinline__ void opaque(int &x) {
+  x = __builtin_amdgcn_readfirstlane(x);
+  asm volatile("" : "+s"(x));
+}
+
+// Points of the wave's rows: the cells' entries in LDS, and (injected points)
+// their values of the levels la, la + dir, .. (nl of them).
+template <typename T, int R, int NW, bool ADJ>
+__device__ __forceinline__ void cd2d_n_points(const Cd2dStepArgs<T> &a, Cd2dNLds<T, R, NW> &L, Cd2dNWin &W, int s,
+                                              int nts, int X0, int la, int nl) {
+  const int64_t ro = (int64_t)s * (a.pt.nrows + 1);
+  const int *irow = (ADJ ? a.pt.rrow : a.pt.srow) + ro, *rrow = a.pt.rrow + ro;
+  const int64_t *icell = ADJ ? a.pt.urec_cell : a.pt.usrc_cell;
+  const int *iptr = ADJ ? a.pt.urec_ptr : a.pt.usrc_ptr, *ilist = ADJ ? a.pt.urec_list : a.pt.usrc_list;
+  const T *tf = ADJ ? a.res + a.pt.off_tr[s] : a.srctf + a.pt.off_tf[s];
+  // bounds of the rows' points, one row per lane
+  const int jl = min(W.j0 + min(W.lane, R), a.nz);
+  const int ib = irow[min(jl, a.nz)], rb = (!ADJ && a.traces) ? rrow[min(jl, a.nz)] : 0;
+  W.imask = W.rmask = 0;
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    if (__shfl(ib, r) != __shfl(ib, r + 1)) W.imask |= 1 << r;
+    if (__shfl(rb, r) != __shfl(rb, r + 1)) W.rmask |= 1 << r;
+  }
+  W.imask = __builtin_amdgcn_readfirstlane(W.imask);
+  W.rmask = __builtin_amdgcn_readfirstlane(W.rmask);
+  if (!(W.imask | W.rmask)) return;
+  for (int r = 0; r < R; r++) {
+    const int64_t c0 = (int64_t)(W.j0 + r) * a.nx + X0;
+    if (W.imask >> r & 1) {
+      L.inj[W.w * R + r][W.lane] = 0;
+      __builtin_amdgcn_wave_barrier();
+      const int q1 = __shfl(ib, r + 1);
+      for (int q = __shfl(ib, r) + W.lane; q < q1; q += TX) {
+        const int64_t o = icell[q] - c0;
+        if (o < 0 || o >= TX) continue;
+        const int k0 = iptr[q], cnt = iptr[q + 1] - k0;
+        const int slot = cnt <= SN_SLOTS ? atomicAdd(&L.used, cnt) : SN_SLOTS;
+        if (slot + cnt > SN_SLOTS) {
+          L.inj[W.w * R + r][o] = -1;
+          continue;
+        }
+        for (int k = 0; k < cnt; k++) {
+          const T *v = tf + (int64_t)nts * ilist[k0 + k] + (la - 1);
+          for (int m = 0; m < nl; m++) L.val[m][slot + k] = v[ADJ ? -m : m];
+        }
+        L.inj[W.w * R + r][o] = (short)((slot + 1) | cnt << 7);
+      }
+    }
+    if (W.rmask >> r & 1) {
+      L.rec[W.w * R + r][W.lane] = 0;
+      __builtin_amdgcn_wave_barrier();
+      const int q1 = __shfl(rb, r + 1);
+      for (int q = __shfl(rb, r) + W.lane; q < q1; q += TX) {
+        const int64_t o = a.pt.urec_cell[q] - c0;
+        if (o < 0 || o >= TX) continue;
+        const int k0 = a.pt.urec_ptr[q], cnt = a.pt.urec_ptr[q + 1] - k0;
+        const int first = cnt <= 127 ? atomicAdd(&L.rused, cnt) : SN_RECS;
+        if (first + cnt > SN_RECS) {
+          L.rec[W.w * R + r][o] = -1;
+          continue;
+        }
+        for (int k = 0; k < cnt; k++) L.col[first + k] = a.pt.urec_list[k0 + k];
+        L.rec[W.w * R + r][o] = (short)((first + 1) | cnt << 8);
+      }
     }
   }
-  o.pnv = pnv;
-  o.dval = interior ? flap + inj : (pov - T(2) * pc) + pnv;
-  return o;
 }
 
-// Stores of an owned cell at level itl: pressure, memory variables,
-// replay history and receiver traces.
-template <typename T>
-__device__ __forceinline__ void cd2d_cell_store(const Cd2dStepArgs<T> &a, const Cd2dCell<T> &o, int s, int nts,
-                                                int itl, int i, int j, T *pn, T *psxn, T *pszn, T *xixn, T *xizn) {
-  const int nx = a.nx, h = a.h;
-  const int64_t so = (int64_t)s * a.N;
-  const int64_t c = (int64_t)j * nx + i;
-  pn[so + c] = o.pnv;
-  if (o.kx >= 0) psxn[(int64_t)s * a.spx + (int64_t)j * (2 * h) + o.kx] = o.psx;
-  if (o.kz >= 0) pszn[(int64_t)s * a.spz + (int64_t)o.kz * nx + i] = o.psz;
-  if (o.xup) xixn[(int64_t)s * a.sxx + (int64_t)j * (2 * h + 2) + o.kx] = o.xix;
-  if (o.zup) xizn[(int64_t)s * a.sxz + (int64_t)o.kz * nx + i] = o.xiz;
-  if (a.traces) {
-    const int r = find_point(a.pt.rrow, a.pt.urec_cell, a.pt.nrows, s, j, c);
-    if (r >= 0) {
-      T *tr = a.traces + a.pt.off_tr[s] + (itl - 1);
-      for (int k = a.pt.urec_ptr[r]; k < a.pt.urec_ptr[r + 1]; k++) tr[(int64_t)nts * a.pt.urec_list[k]] = o.pnv;
-    }
-  }
-  const int slot = cd2d_dslot(a, nts, itl);
-  if (slot >= 0) a.dbuf[(int64_t)slot * a.dslot + so + c] = o.dval;
-}
-
-// Arguments of the second level of a two-level launch: the slots of the
-// second level (it+1 forward, it-1 adjoint: pressure, memory variables)
-// next to those of level it in Cd2dStepArgs.
-template <typename T>
-struct Cd2dStep2Args {
-  Cd2dStepArgs<T> a;
-  T *pnew2;
-  T *psix_n2, *psiz_n2, *xix_n2, *xiz_n2;
-};
-
-// Is the region of tile (I0, J0) of shot s plain: every region cell inside
-// the grid, outside the C-PML strips, and no source or receiver on the
-// region's rows?
-template <typename T>
-__device__ __forceinline__ bool cd2d_step2_is_lean(const Cd2dStepArgs<T> &a, int s, int I0, int J0) {
-  const int nx = a.nx, nz = a.nz, h = a.h;
-  const int i0 = I0 - 1, i1 = I0 + TX, j0 = J0 - 1, j1 = J0 + S2H;
-  if (!(i0 >= max(h, 1) && i1 <= nx - h - 2 && j0 >= max(h, 1) && j1 <= nz - h - 2)) return false;
-  const int64_t o = (int64_t)s * (a.pt.nrows + 1);
-  const int *rowp = a.res == nullptr ? a.pt.srow : a.pt.rrow;
-  if (rowp[o + j0] != rowp[o + j1 + 1]) return false;
-  if (a.traces && a.pt.rrow[o + j0] != a.pt.rrow[o + j1 + 1]) return false;
-  return true;
-}
-
-// Forward (ADJ = false): levels it and it+1 from it-1, it-2.  Adjoint
-// (ADJ = true): adjoint levels it and it-1 from it+1, it+2, with the
-// residual injection of each level and the correlations of both launches
-// the one-level kernel would make (level it correlates the adjoint level
-// it+1, level it-1 the adjoint level it, each with its replay history
-// slot), done by the owner of each cell in the same order.
-template <typename T, bool ADJ>
-__global__ __launch_bounds__(TX *TZ) void cd2d_step2_kernel(Cd2dStep2Args<T> A2) {
-  const Cd2dStepArgs<T> &a = A2.a;
-  __shared__ T sA[S2R][S2W];    // first level on the region
-  __shared__ T sC[S2R][S2W];    // its current level (it-1 forward, it+1 adjoint) on the region
-  __shared__ T sX[S2R][S2W];    // psi_x of the first level (strip cells)
-  __shared__ T sZ[S2R][S2W];    // psi_z of the first level
-  __shared__ T sXI[S2R][S2W];   // xi_x of the first level
-  __shared__ T sZI[S2R][S2W];   // xi_z of the first level
+// Forward / replay levels it .. it+n-1, or (ADJ) adjoint levels it .. it-n+1
+// with their injection and their correlation with the forward history.
+template <typename T, int R, int NW, bool ADJ>
+__global__ __launch_bounds__(NW *TX, sizeof(T) == 4 ? 4 : 2) void cd2d_stepn_kernel(Cd2dStepNArgs<T> A) {
+  const Cd2dStepArgs<T> &a = A.a;
+  __shared__ Cd2dNLds<T, R, NW> L;
+  constexpr int H = NW * R;
+  if (threadIdx.x == 0) L.used = L.rused = 0;
+  __syncthreads();
   const int b = xcd_tile2(blockIdx.x, gridDim.x);
   const int t = b / a.nbx;
   const int bx = b - t * a.nbx, by = t % a.nby, s = t / a.nby;
   const int nts = a.nt_shot[s];
-  if (nts <= a.act_min) return;
-  const int itA = a.it, itB = ADJ ? a.it - 1 : a.it + 1;
-  // a shot takes a level while it is within its nt (an adjoint shot whose
-  // last level is it-1 starts from zero fields at level it)
-  const bool actA = itA <= nts, actB = itB <= nts;
-  if (!actA && !actB) return;
-  const int nx = a.nx, nz = a.nz, h = a.h;
-  const int I0 = bx * TX, J0 = by * S2H;
-  const int tid = threadIdx.y * TX + threadIdx.x;
-  const int64_t so = (int64_t)s * a.N;
-  const T *pc_ = a.pcur + so;
-  const T *po_ = a.pold + so;
-  // correlations (adjoint): level itl correlates the adjoint level itl+1
-  // with history slot itl - cbase while itl+1 is within nt and the segment
-  const bool corrA = ADJ && a.corr && actA && itA + 1 <= nts && itA + 1 <= a.corr_lim;
-  const bool corrB = ADJ && a.corr && actB && itB + 1 <= nts && itB + 1 <= a.corr_lim;
-  T gv[2], dA[2], dB[2];
-  if (ADJ && (corrA || corrB)) {
+  const int n = A.n, nx = a.nx, nz = a.nz, h = a.h;
+  const int X0 = bx * (TX - 2 * n), Z0 = by * (H - 2 * n);
+  Cd2dNWin W;
+  W.lane = threadIdx.x & (TX - 1);
+  W.w = __builtin_amdgcn_readfirstlane(threadIdx.x / TX);
+  W.i = X0 + W.lane;
+  W.j0 = Z0 + W.w * R;
+  W.own = W.i < nx && W.lane >= (bx ? n : 0) && W.lane < (bx < a.nbx - 1 ? TX - n : TX);
+  W.rows = W.jin = W.kzr = W.xzr = 0;
+  const int own0 = by ? Z0 + n : 0, own1 = by < a.nby - 1 ? Z0 + H - n : nz;
 #pragma unroll
-    for (int r = 0; r < 2; r++) {
-      const int i = min(I0 + (int)threadIdx.x, nx - 1), j = min(J0 + (int)threadIdx.y + r * TZ, nz - 1);
-      const int64_t c = (int64_t)j * nx + i;
-      gv[r] = a.grad[so + c];
-      dA[r] = corrA ? a.dbuf[(int64_t)(itA - a.cbase) * a.dslot + so + c] : T(0);
-      dB[r] = corrB ? a.dbuf[(int64_t)(itB - a.cbase) * a.dslot + so + c] : T(0);
+  for (int r = 0; r < R; r++) {
+    const int j = W.j0 + r;
+    if (j >= own0 && j < own1) W.rows |= 1 << r;
+    if (j >= 1 && j <= nz - 2) {
+      W.jin |= 1 << r;
+      if (j < h || j >= nz - h) W.xzr |= 1 << r;
+    }
+    if (j < h || (j >= nz - h - 1 && j <= nz - 2)) W.kzr |= 1 << r;
+  }
+  const int64_t so = (int64_t)s * a.N;
+  const bool xs = X0 < max(h, 1) || X0 + TX - 1 >= nx - h - 1;
+  const bool zs = W.j0 < max(h, 1) || W.j0 + R - 1 >= nz - h - 1;
+  int kx = -1;
+  if (W.i < h) kx = W.i;
+  else if (W.i >= nx - h - 1 && W.i <= nx - 2) kx = W.i + 1 - nx + 2 * h;
+
+  Cd2dNRegs<T, R> G;
+  T g[R], d0[R], d1[R];
+  const T *pc_ = a.pcur + so, *po_ = a.pold + so;
+  // Rows and columns beyond the grid take those of its edge: what they hold
+  // is never read by a cell of the grid (edge cells read no neighbour).
+  const unsigned ic = min(W.i, nx - 1);
+  auto row = [&](const T *p, int r) { return p + (int64_t)min(W.j0 + r, nz - 1) * nx; };
+  auto strip = [&](int r) {      // z strip entry of row r
+    const int j = W.j0 + r;
+    return j < h ? j : j + 1 - nz + 2 * h;
+  };
+  // forward history of level l (ADJ)
+  auto fetch = [&](T *d, int l) {
+    const T *slot = a.dbuf + (int64_t)(max(l, a.it - n + 1) - a.cbase - 1) * a.dslot + so;
+#pragma unroll
+    for (int r = 0; r < R; r++) d[r] = row(slot, r)[ic];
+  };
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    G.pc[r] = row(pc_, r)[ic];
+    G.po[r] = row(po_, r)[ic];
+    G.fa[r] = row(a.fact, r)[ic];
+    G.psx[r] = G.xix[r] = G.psz[r] = G.xiz[r] = T(0);
+    if (ADJ) g[r] = row(a.grad + so, r)[ic];
+  }
+  T xc[4] = {T(0), T(0), T(0), T(0)};
+  if (xs && h > 0) {
+    const AxisCoef<T> cx = axis_coef(a.cpml + (int64_t)s * a.cstride, h, 0);
+    const unsigned k = max(kx, 0);
+    const T c0 = cx.bh(k), c1 = cx.ah(k), c2 = cx.b(k), c3 = cx.a(k);
+    if (kx >= 0) {
+      xc[0] = c0;
+      xc[1] = c1;
+      xc[2] = c2;
+      xc[3] = c3;
+    }
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      const int j = min(W.j0 + r, nz - 1);
+      const T v0 = (a.psix_o + (int64_t)s * a.spx + (int64_t)j * (2 * h))[k];
+      const T v1 = (a.xix_o + (int64_t)s * a.sxx + (int64_t)j * (2 * h + 2))[k];
+      G.psx[r] = kx >= 0 ? v0 : T(0);
+      G.xix[r] = kx >= 0 ? v1 : T(0);
     }
   }
-  // owner's correlation of tile cell r: the current level of each of the
-  // two one-level launches (pcA, then the first level pcB)
-  auto correlate = [&](int r, int64_t c, T pcA, T pcB) {
-    if (!(corrA || corrB)) return;
-    T g = gv[r];
-    if (corrA) g = g + pcA * dA[r];
-    if (corrB) g = g + pcB * dB[r];
-    a.grad[so + c] = g;
-  };
-  if (actA && a.lean && cd2d_step2_is_lean(a, s, I0, J0)) {
-    // Every load first: the current level on the tile + 2 (staged in LDS),
-    // the previous level and the factor on the region, the factor on the
-    // tile's cells.
-    constexpr int PW = TX + 4, PH = S2H + 4, PN = PW * PH;
-    constexpr int PQ = (PN + TX * TZ - 1) / (TX * TZ);
-    __shared__ T sP[PH][PW];      // current level: columns I0-2 .., rows J0-2 ..
-    T pp[PQ], pov[S2Q], fa[S2Q], faB[2];
+  if (zs) {
 #pragma unroll
-    for (int k = 0; k < PQ; k++) {
-      const int q = min(tid + k * TX * TZ, PN - 1);
-      const int ly = q / PW, lx = q - ly * PW;
-      pp[k] = pc_[(J0 - 2 + ly) * nx + (I0 - 2 + lx)];
-    }
-#pragma unroll
-    for (int k = 0; k < S2Q; k++) {
-      const int q = min(tid + k * TX * TZ, S2N - 1);
-      const int ly = q / S2W, lx = q - ly * S2W;
-      const int c = (J0 - 1 + ly) * nx + (I0 - 1 + lx);
-      pov[k] = po_[c];
-      fa[k] = a.fact[c];
-    }
-#pragma unroll
-    for (int r = 0; r < 2; r++) faB[r] = a.fact[(J0 + threadIdx.y + r * TZ) * nx + I0 + threadIdx.x];
-#pragma unroll
-    for (int k = 0; k < PQ; k++) {
-      const int q = tid + k * TX * TZ;
-      if (q < PN) sP[q / PW][q % PW] = pp[k];
-    }
-    const int slotA = cd2d_dslot(a, nts, itA), slotB = cd2d_dslot(a, nts, itB);
+    for (int r = 0; r < R; r++)
+      if (W.kzr >> r & 1) {
+        G.psz[r] = (a.psiz_o + (int64_t)s * a.spz + (int64_t)strip(r) * nx)[ic];
+        G.xiz[r] = (a.xiz_o + (int64_t)s * a.sxz + (int64_t)strip(r) * nx)[ic];
+      }
+  }
+  // levels of this shot: a forward one ends at nts, an adjoint one starts
+  // there (from zero fields).  Tested after the loads above were issued, so
+  // that they do not wait for nts.
+  const int la = ADJ ? min(a.it, nts) : a.it;
+  const int nl = ADJ ? la - (a.it - n) : min(n, nts - a.it + 1);
+  if (nl <= 0 || nts <= a.act_min) return;
+  // the history slot of forward level l is l - seg0 - 1 (none up to seg0)
+  const int seg0 = a.dmode == 1 ? ((nts - 1) / a.S) * a.S : a.dmode == 2 ? a.cbase : a.it + n;
+  if (ADJ) {
+    fetch(d0, la);
+    fetch(d1, la - 1);
+  }
+  // (loaded here: a load in the level loop would wait for the wave's stores)
+  const int64_t otr = a.pt.off_tr[s];
+  cd2d_n_points<T, R, NW, ADJ>(a, L, W, s, nts, X0, la, nl);
+  if (threadIdx.x <= H) {
+    const int j = Z0 - 1 + (int)threadIdx.x;
+    int kz = -1;
+    if (j >= 0 && j < h) kz = j;
+    else if (j >= nz - h - 1 && j <= nz - 2) kz = j + 1 - nz + 2 * h;
+    const AxisCoef<T> cz = axis_coef(a.cpml + (int64_t)s * a.cstride, h, 1);
+    T *q = L.cz[threadIdx.x];
+    q[0] = kz >= 0 ? cz.bh(kz) : T(0);
+    q[1] = kz >= 0 ? cz.ah(kz) : T(0);
+    q[2] = kz >= 0 ? cz.b(kz) : T(0);
+    q[3] = kz >= 0 ? cz.a(kz) : T(0);
+  }
+
+  auto level = [&](int m, T *dv) {
+    opaque(W.j0);
+    opaque(W.rows);
+    opaque(W.jin);
+    opaque(W.kzr);
+    opaque(W.xzr);
+    opaque(W.imask);
+    opaque(W.rmask);
+    const int l = ADJ ? la - m : la + m;
+    const int p = m & 1;
+    L.first[p][W.w][W.lane] = G.pc[0];
+    L.last[p][W.w][W.lane] = G.pc[R - 1];
+    if (zs) L.lastz[p][W.w][W.lane] = G.psz[R - 1];
     __syncthreads();
+    // (the first and last wave read rows of their own: the window's side)
+    const T up = L.last[p][W.w > 0 ? W.w - 1 : 0][W.lane];
+    const T dn = L.first[p][W.w < NW - 1 ? W.w + 1 : NW - 1][W.lane];
+    const T zup = zs ? L.lastz[p][W.w > 0 ? W.w - 1 : 0][W.lane] : T(0);
+    T dval[R];
+    if (xs) cd2d_n_level<T, R, NW, ADJ, true, true>(a, L, W, kx, xc, up, dn, zup, G, dval);
+    else if (zs) cd2d_n_level<T, R, NW, ADJ, false, true>(a, L, W, kx, xc, up, dn, zup, G, dval);
+    else cd2d_n_level<T, R, NW, ADJ, false, false>(a, L, W, kx, xc, up, dn, zup, G, dval);
+    if (W.imask | W.rmask) {
 #pragma unroll
-    for (int k = 0; k < S2Q; k++) {
-      const int q = tid + k * TX * TZ;
-      if (q < S2N) {
-        const int ly = q / S2W, lx = q - ly * S2W;
-        const T pc = sP[ly + 1][lx + 1];
-        const T d2x = (sP[ly + 1][lx] - T(2) * pc + sP[ly + 1][lx + 2]) * a.idx2;
-        const T d2z = (sP[ly][lx + 1] - T(2) * pc + sP[ly + 2][lx + 1]) * a.idz2;
-        const T lxx = d2x, lzz = d2z;
-        const T flap = fa[k] * (lxx + lzz);
-        const T pnv = T(2) * pc - pov[k] + flap;
-        const T inj = 0;
-        sA[ly][lx] = pnv;
-        if (lx >= 1 && lx <= TX && ly >= 1 && ly <= S2H) {
-          const int64_t c = (int64_t)(J0 - 1 + ly) * nx + (I0 - 1 + lx);
-          a.pnew[so + c] = pnv;
-          if (slotA >= 0) a.dbuf[(int64_t)slotA * a.dslot + so + c] = flap + inj;
+      for (int r = 0; r < R; r++) {
+        if (W.imask >> r & 1) {
+          T inj = 0;
+          const T before = G.pc[r];      // of an edge cell: its level before last
+          cd2d_n_inject<T, R, NW, ADJ>(a, L, W, s, nts, r, m, l, G.fa[r], G.pc[r], inj);
+          if (!ADJ) {
+            const bool interior = W.i >= 1 && W.i <= nx - 2 && (W.jin >> r & 1);
+            dval[r] = interior ? dval[r] + inj : (before - T(2) * G.po[r]) + G.pc[r];
+          }
+        }
+        if (!ADJ && (W.rmask & W.rows) >> r & 1 && W.own) {
+          const int e = L.rec[W.w * R + r][W.lane];
+          T *tr = a.traces + otr + (l - 1);
+          if (e > 0) {
+#pragma clang loop unroll(disable)
+            for (int k = 0; k < e >> 8; k++) tr[(int64_t)nts * L.col[(e & 255) - 1 + k]] = G.pc[r];
+          } else if (e < 0) {
+            const int j = W.j0 + r;
+            const int u = find_point(a.pt.rrow, a.pt.urec_cell, a.pt.nrows, s, j, (int64_t)j * nx + W.i);
+#pragma clang loop unroll(disable)
+            for (int k = a.pt.urec_ptr[u]; k < a.pt.urec_ptr[u + 1]; k++)
+              tr[(int64_t)nts * a.pt.urec_list[k]] = G.pc[r];
+          }
         }
       }
     }
-    if (!actB) return;
-    __syncthreads();
+    if constexpr (ADJ) {
 #pragma unroll
-    for (int r = 0; r < 2; r++) {
-      const int lx = threadIdx.x + 1, ly = threadIdx.y + r * TZ + 1;
-      const int64_t c = (int64_t)(J0 - 1 + ly) * nx + (I0 - 1 + lx);
-      const T p = sA[ly][lx];
-      const T d2x = (sA[ly][lx - 1] - T(2) * p + sA[ly][lx + 1]) * a.idx2;
-      const T d2z = (sA[ly - 1][lx] - T(2) * p + sA[ly + 1][lx]) * a.idz2;
-      const T lxx = d2x, lzz = d2z;
-      const T flap = faB[r] * (lxx + lzz);
-      const T pnv = T(2) * p - sP[ly + 1][lx + 1] + flap;
-      const T inj = 0;
-      A2.pnew2[so + c] = pnv;
-      if (slotB >= 0) a.dbuf[(int64_t)slotB * a.dslot + so + c] = flap + inj;
-      correlate(r, c, sP[ly + 1][lx + 1], p);
-    }
-    return;
-  }
-  // General tile: the first level on the region with cd2d_cell's branches
-  // (cells outside the grid are skipped: only interior cells read their
-  // neighbours, and those are inside the grid)
-  T faB[2];
+      for (int r = 0; r < R; r++) g[r] = g[r] + G.pc[r] * dv[r];
+      fetch(dv, l - 2);
+    } else {
+      if (l > seg0 && W.own) {
+        T *D = a.dbuf + (int64_t)(l - seg0 - 1) * a.dslot + so;
 #pragma unroll
-  for (int r = 0; r < 2; r++) {
-    const int i = I0 + threadIdx.x, j = J0 + threadIdx.y + r * TZ;
-    faB[r] = (i < nx && j < nz) ? a.fact[(int64_t)j * nx + i] : T(0);
-  }
-  const T *psxo_ = a.psix_o + (int64_t)s * a.spx, *pszo_ = a.psiz_o + (int64_t)s * a.spz;
-  const T *xixo_ = a.xix_o + (int64_t)s * a.sxx, *xizo_ = a.xiz_o + (int64_t)s * a.sxz;
-  for (int q = tid; q < S2N; q += TX * TZ) {
-    const int ly = q / S2W, lx = q - ly * S2W;
-    const int i = I0 - 1 + lx, j = J0 - 1 + ly;
-    if (i < 0 || i >= nx || j < 0 || j >= nz) continue;
-    if (!actA) {
-      // an adjoint shot that starts at the second level: zero fields
-      sA[ly][lx] = sC[ly][lx] = sX[ly][lx] = sZ[ly][lx] = sXI[ly][lx] = sZI[ly][lx] = T(0);
-      continue;
+        for (int r = 0; r < R; r++)
+          if (W.rows >> r & 1) (D + (int64_t)(W.j0 + r) * nx)[ic] = dval[r];
+      }
     }
-    const int64_t c = (int64_t)j * nx + i;
-    auto pcat = [&](int di, int dj) { return pc_[c + di + (int64_t)dj * nx]; };
-    auto psxo = [&](int, int k) { return psxo_[(int64_t)j * (2 * h) + k]; };
-    auto pszo = [&](int, int k) { return pszo_[(int64_t)k * nx + i]; };
-    const Cd2dCell<T> o = cd2d_cell_eval<T, ADJ>(
-        a, s, nts, itA, i, j, pcat, po_[c], a.fact[c], psxo, pszo,
-        [&]() { return xixo_[(int64_t)j * (2 * h + 2) + (i < h ? i : i + 1 - nx + 2 * h)]; },
-        [&]() { return xizo_[(int64_t)(j < h ? j : j + 1 - nz + 2 * h) * nx + i]; });
-    sA[ly][lx] = o.pnv;
-    sC[ly][lx] = pc_[c];
-    sX[ly][lx] = o.psx;
-    sZ[ly][lx] = o.psz;
-    sXI[ly][lx] = o.xix;
-    sZI[ly][lx] = o.xiz;
-    if (lx >= 1 && lx <= TX && ly >= 1 && ly <= S2H)
-      cd2d_cell_store(a, o, s, nts, itA, i, j, a.pnew, a.psix_n, a.psiz_n, a.xix, a.xiz);
+  };
+  if constexpr (ADJ) {
+    for (int m = 0; m < nl; m += 2) {
+      level(m, d0);
+      if (m + 1 < nl) level(m + 1, d1);
+    }
+  } else {
+#pragma clang loop unroll(disable)
+    for (int m = 0; m < nl; m++) level(m, d0);
   }
-  if (!actB) return;
-  __syncthreads();
-  // the second level on the tile, from the region in LDS
-  for (int r = 0; r < 2; r++) {
-    const int lx = threadIdx.x + 1, ly = threadIdx.y + r * TZ + 1;
-    const int i = I0 - 1 + lx, j = J0 - 1 + ly;
-    if (i >= nx || j >= nz) continue;
-    const int64_t c = (int64_t)j * nx + i;
-    auto pcat = [&](int di, int dj) { return sA[ly + dj][lx + di]; };
-    auto psxo = [&](int ii, int) { return sX[ly][ii - (I0 - 1)]; };
-    auto pszo = [&](int jj, int) { return sZ[jj - (J0 - 1)][lx]; };
-    const Cd2dCell<T> o = cd2d_cell_eval<T, ADJ>(a, s, nts, itB, i, j, pcat, sC[ly][lx], faB[r], psxo, pszo,
-                                                 [&]() { return sXI[ly][lx]; }, [&]() { return sZI[ly][lx]; });
-    cd2d_cell_store(a, o, s, nts, itB, i, j, A2.pnew2, A2.psix_n2, A2.psiz_n2, A2.xix_n2, A2.xiz_n2);
-    correlate(r, c, sC[ly][lx], sA[ly][lx]);
+
+  if (!W.own) return;
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    if (!(W.rows >> r & 1)) continue;
+    const int64_t j = W.j0 + r, o = so + j * nx;
+    (a.pnew + o)[ic] = G.pc[r];
+    if (n > 1) (A.pnew0 + o)[ic] = G.po[r];
+    if (ADJ) (a.grad + o)[ic] = g[r];
+    if (kx >= 0) {
+      (a.psix_n + (int64_t)s * a.spx + j * (2 * h))[(unsigned)kx] = G.psx[r];
+      (a.xix + (int64_t)s * a.sxx + j * (2 * h + 2))[(unsigned)kx] = G.xix[r];
+    }
+    if (W.kzr >> r & 1) {
+      (a.psiz_n + (int64_t)s * a.spz + (int64_t)strip(r) * nx)[ic] = G.psz[r];
+      (a.xiz + (int64_t)s * a.sxz + (int64_t)strip(r) * nx)[ic] = G.xiz[r];
+    }
   }
 }
 
@@ -666,29 +785,33 @@ class Cd2dEngine final : public Engine {
     sxx_ = (int64_t)(2 * h_ + 2) * nz_;
     sxz_ = (int64_t)nx_ * (2 * h_ + 2);
     cstride_ = 2 * (8 * h_ + 4);
-    // rows per thread (1, 2 or 4) and the interior-tile path; env overrides
-    // for measurement
+    // rows per thread (1, 2 or 4) and the interior-tile path of
+    // cd2d_step_kernel, which the environment picks (one level per launch)
     if (const char *v = std::getenv("SWX_CD2D_ROWS")) {
       const int r = std::atoi(v);
       SWX_REQUIRE(r == 1 || r == 2 || r == 4, SWX_EINVAL, "SWX_CD2D_ROWS must be 1, 2 or 4");
       rows_ = r;
-      tuned_ = true;
+      steps_env_ = 1;
     }
     if (const char *v = std::getenv("SWX_CD2D_LEAN")) lean_ = std::atoi(v) != 0;
-    // levels per forward / replay launch (1 or 2, cd2d_step2_kernel)
+    // most levels per launch (1: cd2d_step_kernel, else cd2d_stepn_kernel) and
+    // window shape of the latter (10 x adjoint + forward)
     if (const char *v = std::getenv("SWX_CD2D_STEPS")) {
-      const int n = std::atoi(v);
-      SWX_REQUIRE(n == 1 || n == 2, SWX_EINVAL, "SWX_CD2D_STEPS must be 1 or 2");
-      steps_ = n;
-      steps_env_ = true;
+      steps_env_ = std::atoi(v);
+      SWX_REQUIRE(steps_env_ >= 1 && steps_env_ <= SN_MAX, SWX_EINVAL, "SWX_CD2D_STEPS must be 1 .. 8");
+    }
+    if (const char *v = std::getenv("SWX_CD2D_SHAPE")) {
+      shape_env_ = std::atoi(v);
+      const int f = shape_env_ % 10, b = shape_env_ / 10;
+      SWX_REQUIRE(shape_env_ >= 0 && f <= 2 && b <= 2 && !(b == 0) && !(f == 0 && sizeof(T) == 8) &&
+                      !(b == 1 && sizeof(T) == 8), SWX_EINVAL, "SWX_CD2D_SHAPE names a shape that is not built");
     }
     const size_t e = sizeof(T);
     fact_.alloc(N_ * e);
-    // forward state: four pressure levels (slot k mod 4) and the C-PML
-    // memory variables of three levels (buffer k mod 3), so that a launch
-    // stepping two levels never overwrites a level a neighbouring block
-    // still reads (cd2d_step2_kernel); the one-step kernel works on any
-    // distinct slots
+    // forward state: four pressure levels and the C-PML memory variables of
+    // three: a launch reads the two last levels and writes its own two last
+    // ones to the other slots, so that it never overwrites what a
+    // neighbouring block still reads (cd2d_stepn_kernel)
     p_.alloc(4 * ns_ * N_ * e);
     psix_.alloc(std::max<int64_t>(3 * ns_ * spx_, 1) * e);
     psiz_.alloc(std::max<int64_t>(3 * ns_ * spz_, 1) * e);
@@ -754,36 +877,35 @@ class Cd2dEngine final : public Engine {
     SWX_REQUIRE(model_set_, SWX_ESTATE, "swx_set_model must be called before running");
     zero_forward_state();
     T *tr = c_.pts.d_traces.as<T>();
-    if (!tuned_) tune_rows(save, tr);
-    if (!steps_tuned_) tune_steps(save, tr);
+    choose_steps();
     for (int it = 1; it <= ntmax_;) {
       progress("forward step", it, ntmax_);
-      // two levels per launch: the state of both levels is in memory
-      // afterwards, so snapshots and checkpoints of either are taken after it
-      const int n = steps_ == 2 && it + 1 <= ntmax_ ? 2 : 1;
-      if (n == 2) step2_fwd(it, /*act_min=*/0, save ? 1 : 0, /*cbase=*/0, tr);
-      else step_fwd(it, /*act_min=*/0, save ? 1 : 0, /*cbase=*/0, tr);
-      for (int l = it; l < it + n; l++) {
-        take_snapshots(c_, *this, l);
-        if (save && l % S_ == 0) {
-          const int k = l / S_;
-          if (k >= 1 && k <= K_ - 2) save_ckpt(k, l);
-        }
-      }
+      // a launch ends at the levels whose state is kept: checkpoints (its two
+      // last levels) and snapshots
+      int end = ntmax_;
+      if (save) end = std::min<int64_t>(end, ceil_div(it, S_) * (int64_t)S_);
+      if (c_.snap_every > 0) end = std::min<int64_t>(end, ceil_div(it, c_.snap_every) * (int64_t)c_.snap_every);
+      const int n = levels(end - it + 1);
+      step_fwd(it, n, /*act_min=*/0, save ? 1 : 0, /*cbase=*/0, tr);
       it += n;
+      const int l = it - 1;
+      take_snapshots(c_, *this, l);
+      if (save && l % S_ == 0) {
+        const int k = l / S_;
+        if (k >= 1 && k <= K_ - 2) save_ckpt(k);
+      }
     }
   }
 
-  // "pcur" (acou_forward.jl:55-57): level it is in slot it mod 4
-  int snap_fields(int it, int s, SnapPiece *out) const override {
-    out[0] = {P(it) + (int64_t)s * N_, (int64_t)(N_ * sizeof(T)), (int64_t)(N_ * sizeof(T)), 1};
+  // "pcur" (acou_forward.jl:55-57): the level stepped last
+  int snap_fields(int, int s, SnapPiece *out) const override {
+    out[0] = {P(f_.cur) + (int64_t)s * N_, (int64_t)(N_ * sizeof(T)), (int64_t)(N_ * sizeof(T)), 1};
     return 1;
   }
 
   void adjoint(bool per_shot) override {
     (void)per_shot;
-    const int64_t e = sizeof(T);
-    if (!adj_steps_tuned_) tune_adj_steps();
+    b_ = Pos{};
     SWX_HIP(hipMemsetAsync(a_.get(), 0, a_.bytes(), c_.stream));
     SWX_HIP(hipMemsetAsync(apsix_.get(), 0, apsix_.bytes(), c_.stream));
     SWX_HIP(hipMemsetAsync(apsiz_.get(), 0, apsiz_.bytes(), c_.stream));
@@ -798,32 +920,32 @@ class Cd2dEngine final : public Engine {
       bool need = false;
       for (int s = 0; s < nsh_; s++) need |= nt_[s] > cb + S_;
       if (need) {
-        restore_ckpt(k, cb);
+        restore_ckpt(k);
         for (int it = cb + 1; it <= cb + S_;) {
-          const int n = steps_ == 2 && it + 1 <= cb + S_ ? 2 : 1;
-          if (n == 2) step2_fwd(it, cb + S_, 2, cb, nullptr);
-          else step_fwd(it, cb + S_, 2, cb, nullptr);
+          const int n = levels(cb + S_ - it + 1);
+          step_fwd(it, n, cb + S_, 2, cb, nullptr);
           it += n;
         }
       }
       const int top = std::min(cb + S_, ntmax_);
       for (int it = top; it >= cb + 1;) {
-        const int n = adj_steps_ == 2 && it - 1 >= cb + 1 ? 2 : 1;
-        if (n == 2) step2_adj(it, cb);
-        else step_adj(it, cb);
+        const int n = levels(it - cb);
+        step_adj(it, n, cb);
         it -= n;
       }
-      // correlation of the first step of the segment
-      dim3 g((unsigned)std::min<int64_t>(ceil_div(N_, 256), 1024), nsh_);
-      cd2d_correlate_kernel<T><<<g, 256, 0, c_.stream>>>(grad_.as<T>(), A(cb + 1),
-                                                          dbuf_.as<T>(), N_, c_.pts.d_nt.as<int>(), cb);
-      SWX_HIP(hipGetLastError());
+      if (steps_ == 1) {
+        // correlation of the first step of the segment (cd2d_stepn_kernel
+        // correlates every level that it steps)
+        dim3 g((unsigned)std::min<int64_t>(ceil_div(N_, 256), 1024), nsh_);
+        cd2d_correlate_kernel<T><<<g, 256, 0, c_.stream>>>(grad_.as<T>(), A(b_.cur), dbuf_.as<T>(), N_,
+                                                            c_.pts.d_nt.as<int>(), cb);
+        SWX_HIP(hipGetLastError());
+      }
     }
     const T scale = T(1.0 / (c_.d.dt * c_.d.dt));
     dim3 g((unsigned)std::min<int64_t>(ceil_div(N_, 256), 4096));
     reduce_shots<T><<<g, 256, 0, c_.stream>>>(gout_.as<T>(), grad_.as<T>(), N_, nsh_, scale, per_shot ? 1 : 0);
     SWX_HIP(hipGetLastError());
-    (void)e;
   }
 
   void copy_grad(void *host, bool per_shot) override {
@@ -835,24 +957,77 @@ class Cd2dEngine final : public Engine {
   int64_t bytes_checkpoints() const override { return ck_.bytes(); }
   int64_t bytes_replay() const override { return dbuf_.bytes(); }
   int segment() const override { return S_; }
-  // rows per thread of the one-level kernel; levels per launch, 10 x
-  // adjoint + forward / replay
-  void variants(int32_t v[2]) const override { v[0] = rows_; v[1] = 10 * adj_steps_ + steps_; }
+  // rows per thread of the one-level kernel, or window shapes of the n-level
+  // one (10 x adjoint + forward); most levels per launch, 10 x adjoint +
+  // forward / replay
+  void variants(int32_t v[2]) const override {
+    v[0] = steps_ == 1 ? rows_ : 10 * shape_[1] + shape_[0];
+    v[1] = 11 * steps_;
+  }
 
  private:
-  T *P(int k) const { return p_.as<T>() + (int64_t)(((k % 4) + 4) % 4) * ns_ * N_; }
-  // forward C-PML memory variables of level k
-  T *PSX(int k) const { return psix_.as<T>() + (int64_t)mod3(k) * ns_ * spx_; }
-  T *PSZ(int k) const { return psiz_.as<T>() + (int64_t)mod3(k) * ns_ * spz_; }
-  T *XIX(int k) const { return xix_.as<T>() + (int64_t)mod3(k) * ns_ * sxx_; }
-  T *XIZ(int k) const { return xiz_.as<T>() + (int64_t)mod3(k) * ns_ * sxz_; }
-  T *A(int k) const { return a_.as<T>() + (int64_t)(((k % 4) + 4) % 4) * ns_ * N_; }
-  T *APSX(int k) const { return apsix_.as<T>() + (int64_t)mod3(k) * ns_ * spx_; }
-  T *APSZ(int k) const { return apsiz_.as<T>() + (int64_t)mod3(k) * ns_ * spz_; }
-  T *AXIX(int k) const { return axix_.as<T>() + (int64_t)mod3(k) * ns_ * sxx_; }
-  T *AXIZ(int k) const { return axiz_.as<T>() + (int64_t)mod3(k) * ns_ * sxz_; }
+  // Slots of the levels of a state: the last level is in pressure slot cur,
+  // the one before it in cur - 1 (mod 4), the memory variables in buffer mv.
+  struct Pos {
+    int cur = 0, mv = 0;
+  };
+  void advance(Pos &p, int n) const {
+    p.cur = (p.cur + std::min(n, 2)) & 3;
+    p.mv = (p.mv + 1) % 3;
+  }
+  T *P(int k) const { return p_.as<T>() + (int64_t)(k & 3) * ns_ * N_; }
+  T *PSX(int k) const { return psix_.as<T>() + (int64_t)(k % 3) * ns_ * spx_; }
+  T *PSZ(int k) const { return psiz_.as<T>() + (int64_t)(k % 3) * ns_ * spz_; }
+  T *XIX(int k) const { return xix_.as<T>() + (int64_t)(k % 3) * ns_ * sxx_; }
+  T *XIZ(int k) const { return xiz_.as<T>() + (int64_t)(k % 3) * ns_ * sxz_; }
+  T *A(int k) const { return a_.as<T>() + (int64_t)(k & 3) * ns_ * N_; }
+  T *APSX(int k) const { return apsix_.as<T>() + (int64_t)(k % 3) * ns_ * spx_; }
+  T *APSZ(int k) const { return apsiz_.as<T>() + (int64_t)(k % 3) * ns_ * spz_; }
+  T *AXIX(int k) const { return axix_.as<T>() + (int64_t)(k % 3) * ns_ * sxx_; }
+  T *AXIZ(int k) const { return axiz_.as<T>() + (int64_t)(k % 3) * ns_ * sxz_; }
+
+  // Levels of the next launch when `left` remain: launches of nearly equal
+  // size, none above steps_.
+  int levels(int left) const {
+    const int launches = (int)ceil_div(left, steps_);
+    return (int)ceil_div(left, launches);
+  }
+
+  // Windows of a launch of n levels over the batch, H rows each.
+  int64_t windows(int H, int n) const {
+    return std::max<int64_t>(ceil_div(nx_ - 2 * n, TX - 2 * n), 1) *
+           std::max<int64_t>(ceil_div(nz_ - 2 * n, H - 2 * n), 1) * nsh_;
+  }
+
+  // Levels per launch: as many as a window can step, since a launch costs 5-7
+  // us (loads, stores, the gap to the next one) whatever it steps and a level
+  // 1-3 us: 8 levels are the fastest everywhere from 121 x 101 cells to
+  // 4 x 2000 x 1000 (4 levels: 1.1 to 1.6 times as long per level).
+  // Window shape, us per level measured forward / adjoint:
+  //   2 (16 waves, 2 rows per thread, 32 rows): the shortest level, for grids
+  //     that leave CUs idle.  f32 201 x 151: 2.1 / 1.5 against 2.5 / 2.1 in
+  //     shape 1; 500 x 400 (264 windows): 2.2 / 1.7 against 2.5 / 2.1;
+  //     4 x 300 x 250 (360 windows): 2.8 / 2.7 against 2.5 / 2.3.
+  //   1 (16 waves, 4 rows, 64 rows): less work on cells that the neighbours
+  //     step too.  f32 700 x 700 (225 windows): 2.6 / 2.3 against 3.6 / 4.4
+  //     in shape 0; f64 16 x 600 x 400 forward: 15.7 against 23.8 in shape 2.
+  //     The f64 adjoint spills in it (37.8 against 25.6) and stays in shape 2.
+  //   0 (8 waves, 8 rows, 64 rows): f32 forward with more windows of 64 rows
+  //     than CUs, two blocks to a CU: 16 x 600 x 400: 9.6 against 11.3 in
+  //     shape 1; the f32 adjoint spills (19.7 against 11.6).
+  void choose_steps() {
+    steps_ = steps_env_ ? steps_env_ : SN_MAX;
+    const bool small = windows(32, SN_MAX) <= 300, many = windows(64, SN_MAX) > 256;
+    shape_[0] = small ? 2 : many && sizeof(T) == 4 ? 0 : 1;
+    shape_[1] = small || sizeof(T) == 8 ? 2 : 1;
+    if (shape_env_ >= 0) {
+      shape_[0] = shape_env_ % 10;
+      shape_[1] = shape_env_ / 10;
+    }
+  }
 
   void zero_forward_state() {
+    f_ = Pos{};
     SWX_HIP(hipMemsetAsync(p_.get(), 0, p_.bytes(), c_.stream));
     SWX_HIP(hipMemsetAsync(psix_.get(), 0, psix_.bytes(), c_.stream));
     SWX_HIP(hipMemsetAsync(psiz_.get(), 0, psiz_.bytes(), c_.stream));
@@ -901,31 +1076,13 @@ class Cd2dEngine final : public Engine {
     SWX_HIP(hipGetLastError());
   }
 
-  // Rows per thread (1, 2 or 4) timed on step 1 of the zero initial state,
-  // which every repetition recomputes identically (all stencil inputs are
-  // zero; the new level is the injection alone).  Every choice gives
-  // bitwise the same results.
-  void tune_rows(bool save, T *tr) {
-    static const int rows[3] = {2, 1, 4};
-    Cd2dStepArgs<T> a = fwd_args(1, 0, save ? 1 : 0, 0, tr);
-    a.lean = lean_ ? 1 : 0;
-    const int k = fastest_candidate(c_.stream, 3, [&](int c) {
-      if (rows[c] == 4) launch_rows<4>(a);
-      else if (rows[c] == 1) launch_rows<1>(a);
-      else launch_rows<2>(a);
-      SWX_HIP(hipGetLastError());
-    });
-    rows_ = rows[k];
-    tuned_ = true;
-  }
-
   Cd2dStepArgs<T> fwd_args(int it, int act_min, int dmode, int cbase, T *traces) const {
     Cd2dStepArgs<T> a = base_args(it);
-    a.pold = P(it - 2); a.pcur = P(it - 1); a.pnew = P(it);
-    a.psix_o = PSX(it - 1); a.psix_n = PSX(it);
-    a.psiz_o = PSZ(it - 1); a.psiz_n = PSZ(it);
-    a.xix_o = XIX(it - 1); a.xix = XIX(it);
-    a.xiz_o = XIZ(it - 1); a.xiz = XIZ(it);
+    a.pold = P(f_.cur + 3); a.pcur = P(f_.cur); a.pnew = P(f_.cur + 1);
+    a.psix_o = PSX(f_.mv); a.psix_n = PSX(f_.mv + 1);
+    a.psiz_o = PSZ(f_.mv); a.psiz_n = PSZ(f_.mv + 1);
+    a.xix_o = XIX(f_.mv); a.xix = XIX(f_.mv + 1);
+    a.xiz_o = XIZ(f_.mv); a.xiz = XIZ(f_.mv + 1);
     a.act_min = act_min;
     a.dmode = c_.d.gradient ? dmode : 0;
     a.cbase = cbase;
@@ -934,70 +1091,57 @@ class Cd2dEngine final : public Engine {
     return a;
   }
 
-  void step_fwd(int it, int act_min, int dmode, int cbase, T *traces) {
-    launch(fwd_args(it, act_min, dmode, cbase, traces));
-  }
-
-  // levels it and it+1 in one launch (cd2d_step2_kernel)
-  Cd2dStep2Args<T> step2_args(int it, int act_min, int dmode, int cbase, T *traces) const {
-    Cd2dStep2Args<T> b;
-    b.a = fwd_args(it, act_min, dmode, cbase, traces);
-    b.a.lean = lean_ ? 1 : 0;
-    b.a.nbx = (int)ceil_div(nx_, TX);
-    b.a.nby = (int)ceil_div(nz_, S2H);
-    b.pnew2 = P(it + 1);
-    b.psix_n2 = PSX(it + 1);
-    b.psiz_n2 = PSZ(it + 1);
-    b.xix_n2 = XIX(it + 1);
-    b.xiz_n2 = XIZ(it + 1);
-    return b;
-  }
-  template <bool ADJ>
-  void launch_step2(const Cd2dStep2Args<T> &b, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr) {
-    const unsigned nb = (unsigned)((int64_t)b.a.nbx * b.a.nby * nsh_);
-    hipExtLaunchKernelGGL(cd2d_step2_kernel<T, ADJ>, dim3(nb), dim3(TX, TZ), 0, c_.stream, e0, e1, 0, b);
-  }
-  void step2_fwd(int it, int act_min, int dmode, int cbase, T *traces) {
+  template <int R, int NW, bool ADJ>
+  void launch_shape(Cd2dStepNArgs<T> &A) {
+    constexpr int H = NW * R;
+    A.a.nbx = (int)std::max<int64_t>(ceil_div(nx_ - 2 * A.n, TX - 2 * A.n), 1);
+    A.a.nby = (int)std::max<int64_t>(ceil_div(nz_ - 2 * A.n, H - 2 * A.n), 1);
     hipEvent_t e0, e1;
-    c_.ktimer.dispatch_events(0, &e0, &e1);
-    launch_step2<false>(step2_args(it, act_min, dmode, cbase, traces), e0, e1);
+    c_.ktimer.dispatch_events(ADJ ? 1 : 0, &e0, &e1);
+    hipExtLaunchKernelGGL((cd2d_stepn_kernel<T, R, NW, ADJ>), dim3((unsigned)((int64_t)A.a.nbx * A.a.nby * nsh_)),
+                          dim3(NW * TX), 0, c_.stream, e0, e1, 0, A);
     SWX_HIP(hipGetLastError());
   }
-
-  // One level per launch (two launches of the tuned row count) against two
-  // levels per launch, timed on levels 1 and 2 of the zero initial state,
-  // which every repetition recomputes identically.  Both give bitwise the
-  // same results; SWX_CD2D_STEPS pins the choice.
-  void tune_steps(bool save, T *tr) {
-    steps_tuned_ = true;
-    if (steps_env_ || ntmax_ < 2) return;
-    Cd2dStepArgs<T> a1 = fwd_args(1, 0, save ? 1 : 0, 0, tr), a2 = fwd_args(2, 0, save ? 1 : 0, 0, tr);
-    a1.lean = a2.lean = lean_ ? 1 : 0;
-    const Cd2dStep2Args<T> b = step2_args(1, 0, save ? 1 : 0, 0, tr);
-    auto one = [&](Cd2dStepArgs<T> x) {
-      if (rows_ == 4) launch_rows<4>(x);
-      else if (rows_ == 1) launch_rows<1>(x);
-      else launch_rows<2>(x);
-    };
-    const int k = fastest_candidate(c_.stream, 2, [&](int c) {
-      if (c == 0) {
-        one(a1);
-        one(a2);
-      } else {
-        launch_step2<false>(b);
+  template <bool ADJ>
+  void launch_stepn(const Cd2dStepArgs<T> &a, T *pnew0, int n) {
+    Cd2dStepNArgs<T> A;
+    A.a = a;
+    A.pnew0 = pnew0;
+    A.n = n;
+    const int shape = shape_[ADJ];
+    if (shape == 2) {
+      launch_shape<2, 16, ADJ>(A);
+      return;
+    }
+    if constexpr (sizeof(T) == 4 || !ADJ) {
+      if (shape == 1) {
+        launch_shape<4, 16, ADJ>(A);
+        return;
       }
-      SWX_HIP(hipGetLastError());
-    });
-    steps_ = k == 0 ? 1 : 2;
+    }
+    if constexpr (sizeof(T) == 4 && !ADJ) launch_shape<8, 8, ADJ>(A);
+  }
+
+  // forward / replay levels it .. it+n-1
+  void step_fwd(int it, int n, int act_min, int dmode, int cbase, T *traces) {
+    Cd2dStepArgs<T> a = fwd_args(it, act_min, dmode, cbase, traces);
+    if (steps_ == 1) {
+      launch(a);
+    } else {
+      T *older = a.pnew;
+      if (n > 1) a.pnew = P(f_.cur + 2);
+      launch_stepn<false>(a, older, n);
+    }
+    advance(f_, n);
   }
 
   Cd2dStepArgs<T> adj_args(int it, int cbase) const {
     Cd2dStepArgs<T> a = base_args(it);
-    a.pold = A(it + 2); a.pcur = A(it + 1); a.pnew = A(it);
-    a.psix_o = APSX(it + 1); a.psix_n = APSX(it);
-    a.psiz_o = APSZ(it + 1); a.psiz_n = APSZ(it);
-    a.xix_o = AXIX(it + 1); a.xix = AXIX(it);
-    a.xiz_o = AXIZ(it + 1); a.xiz = AXIZ(it);
+    a.pold = A(b_.cur + 3); a.pcur = A(b_.cur); a.pnew = A(b_.cur + 1);
+    a.psix_o = APSX(b_.mv); a.psix_n = APSX(b_.mv + 1);
+    a.psiz_o = APSZ(b_.mv); a.psiz_n = APSZ(b_.mv + 1);
+    a.xix_o = AXIX(b_.mv); a.xix = AXIX(b_.mv + 1);
+    a.xiz_o = AXIZ(b_.mv); a.xiz = AXIZ(b_.mv + 1);
     a.act_min = 0;
     a.dmode = 0;
     a.cbase = cbase;
@@ -1007,70 +1151,32 @@ class Cd2dEngine final : public Engine {
     a.res = c_.pts.d_res.as<T>();
     return a;
   }
-  void step_adj(int it, int cbase) { launch(adj_args(it, cbase)); }
-
-  // adjoint levels it and it-1 in one launch
-  Cd2dStep2Args<T> adj2_args(int it, int cbase) const {
-    Cd2dStep2Args<T> b;
-    b.a = adj_args(it, cbase);
-    b.a.lean = lean_ ? 1 : 0;
-    b.a.nbx = (int)ceil_div(nx_, TX);
-    b.a.nby = (int)ceil_div(nz_, S2H);
-    b.pnew2 = A(it - 1);
-    b.psix_n2 = APSX(it - 1);
-    b.psiz_n2 = APSZ(it - 1);
-    b.xix_n2 = AXIX(it - 1);
-    b.xiz_n2 = AXIZ(it - 1);
-    return b;
-  }
-  void step2_adj(int it, int cbase) {
-    hipEvent_t e0, e1;
-    c_.ktimer.dispatch_events(1, &e0, &e1);
-    launch_step2<true>(adj2_args(it, cbase), e0, e1);
-    SWX_HIP(hipGetLastError());
-  }
-
-  // Adjoint levels per launch, timed like tune_steps on the top two levels
-  // of the first segment before the adjoint state and the gradient are
-  // cleared (what the timed launches write is discarded).
-  void tune_adj_steps() {
-    adj_steps_tuned_ = true;
-    adj_steps_ = steps_;
-    if (steps_env_ || ntmax_ < 2 || S_ < 2) return;
-    const int it = std::min(S_, ntmax_);
-    Cd2dStepArgs<T> a1 = adj_args(it, 0), a2 = adj_args(it - 1, 0);
-    a1.lean = a2.lean = lean_ ? 1 : 0;
-    const Cd2dStep2Args<T> b = adj2_args(it, 0);
-    auto one = [&](Cd2dStepArgs<T> x) {
-      if (rows_ == 4) launch_rows<4>(x);
-      else if (rows_ == 1) launch_rows<1>(x);
-      else launch_rows<2>(x);
-    };
-    const int k = fastest_candidate(c_.stream, 2, [&](int c) {
-      if (c == 0) {
-        one(a1);
-        one(a2);
-      } else {
-        launch_step2<true>(b);
-      }
-      SWX_HIP(hipGetLastError());
-    });
-    adj_steps_ = k == 0 ? 1 : 2;
+  // adjoint levels it .. it-n+1
+  void step_adj(int it, int n, int cbase) {
+    Cd2dStepArgs<T> a = adj_args(it, cbase);
+    if (steps_ == 1) {
+      launch(a);
+    } else {
+      T *older = a.pnew;
+      if (n > 1) a.pnew = A(b_.cur + 2);
+      launch_stepn<true>(a, older, n);
+    }
+    advance(b_, n);
   }
 
   // checkpoint layout (all shots): p^{c-1} | p^c | psi_x | psi_z | xi_x | xi_z
-  void ckpt_copy(int k, int cb, bool save) {
+  void ckpt_copy(int k, bool save) {
     const int64_t e = sizeof(T);
     char *base = ck_.as<char>() + (int64_t)(k - 1) * ck_bytes_one_;
     const int64_t fb = (int64_t)ns_ * N_ * e;
     struct Part { void *dev; int64_t bytes; };
     Part parts[6] = {
-        {P(cb - 1), fb},
-        {P(cb), fb},
-        {PSX(cb), ns_ * spx_ * e},
-        {PSZ(cb), ns_ * spz_ * e},
-        {XIX(cb), ns_ * sxx_ * e},
-        {XIZ(cb), ns_ * sxz_ * e},
+        {P(f_.cur + 3), fb},
+        {P(f_.cur), fb},
+        {PSX(f_.mv), ns_ * spx_ * e},
+        {PSZ(f_.mv), ns_ * spz_ * e},
+        {XIX(f_.mv), ns_ * sxx_ * e},
+        {XIZ(f_.mv), ns_ * sxz_ * e},
     };
     int64_t off = 0;
     for (auto &pt : parts) {
@@ -1083,12 +1189,12 @@ class Cd2dEngine final : public Engine {
       off += pt.bytes;
     }
   }
-  void save_ckpt(int k, int it) { ckpt_copy(k, it, true); }
-  void restore_ckpt(int k, int cb) {
+  void save_ckpt(int k) { ckpt_copy(k, true); }
+  void restore_ckpt(int k) {
     if (k == 0) {
       zero_forward_state();
     } else {
-      ckpt_copy(k, cb, false);
+      ckpt_copy(k, false);
     }
   }
 
@@ -1096,11 +1202,10 @@ class Cd2dEngine final : public Engine {
   int nx_, nz_, h_, ns_;
   int64_t N_, spx_, spz_, sxx_, sxz_;
   int cstride_;
-  int rows_ = 2;
-  bool tuned_ = false;   // rows_ chosen (by SWX_CD2D_ROWS or tune_rows)
-  int steps_ = 1;        // levels per forward / replay launch
-  int adj_steps_ = 1;    // levels per adjoint launch
-  bool steps_env_ = false, steps_tuned_ = false, adj_steps_tuned_ = false;
+  int rows_ = 2;         // rows per thread of cd2d_step_kernel
+  int steps_ = 1, shape_[2] = {0, 0};     // most levels per launch, block shapes (forward, adjoint)
+  int steps_env_ = 0, shape_env_ = -1;    // pinned by the environment (0, -1: not)
+  Pos f_, b_;                             // forward and adjoint state
   bool lean_ = true;
   DevBuf fact_, p_, psix_, psiz_, xix_, xiz_, cpml_;
   DevBuf a_, apsix_, apsiz_, axix_, axiz_, grad_, gout_;
