@@ -45,19 +45,45 @@ def coeffsinc1d(x0, dx, nx, r=KAISER_R, beta=KAISER_BETA, xstart=0.0, mirror=Fal
     return uniq.astype(np.int64), w
 
 
+def _axis_taps(x, dx, nx, r, beta, xstart, mirror, xbl, xbr):
+    """coeffsinc1d of every coordinate of x, with the same arithmetic on all
+    of them at once (a gather of hundreds of receivers spends its time in
+    the window's Bessel functions otherwise: 0.11 ms a coordinate one by one,
+    5 us together).  Coordinates whose taps fold back over a boundary go
+    through coeffsinc1d."""
+    x = np.asarray(x, dtype=np.float64)
+    # nearest grid point, the first of two at the same distance
+    i0 = np.clip(np.floor((x - xstart) / dx + 0.5).astype(np.int64), 0, nx - 1)
+    cand = np.clip(i0[:, None] + np.arange(-1, 2), 0, nx - 1)
+    i0 = cand[np.arange(len(x)), np.argmin(np.abs(x[:, None] - (xstart + dx * cand)), axis=1)] + 1
+    idx = i0[:, None] + np.arange(-r - 1, r + 2)
+    xc = (idx - 1) * dx + xstart
+    d = xc - x[:, None]
+    rr = r * dx
+    win = np.where(np.abs(d) <= rr, np.i0(beta * np.sqrt(np.clip(1.0 - (d / rr) ** 2, 0.0, None))) / np.i0(beta), 0.0)
+    coe = win * np.sinc(d / dx)
+    keep = ~(np.abs(coe) <= 1e-15)
+    folded = np.any(keep & ((xc < xbl) | (xc > xbr)), axis=1)
+    return [coeffsinc1d(x[p], dx, nx, r, beta, xstart, mirror, xbl, xbr) if folded[p]
+            else (idx[p][keep[p]], coe[p][keep[p]]) for p in range(len(x))]
+
+
 def spread_positions(positions, spacing, gridsize, shift=(0.0, 0.0), mirror=False, r=KAISER_R, beta=KAISER_BETA):
     """spread_positions with freesurfposition=:ongridbound: per point, the
     taps (ntaps, 2) 1-based and their weights, first dimension fastest."""
     positions = np.atleast_2d(np.asarray(positions, dtype=np.float64))
-    ndim = positions.shape[1]
+    per = []
+    for d in range(positions.shape[1]):
+        # points often share a coordinate (a line of receivers at one depth)
+        x, inv = np.unique(positions[:, d], return_inverse=True)
+        taps = _axis_taps(x, spacing[d], gridsize[d], r, beta, shift[d], mirror, 0.0, (gridsize[d] - 1) * spacing[d])
+        per.append([taps[k] for k in inv.ravel()])
     out = []
-    for p in positions:
-        per = [coeffsinc1d(p[d], spacing[d], gridsize[d], r, beta, shift[d], mirror, 0.0,
-                           (gridsize[d] - 1) * spacing[d]) for d in range(ndim)]
-        ii, jj = np.meshgrid(per[0][0], per[1][0], indexing="ij")
-        wi, wj = np.meshgrid(per[0][1], per[1][1], indexing="ij")
-        ij = np.stack([ii.ravel(order="F"), jj.ravel(order="F")], axis=1)
-        out.append((ij, (wi * wj).ravel(order="F")))
+    for (ii, wi), (jj, wj) in zip(per[0], per[1]):
+        ij = np.empty((len(ii) * len(jj), 2), dtype=np.int64)
+        ij[:, 0] = np.tile(ii, len(jj))
+        ij[:, 1] = np.repeat(jj, len(ii))
+        out.append((ij, (wj[:, None] * wi).ravel()))
     return out
 
 
