@@ -185,12 +185,12 @@ class _AcousticCPMLWaveSimulation:
                  & (positions <= np.array([e - b for e, b in zip(extent, edge)], dtype=T)))
         if self.cpmlparams.freeboundtop:
             clear[:, N - 1] = True
-        for p, inn, clr in zip(positions, inside, clear):
-            if not (inn.all() and clr.all()):
-                for c in range(N):
-                    assert inn[c], f"Position {p} is not inside the grid!"
-                    if not clr[c]:
-                        self.runparams.logger.warning("Position %s is inside the CPML region!", p)
+        for k in np.flatnonzero(~(inside & clear).all(axis=1)):
+            p = positions[k]
+            for c in range(N):
+                assert inside[k, c], f"Position {p} is not inside the grid!"
+                if not clear[k, c]:
+                    self.runparams.logger.warning("Position %s is inside the CPML region!", p)
 
     def check_shot(self, shot):
         self.check_numerics(shot)
