@@ -453,6 +453,8 @@ def kernel_names(physics, variant):
     if physics == "cd3d":
         # [launch shape, planes per z chunk]
         v = variant[0] or 4
+        if v > 300:   # a row of 64 columns per wave
+            return "cd3d_row_kernel<float, false> (forward)", "cd3d_row_kernel<float, true> (adjoint)"
         if v > 200:   # one launch, interior march staged through LDS
             k = f"cd3d_step_kernel<float, {v - 200}, 3>"
         elif v > 100:   # interior tiles and the others in two launches

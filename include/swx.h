@@ -161,8 +161,8 @@ typedef struct {
    * codes (0/1 stress and displacement launches, 2 one fused launch); CD 2D
    * [window shapes (or, with one level per launch, rows per thread), most
    * levels per launch], each 10 x adjoint + forward; CD 3D
-   * [launch shape 8/4/2/108/104/102/208/204/202, planes per z chunk]; 0
-   * where there is one shape. */
+   * [301 row march, 8/4/2/108/104/102/208/204/202 tiles; planes per z
+   * chunk]; 0 where there is one shape. */
   int32_t kernel_variant[2];
 } swx_plan_info;
 

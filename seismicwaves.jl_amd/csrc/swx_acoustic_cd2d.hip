@@ -322,22 +322,6 @@ struct Cd2dStepNArgs {
   int n;               // levels
 };
 
-// Value of the lane before / after (0 beyond the wave's ends).
-template <int CTRL>
-__device__ __forceinline__ float lane_shift(float x) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true));
-}
-template <int CTRL>
-__device__ __forceinline__ double lane_shift(double x) {
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, 0xf, 0xf, true);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, 0xf, 0xf, true);
-  return __hiloint2double(hi, lo);
-}
-template <typename T>
-__device__ __forceinline__ T lane_before(T x) { return lane_shift<0x138>(x); }   // wave_shr:1
-template <typename T>
-__device__ __forceinline__ T lane_after(T x) { return lane_shift<0x130>(x); }    // wave_shl:1
-
 template <typename T, int R, int NW>
 struct Cd2dNLds {
   T first[2][NW][TX], last[2][NW][TX], lastz[2][NW][TX];   // rows 0 and R-1 of p, row R-1 of psi_z
@@ -471,15 +455,6 @@ __device__ __forceinline__ void cd2d_n_level(const Cd2dStepArgs<T> &a, const Cd2
     G.pc[r] = pnv;
     if (!ADJ) dv[r] = dval;
   }
-}
-
-// Makes x opaque: the compiler otherwise keeps what follows from it for every
-// row (tests, addresses) in scalar registers over the levels, spills them and
-// pays a lane read for each use, more than computing it again.
-// (x is the same in all lanes of the wave.)
-__device__ __forceinline__ void opaque(int &x) {
-  x = __builtin_amdgcn_readfirstlane(x);
-  asm volatile("" : "+s"(x));
 }
 
 // Points of the wave's rows: the cells' entries in LDS, and (injected points)

@@ -9,7 +9,9 @@
 //   driver     src/models/acoustic/acou_gradient.jl:4-95
 //   correlate  src/models/acoustic/backends/shared/correlate_gradient_xPU.jl:1-10
 //
-// Kernel shape: a block is a 64 x 4 column tile of the (x, y) plane that
+// A step is launched as the row march (cd3d_row_kernel, described there).
+// Fields of 4 GiB per shot and more, which its 32-bit offsets do not reach,
+// take the tile kernels: a block is a 64 x 4 column tile of the (x, y) plane that
 // marches along z (the slow axis) over a chunk of planes.  Each thread keeps
 // p(k-1), p(k), p(k+1) in registers and rotates them, so the z neighbours
 // and the current plane are read from HBM once; x/y neighbours come from
@@ -27,6 +29,7 @@
 //   grad    [ns][N]
 #include <algorithm>
 #include <cstdlib>
+#include <type_traits>
 
 #include "swx_device.hpp"
 #include "swx_internal.hpp"
@@ -582,6 +585,374 @@ __global__ __launch_bounds__(TX *TY) void cd3d_step_kernel(Cd3dArgs<T> a) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// Row march (cd3d_row_kernel)
+//
+// A wave steps one row of 64 cells along x and marches along z over a chunk of
+// planes; a block is RM_W rows.  x neighbours come from the adjacent lanes (a
+// window owns 62 of its 64 columns, all of them up to a grid side), z
+// neighbours from the planes before and after, y neighbours from the block's
+// other row through LDS (against a load of both by every wave, us per step
+// forward / adjoint: 812 / 1315 for 825 / 1392 at 600 x 600 x 400 float32, 28 /
+// 39 for 29 / 40 at 129 x 117 x 91 float64; four and eight rows are no better,
+// their barrier couples more waves).
+// The row is the same for all lanes, so that everything but the x strips is
+// decided per wave: the C-PML variables, like the fields, are loaded two
+// planes ahead without per-cell tests, and points are dealt with after the
+// march, in the planes that one load at the start has found to hold any.
+// The tile kernels above decide all that per cell; they issue several times
+// the instructions and load a plane's strips only once they are needed.  us
+// per step, tile / row march, forward with history and adjoint: 129 x 117 x 91
+// float64 47 / 28 and 49 / 39; 300 x 280 x 200 float32 199 / 123 and 217 / 184;
+// 600 x 600 x 400 float32 1009 / 812 (4.2 TB/s of the 24 bytes per cell that
+// it cannot do without) and 1307 / 1315.  What bounds the march at 300 x 280 x
+// 200: 0.5 of the wave cycles wait on memory at 4 waves per SIMD, the address
+// units are busy 0.65 of the time (rows start at any alignment, so that a
+// window touches three cache lines instead of two), and a quarter of the cells
+// have strips to step besides.
+// Expressions are those of cd3d_step_kernel: results are bitwise the same.
+constexpr int RM_W = 2;      // rows (waves) per block
+
+template <typename T>
+struct Cd3dPlane {
+  T pc, px, po, fa, g, d;                // row j of the level, the row beyond the block, the rest of row j
+  T psx, xix, psy0, psy, xiy, psz, xiz;  // psy0: psi_y of the row before the block
+};
+
+template <typename T>
+struct Cd3dRowLds {
+  T p[2][RM_W][TX], psy[2][RM_W][TX];    // by parity of the plane
+};
+
+// Points of row `row` (cells [c0, c0 + 64)): the unique point of each lane's
+// cell, or -1.
+__device__ __forceinline__ int cd3d_row_points(const int *rowp, const int64_t *cell, int64_t row, int64_t c0,
+                                               int lane) {
+  const int q0 = __builtin_amdgcn_readfirstlane(rowp[row]), q1 = __builtin_amdgcn_readfirstlane(rowp[row + 1]);
+  int u = 0;
+  for (int q = q0; q < q1; q += TX) {
+    const int64_t o = q + lane < q1 ? cell[q + lane] - c0 : -1;
+    const bool hit = o >= 0 && o < TX;
+    // lanes with a point send its number to the lane of its cell
+    for (uint64_t m = __ballot(hit); m; m &= m - 1) {
+      const int from = __builtin_ctzll(m);
+      const int to = __shfl((int)o, from);
+      if (lane == to) u = q + from + 1;
+    }
+  }
+  return u - 1;
+}
+
+// Element of an array at a 32-bit byte offset: base in scalar registers, one
+// vector add per offset (a 64-bit index per row and array costs a dozen scalar
+// instructions, and the four SIMDs of a CU share one scalar unit).
+template <typename T>
+__device__ __forceinline__ T ld_off(const T *base, unsigned off) {
+  return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + off);
+}
+template <typename T>
+__device__ __forceinline__ void st_off(T *base, unsigned off, T v) {
+  *reinterpret_cast<T *>(reinterpret_cast<char *>(base) + off) = v;
+}
+
+// A uniform value of plane m of the chunk, held by lane m.
+__device__ __forceinline__ float lane_value(float x, int m) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), m));
+}
+__device__ __forceinline__ double lane_value(double x, int m) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), m),
+                          __builtin_amdgcn_readlane(__double2loint(x), m));
+}
+
+// XS, YS: the window, some row of the block is in a strip or at an edge.
+template <typename T, bool XS, bool YS, bool CORR>
+__device__ __forceinline__ void cd3d_row_march(const Cd3dArgs<T> &a, int s, Cd3dRowLds<T> &lds, int X0, int j, int w,
+                                               int K0, int K1, bool own, int dslot) {
+  constexpr unsigned E = sizeof(T);
+  const int nx = a.n[0], ny = a.n[1], nz = a.n[2], h = a.h;
+  const int lane = threadIdx.x & (TX - 1), i = X0 + lane;
+  const unsigned ic = min(i, nx - 1);
+  const unsigned plane = (unsigned)nx * ny * E;
+  const int64_t so = (int64_t)s * a.N;
+  const T *cb = a.cpml + (int64_t)s * a.cstride;
+  const AxisCoef<T> cx = axis_coef(cb, h, 0), cy = axis_coef(cb, h, 1), cz = axis_coef(cb, h, 2);
+  const T *pc_ = a.pcur + so, *po_ = a.pold + so;
+  T *pn_ = a.pnew + so, *g_ = a.grad + so, *dn_ = dslot >= 0 ? a.dbuf + (int64_t)dslot * a.dslot + so : nullptr;
+  const T *dc_ = CORR ? a.dbuf + (int64_t)(a.it - a.cbase) * a.dslot + so : nullptr;
+  // x strip: entry of the column, its coefficients
+  const int kx = XS ? psi_owner(i, nx, h) : -1;
+  const bool xin = !XS || (i >= 1 && i <= nx - 2), xst = XS && xin && (i < h || i >= nx - h);
+  const unsigned kxc = max(kx, 0);
+  T xc[4] = {T(0), T(0), T(0), T(0)};
+  if (XS && kx >= 0) {
+    xc[0] = cx.bh(kx);
+    xc[1] = cx.ah(kx);
+    xc[2] = cx.b(kx);
+    xc[3] = cx.a(kx);
+  }
+  // y strip: entry of the row, coefficients of the entry and of the one before
+  const int ky = YS ? psi_owner(j, ny, h) : -1;
+  const bool yin = !YS || (j >= 1 && j <= ny - 2), yst = YS && yin && (j < h || j >= ny - h);
+  T yc[6] = {T(0), T(0), T(0), T(0), T(0), T(0)};
+  if (YS && ky >= 0) {
+    yc[0] = cy.bh(ky);
+    yc[1] = cy.ah(ky);
+    yc[2] = cy.b(ky);
+    yc[3] = cy.a(ky);
+    if (yst) {
+      yc[4] = cy.bh(ky - 1);
+      yc[5] = cy.ah(ky - 1);
+    }
+  }
+  // z strips: lane m holds the coefficients of plane K0 + m
+  T zl[4] = {T(0), T(0), T(0), T(0)};
+  uint64_t zown, zin, zst;      // planes with a psi_z, inside the z edges, with a xi_z
+  {
+    const int k = K0 + lane, kl = k < K1 ? psi_owner(k, nz, h) : -1;
+    if (kl >= 0) {
+      zl[0] = cz.bh(kl);
+      zl[1] = cz.ah(kl);
+      zl[2] = cz.b(kl);
+      zl[3] = cz.a(kl);
+    }
+    zown = __ballot(kl >= 0);
+    zin = __ballot(k >= 1 && k <= nz - 2);
+    zst = __ballot(k >= 1 && k <= nz - 2 && (k < h || k >= nz - h));
+  }
+  const T *psx_ = a.psi_o[0] + (int64_t)s * a.sps[0], *psy_ = a.psi_o[1] + (int64_t)s * a.sps[1],
+          *psz_ = a.psi_o[2] + (int64_t)s * a.sps[2];
+  T *psxn_ = a.psi_n[0] + (int64_t)s * a.sps[0], *psyn_ = a.psi_n[1] + (int64_t)s * a.sps[1],
+    *pszn_ = a.psi_n[2] + (int64_t)s * a.sps[2];
+  T *xx_ = a.xi[0] + (int64_t)s * a.sxi[0], *xy_ = a.xi[1] + (int64_t)s * a.sxi[1],
+    *xz_ = a.xi[2] + (int64_t)s * a.sxi[2];
+  // byte offsets in plane 0, and planes of psi and xi
+  const unsigned oc = ((unsigned)j * nx + ic) * E;
+  const unsigned ox = ((unsigned)j * (2 * h) + kxc) * E, oxx = ((unsigned)j * (2 * h + 2) + kxc) * E;
+  const unsigned oy = ((unsigned)max(ky, 0) * nx + ic) * E;
+  // the row beyond the block and psi_y of the row before it: the other waves
+  // make the load too, of one word
+  const T *px_ = w == 0 || w == RM_W - 1 ? pc_ : a.fact, *psy0_ = w == 0 && ky > 0 ? psy_ : a.fact;
+  const unsigned opx = w == 0 || w == RM_W - 1 ? ((unsigned)(w == 0 ? max(j - 1, 0) : min(j + 1, ny - 1)) * nx + ic) * E : 0,
+                 kpx = w == 0 || w == RM_W - 1 ? plane : 0;
+  const unsigned ppx = (unsigned)ny * (2 * h) * E, pxx = (unsigned)ny * (2 * h + 2) * E;
+  const unsigned ppy = (unsigned)nx * (2 * h) * E, pxy = (unsigned)nx * (2 * h + 2) * E;
+  const unsigned opy0 = w == 0 && ky > 0 ? oy - nx * E : 0, kpy0 = w == 0 && ky > 0 ? ppy : 0;
+  auto zentry = [&](int k) { return (unsigned)(k < h ? k : k + 1 - nz + 2 * h); };
+  auto load = [&](int k_) {
+    Cd3dPlane<T> q;
+    const unsigned k = min(k_, nz - 1), kb = k * plane;
+    q.pc = ld_off(pc_, oc + kb);
+    q.px = ld_off(px_, opx + k * kpx);
+    q.po = ld_off(po_, oc + kb);
+    q.fa = ld_off(a.fact, oc + kb);
+    if (CORR) {
+      q.g = ld_off(g_, oc + kb);
+      q.d = ld_off(dc_, oc + kb);
+    }
+    if (XS && h > 0) {
+      q.psx = ld_off(psx_, ox + k * ppx);
+      q.xix = ld_off(xx_, oxx + k * pxx);
+    }
+    if (YS && h > 0) {
+      q.psy0 = ld_off(psy0_, opy0 + k * kpy0);
+      q.psy = ld_off(psy_, oy + k * ppy);
+      q.xiy = ld_off(xy_, oy + k * pxy);
+    }
+    if (zown >> (k_ - K0) & 1) {
+      const unsigned zb = zentry(k_) * plane;
+      q.psz = ld_off(psz_, oc + zb);
+      q.xiz = ld_off(xz_, oc + zb);
+    }
+    return q;
+  };
+
+  T pm = ld_off(pc_, oc + max(K0 - 1, 0) * plane), pszp = 0;      // plane k-1: pressure, new psi_z
+  if (K0 > 0) {
+    const int kn = psi_owner(K0 - 1, nz, h);
+    if (kn >= 0) {
+      const T d = (ld_off(pc_, oc + K0 * plane) - pm) * a.id[2];
+      pszp = cz.bh(kn) * ld_off(psz_, oc + kn * plane) + cz.ah(kn) * d;
+    }
+  }
+  // plane k (q), pp: the pressure of the one after it
+  auto step = [&](int k, const Cd3dPlane<T> &q, T pp) {
+    const int m = k - K0;
+    const T pc = q.pc;
+    auto &lp = lds.p[m & 1];
+    auto &ly_ = lds.psy[m & 1];
+    lp[w][lane] = pc;
+    if (YS && h > 0) ly_[w][lane] = q.psy;
+    __syncthreads();
+    T pd = lp[max(w - 1, 0)][lane], pu = lp[min(w + 1, RM_W - 1)][lane], psy0 = 0;
+    if (w == 0) pd = q.px;
+    if (w == RM_W - 1) pu = q.px;
+    if (YS && h > 0) psy0 = w == 0 ? q.psy0 : ly_[max(w - 1, 0)][lane];
+    const T pl = lane_before(pc), pr = lane_after(pc);
+    const T d2x = (pl - T(2) * pc + pr) * a.id2[0];
+    const T d2y = (pd - T(2) * pc + pu) * a.id2[1];
+    const T d2z = (pm - T(2) * pc + pp) * a.id2[2];
+    T lx = d2x, ly = d2y, lz = d2z;
+    const bool interior = xin && yin && (zin >> m & 1);
+    const bool zo = zown >> m & 1;
+    T psx = 0, xix = 0, psy = 0, xiy = 0, psz = 0, xiz = 0;      // (a xi outside the update's range keeps its value)
+    if (XS && h > 0) {
+      const T d = (pr - pc) * a.id[0];
+      psx = kx >= 0 ? xc[0] * q.psx + xc[1] * d : T(0);
+      const T psn = lane_before(psx);
+      const T dpsi = (psx - psn) * a.id[0];
+      const T x = xc[2] * q.xix + xc[3] * (d2x + dpsi);
+      xix = xst && interior ? x : q.xix;
+      lx = xst ? d2x + dpsi + x : d2x;
+    }
+    if (YS && h > 0) {
+      const T d = (pu - pc) * a.id[1];
+      psy = yc[0] * q.psy + yc[1] * d;
+      const T dp = (pc - pd) * a.id[1];
+      const T psn = yc[4] * psy0 + yc[5] * dp;
+      const T dpsi = (psy - psn) * a.id[1];
+      const T x = yc[2] * q.xiy + yc[3] * (d2y + dpsi);
+      xiy = yst && interior ? x : q.xiy;
+      ly = yst ? d2y + dpsi + x : d2y;
+    }
+    if (zo) {
+      const T d = (pp - pc) * a.id[2];
+      psz = lane_value(zl[0], m) * q.psz + lane_value(zl[1], m) * d;
+      xiz = q.xiz;
+      if (zst >> m & 1) {
+        const T dpsi = (psz - pszp) * a.id[2];
+        const T x = lane_value(zl[2], m) * q.xiz + lane_value(zl[3], m) * (d2z + dpsi);
+        xiz = interior ? x : q.xiz;
+        lz = d2z + dpsi + x;
+      }
+    }
+    const T flap = q.fa * (lx + ly + lz);
+    T pnv = T(2) * pc - q.po + flap;
+    pnv = interior ? pnv : q.po;
+    const unsigned kb = (unsigned)k * plane;
+    if (own) {
+      st_off(pn_, oc + kb, pnv);
+      // p^{it} - 2 p^{it-1} + p^{it-2}: in the interior the stencil term
+      if (dslot >= 0) st_off(dn_, oc + kb, interior ? flap : (q.po - T(2) * pc) + pnv);
+      if (CORR) st_off(g_, oc + kb, q.g + pc * q.d);
+      if (XS && kx >= 0) {
+        st_off(psxn_, ox + (unsigned)k * ppx, psx);
+        st_off(xx_, oxx + (unsigned)k * pxx, xix);
+      }
+      if (YS && ky >= 0) {
+        st_off(psyn_, oy + (unsigned)k * ppy, psy);
+        st_off(xy_, oy + (unsigned)k * pxy, xiy);
+      }
+      if (zo) {
+        const unsigned zb = zentry(k) * plane;
+        st_off(pszn_, oc + zb, psz);
+        st_off(xz_, oc + zb, xiz);
+      }
+    }
+    pszp = psz;
+    pm = pc;
+  };
+  // three plane buffers in turn: planes k+1 and k+2 are in flight while
+  // plane k is stepped
+  Cd3dPlane<T> A = load(K0), B = load(K0 + 1);
+  for (int k = K0; k < K1; k += 3) {
+    const Cd3dPlane<T> C = load(k + 2);
+    step(k, A, B.pc);
+    if (k + 1 >= K1) break;
+    A = load(k + 3);
+    step(k + 1, B, C.pc);
+    if (k + 2 >= K1) break;
+    B = load(k + 4);
+    step(k + 2, C, A.pc);
+  }
+}
+
+// Points of the planes `planes` (bits from K0) of row j, after the march: the
+// injections are added to the level that the lane stored (and to its history),
+// then receivers record it.  One copy of rarely run code, out of the march's
+// way.
+template <typename T>
+__device__ __forceinline__ void cd3d_row_finish(const Cd3dArgs<T> &a, int s, int nts, int X0, int j, int K0,
+                                                uint64_t planes, bool own, int dslot) {
+  const int nx = a.n[0], ny = a.n[1], nz = a.n[2];
+  const int lane = threadIdx.x & (TX - 1), i = X0 + lane;
+  const int64_t so = (int64_t)s * a.N, sxy = (int64_t)nx * ny;
+  const int64_t ro = (int64_t)s * (a.pt.nrows + 1);
+  const bool adj = a.res != nullptr;
+  for (; planes; planes &= planes - 1) {
+    const int k = K0 + __builtin_ctzll(planes);
+    const int64_t row = j + (int64_t)ny * k, c = k * sxy + (int64_t)j * nx + i;
+    const int u = cd3d_row_points((adj ? a.pt.rrow : a.pt.srow) + ro, adj ? a.pt.urec_cell : a.pt.usrc_cell, row,
+                                  c - lane, lane);
+    const int v = a.traces ? cd3d_row_points(a.pt.rrow + ro, a.pt.urec_cell, row, c - lane, lane) : -1;
+    if (!own || (u < 0 && v < 0)) continue;
+    T pnv = a.pnew[so + c];
+    if (u >= 0) {
+      T inj = 0;
+      if (!adj) {
+        const T *tf = a.srctf + a.pt.off_tf[s] + (a.it - 1);
+        for (int e = a.pt.usrc_ptr[u]; e < a.pt.usrc_ptr[u + 1]; e++) {
+          const T x = tf[(int64_t)nts * a.pt.usrc_list[e]];
+          pnv += x;
+          inj += x;
+        }
+      } else {
+        const T *rs = a.res + a.pt.off_tr[s] + (a.it - 1);
+        const T f = a.fact[c];
+        for (int e = a.pt.urec_ptr[u]; e < a.pt.urec_ptr[u + 1]; e++) pnv += rs[(int64_t)nts * a.pt.urec_list[e]] * f;
+      }
+      a.pnew[so + c] = pnv;
+      if (dslot >= 0) {
+        const bool interior = i >= 1 && i <= nx - 2 && j >= 1 && j <= ny - 2 && k >= 1 && k <= nz - 2;
+        T *D = a.dbuf + (int64_t)dslot * a.dslot + so + c;
+        *D = interior ? *D + inj : (a.pold[so + c] - T(2) * a.pcur[so + c]) + pnv;
+      }
+    }
+    if (v >= 0) {
+      T *tr = a.traces + a.pt.off_tr[s] + (a.it - 1);
+      for (int e = a.pt.urec_ptr[v]; e < a.pt.urec_ptr[v + 1]; e++) tr[(int64_t)nts * a.pt.urec_list[e]] = pnv;
+    }
+  }
+}
+
+template <typename T, bool CORR>
+__global__ __launch_bounds__(TX *RM_W) void cd3d_row_kernel(Cd3dArgs<T> a) {
+  __shared__ Cd3dRowLds<T> lds;
+  const int b = xcd_tile3(blockIdx.x, gridDim.x);
+  int t = b;
+  const int bx = t % a.nbx; t /= a.nbx;
+  const int by = t % a.nby; t /= a.nby;
+  const int bk = t % a.nbk;
+  const int s = t / a.nbk;
+  const int nts = a.nt_shot[s];
+  if (a.it > nts || nts <= a.act_min) return;
+  const int nx = a.n[0], ny = a.n[1], nz = a.n[2], h = a.h;
+  const int lane = threadIdx.x & (TX - 1);
+  const int X0 = bx * (TX - 2), j0 = by * RM_W, w = __builtin_amdgcn_readfirstlane(threadIdx.x / TX);
+  const int j = min(j0 + w, ny - 1);
+  const bool own = j0 + w < ny && X0 + lane < nx && lane >= (bx ? 1 : 0) && lane < (bx < a.nbx - 1 ? TX - 1 : TX);
+  const int K0 = bk * a.kch, K1 = min(K0 + a.kch, nz);
+  // planes of the chunk (at most 64) with points on the row
+  uint64_t points;
+  {
+    const int64_t ro = (int64_t)s * (a.pt.nrows + 1) + j + (int64_t)ny * min(K0 + lane, nz - 1);
+    const int *rowp = (a.res == nullptr ? a.pt.srow : a.pt.rrow) + ro, *rowr = a.pt.rrow + ro;
+    points = __ballot(K0 + lane < K1 && (rowp[0] != rowp[1] || (a.traces && rowr[0] != rowr[1])));
+  }
+  const int dslot = cd3d_dslot(a, nts);
+  const bool corr = CORR && a.it + 1 <= nts && a.it + 1 <= a.corr_lim;
+  const bool xs = X0 < max(h, 1) || X0 + TX - 1 >= nx - h - 1;
+  const bool ys = j0 < max(h, 1) || j0 + RM_W - 1 >= ny - h - 1;
+  auto run = [&](auto xsc, auto ysc) {
+    if (CORR && !corr) cd3d_row_march<T, xsc(), ysc(), false>(a, s, lds, X0, j, w, K0, K1, own, dslot);
+    else cd3d_row_march<T, xsc(), ysc(), CORR>(a, s, lds, X0, j, w, K0, K1, own, dslot);
+  };
+  if (xs && ys) run(std::true_type{}, std::true_type{});
+  else if (xs) run(std::true_type{}, std::false_type{});
+  else if (ys) run(std::false_type{}, std::true_type{});
+  else run(std::false_type{}, std::false_type{});
+  if (points) cd3d_row_finish(a, s, nts, X0, j, K0, points, own, dslot);
+}
+
 // grad += adjcur * D for the first step of a segment
 template <typename T>
 __global__ void cd3d_correlate_kernel(T *grad, const T *adj, const T *d, int64_t N, const int *nt_shot, int cbase) {
@@ -635,7 +1006,7 @@ class Cd3dEngine final : public Engine {
       nck_ = std::max(K_ - 2, 0);
       ck_.alloc(std::max<int64_t>(nck_ * ck_one_, 1));
     }
-    // 64 x 4 tiles in one launch, 24 planes per chunk: measured best of
+    // tile kernels: 64 x 4 tiles in one launch, 24 planes per chunk: measured best of
     // 64 x {8, 4, 2} tiles, one or two launches and 8 to 64 planes on
     // 600 x 600 x 400 (the smaller blocks let more of them share a CU than
     // the general path's register count would with 64 x 8)
@@ -647,11 +1018,12 @@ class Cd3dEngine final : public Engine {
     if (const char *v = std::getenv("SWX_CD3D_LEAN")) lean_ = std::atoi(v) != 0;
     // launch shape: 8 / 4 / 2 = one launch with 64 x 8 / 64 x 4 / 64 x 2
     // tiles, 108 / 104 / 102 = interior tiles and the others in two launches,
-    // 208 / 204 / 202 = one launch with the LDS-staged interior march
+    // 208 / 204 / 202 = one launch with the LDS-staged interior march,
+    // 301 = row march
     if (const char *v = std::getenv("SWX_CD3D_VARIANT")) {
       const int c = std::atoi(v);
-      SWX_REQUIRE((c % 100 == 8 || c % 100 == 4 || c % 100 == 2) && c > 0 && c < 300, SWX_EINVAL,
-                  "SWX_CD3D_VARIANT must be 8, 4, 2, 108, 104, 102, 208, 204 or 202");
+      SWX_REQUIRE(((c % 100 == 8 || c % 100 == 4 || c % 100 == 2) && c > 0 && c < 300) || c == 301, SWX_EINVAL,
+                  "SWX_CD3D_VARIANT must be 8, 4, 2, 108, 104, 102, 208, 204, 202 or 301");
       variant_ = c;
       variant_env_ = true;
     }
@@ -678,7 +1050,7 @@ class Cd3dEngine final : public Engine {
     SWX_REQUIRE(model_set_, SWX_ESTATE, "swx_set_model must be called before running");
     zero_forward_state();
     T *tr = c_.pts.d_traces.as<T>();
-    if (!tuned_) tune_shape(save, tr);
+    choose_shape(save, tr);
     for (int it = 1; it <= ntmax_; it++) {
       progress("forward step", it, ntmax_);
       step_fwd(it, 0, save ? 1 : 0, 0, tr);
@@ -800,8 +1172,27 @@ class Cd3dEngine final : public Engine {
     }
   }
 
+  // blocks of one chunk of the row march, planes per chunk (64: the march's
+  // plane masks)
+  int64_t row_columns() const {
+    return std::max<int64_t>(ceil_div(n_[0] - 2, TX - 2), 1) * ceil_div(n_[1], RM_W) * nsh_;
+  }
+  void launch_rows(Cd3dArgs<T> a) {
+    a.nbx = (int)std::max<int64_t>(ceil_div(n_[0] - 2, TX - 2), 1);
+    a.nby = (int)ceil_div(n_[1], RM_W);
+    a.kch = std::min(a.kch, 64);
+    a.nbk = (int)ceil_div(n_[2], a.kch);
+    const unsigned nb = (unsigned)(row_columns() * a.nbk);
+    if (a.corr) cd3d_row_kernel<T, true><<<nb, TX * RM_W, 0, c_.stream>>>(a);
+    else cd3d_row_kernel<T, false><<<nb, TX * RM_W, 0, c_.stream>>>(a);
+  }
+
   void launch_variant(const Cd3dArgs<T> &a, int variant) {
     const int ty = variant % 100, kind = variant / 100;
+    if (kind == 3) {
+      launch_rows(a);
+      return;
+    }
     if (ty == 4) launch_shape<4>(a, kind);
     else if (ty == 2) launch_shape<2>(a, kind);
     else launch_shape<8>(a, kind);
@@ -814,10 +1205,38 @@ class Cd3dEngine final : public Engine {
     SWX_HIP(hipGetLastError());
   }
 
-  // Launch shape (tile height 8 / 4 / 2; one launch, two launches or the
-  // LDS-staged march) and then the planes per chunk, timed on step 1 of the zero initial state, which every
-  // repetition recomputes identically.  Every choice gives bitwise the same
-  // results; SWX_CD3D_VARIANT / SWX_CD3D_ZCHUNK pin them instead.
+  // The row march, unless its 32-bit byte offsets do not reach over a shot's
+  // field (from 4 GiB on).  It is the faster one at every size: us per step,
+  // row march / best tile shape, forward with history and adjoint, 600 x 600 x 400 float32
+  // 812 / 1009 and 1315 / 1307, 400 x 400 x 300 float64 575 / 755 and 950 / 930,
+  // 300 x 280 x 200 float32 123 / 199 and 184 / 217, 129 x 117 x 91 float64
+  // 28 / 47 and 39 / 49.
+  // Planes per chunk: as few as still let every block of the grid be resident
+  // at once, from 6 on; grids that need more than 12 take several
+  // rounds anyway, and 12 is the best for them (8: more planes loaded twice,
+  // 24: fewer blocks to fill the last round; 300 x 280 x 200 float32 127, 123
+  // and 128 us with 8, 12 and 24).
+  void choose_shape(bool save, T *tr) {
+    const int64_t widest = std::max({N_, sps_[0], sps_[1], sps_[2], sxi_[0], sxi_[1], sxi_[2]});
+    const bool reach = widest * (int64_t)sizeof(T) < (int64_t(1) << 32);
+    if (!variant_env_ && reach) variant_ = 301;
+    if (variant_ != 301) {
+      if (!tuned_) tune_shape(save, tr);
+    } else if (!kch_env_) {
+      int per_cu = 0, cus = 0, dev = 0;
+      SWX_HIP(hipGetDevice(&dev));
+      SWX_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+      SWX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, cd3d_row_kernel<T, false>, TX * RM_W, 0));
+      const int64_t chunks = std::max<int64_t>((int64_t)per_cu * cus / row_columns(), 1);
+      kch_ = (int)std::clamp<int64_t>(ceil_div(n_[2], chunks), 6, 12);
+    }
+  }
+
+  // Launch shape of the tile kernels (tile height 8 / 4 / 2; one launch, two
+  // launches or the LDS-staged march) and then the planes per chunk, timed on
+  // step 1 of the zero initial state, which every repetition recomputes
+  // identically.  Every choice gives bitwise the same results;
+  // SWX_CD3D_VARIANT / SWX_CD3D_ZCHUNK pin them instead.
   void tune_shape(bool save, T *tr) {
     auto run = [&](int variant, int kch) {
       variant_ = variant;

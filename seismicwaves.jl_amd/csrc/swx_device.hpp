@@ -17,6 +17,48 @@ __device__ __forceinline__ void st_nt(T *p, T v) {
   __builtin_nontemporal_store(v, p);
 }
 
+// Value of the lane before / after; the wave's end lane, which has none, gets
+// its value of `end`.
+template <int CTRL>
+__device__ __forceinline__ float lane_shift(float x, float end) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(end), __float_as_int(x), CTRL, 0xf, 0xf, false));
+}
+template <int CTRL>
+__device__ __forceinline__ double lane_shift(double x, double end) {
+  const int lo = __builtin_amdgcn_update_dpp(__double2loint(end), __double2loint(x), CTRL, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(__double2hiint(end), __double2hiint(x), CTRL, 0xf, 0xf, false);
+  return __hiloint2double(hi, lo);
+}
+template <typename T>
+__device__ __forceinline__ T lane_before(T x, T end) { return lane_shift<0x138>(x, end); }   // wave_shr:1
+template <typename T>
+__device__ __forceinline__ T lane_after(T x, T end) { return lane_shift<0x130>(x, end); }    // wave_shl:1
+
+// The same, 0 in the end lane.
+template <int CTRL>
+__device__ __forceinline__ float lane_shift(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true));
+}
+template <int CTRL>
+__device__ __forceinline__ double lane_shift(double x) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+template <typename T>
+__device__ __forceinline__ T lane_before(T x) { return lane_shift<0x138>(x); }
+template <typename T>
+__device__ __forceinline__ T lane_after(T x) { return lane_shift<0x130>(x); }
+
+// Makes x opaque: the compiler otherwise keeps what follows from it for every
+// row (tests, addresses) in scalar registers over the levels, spills them and
+// pays a lane read for each use, more than computing it again.
+// (x is the same in all lanes of the wave.)
+__device__ __forceinline__ void opaque(int &x) {
+  x = __builtin_amdgcn_readfirstlane(x);
+  asm volatile("" : "+s"(x));
+}
+
 // Index of the unique point group at linear cell `cell` (grid row `row`) of
 // shot s, or -1.  rowptr/cells are a PointTables row index (sorted cells).
 __device__ __forceinline__ int find_point(const int *rowptr, const int64_t *cells, int64_t nrows, int s,
