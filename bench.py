@@ -444,6 +444,8 @@ def kernel_names(physics, variant):
                 return f"el_march_kernel<float, {v - 100}, {'true' if adj else 'false'}>"
             if v == 2:   # stresses in LDS, one launch per step
                 return f"el_tile_kernel<float, {'true' if adj else 'false'}>"
+            if v == 3:   # a window of 64 columns per wave
+                return f"el_row_kernel<float, {'true' if adj else 'false'}>"
             tail = " (adjoint)" if adj else " (forward)"
             if v == 1:   # interior and other blocks in one launch per kernel
                 return "el_stress_kernel<float, true> + el_disp_kernel<float, true>" + tail

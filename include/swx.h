@@ -158,7 +158,8 @@ typedef struct {
    * VD [forward, adjoint] tile codes (8/16/32 interior + other launches,
    * 308/316/332 one launch, 102/104 z-marching strips; + 1000 k: shots in
    * groups of 2^k in the block order); elastic [forward, adjoint] variant
-   * codes (0/1 stress and displacement launches, 2 one fused launch); CD 2D
+   * codes (0/1 stress and displacement launches, 2 one fused launch, 3 row
+   * march); CD 2D
    * [window shapes (or, with one level per launch, rows per thread), most
    * levels per launch], each 10 x adjoint + forward; CD 3D
    * [301 row march, 8/4/2/108/104/102/208/204/202 tiles; planes per z

@@ -643,27 +643,6 @@ __device__ __forceinline__ int cd3d_row_points(const int *rowp, const int64_t *c
   return u - 1;
 }
 
-// Element of an array at a 32-bit byte offset: base in scalar registers, one
-// vector add per offset (a 64-bit index per row and array costs a dozen scalar
-// instructions, and the four SIMDs of a CU share one scalar unit).
-template <typename T>
-__device__ __forceinline__ T ld_off(const T *base, unsigned off) {
-  return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + off);
-}
-template <typename T>
-__device__ __forceinline__ void st_off(T *base, unsigned off, T v) {
-  *reinterpret_cast<T *>(reinterpret_cast<char *>(base) + off) = v;
-}
-
-// A uniform value of plane m of the chunk, held by lane m.
-__device__ __forceinline__ float lane_value(float x, int m) {
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), m));
-}
-__device__ __forceinline__ double lane_value(double x, int m) {
-  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), m),
-                          __builtin_amdgcn_readlane(__double2loint(x), m));
-}
-
 // XS, YS: the window, some row of the block is in a strip or at an edge.
 template <typename T, bool XS, bool YS, bool CORR>
 __device__ __forceinline__ void cd3d_row_march(const Cd3dArgs<T> &a, int s, Cd3dRowLds<T> &lds, int X0, int j, int w,

@@ -50,6 +50,27 @@ __device__ __forceinline__ T lane_before(T x) { return lane_shift<0x138>(x); }
 template <typename T>
 __device__ __forceinline__ T lane_after(T x) { return lane_shift<0x130>(x); }
 
+// Element of an array at a 32-bit byte offset: base in scalar registers, one
+// vector add per offset (a 64-bit index per row and array costs a dozen scalar
+// instructions, and the four SIMDs of a CU share one scalar unit).
+template <typename T>
+__device__ __forceinline__ T ld_off(const T *base, unsigned off) {
+  return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + off);
+}
+template <typename T>
+__device__ __forceinline__ void st_off(T *base, unsigned off, T v) {
+  *reinterpret_cast<T *>(reinterpret_cast<char *>(base) + off) = v;
+}
+
+// A uniform value held by lane m.
+__device__ __forceinline__ float lane_value(float x, int m) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), m));
+}
+__device__ __forceinline__ double lane_value(double x, int m) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), m),
+                          __builtin_amdgcn_readlane(__double2loint(x), m));
+}
+
 // Makes x opaque: the compiler otherwise keeps what follows from it for every
 // row (tests, addresses) in scalar registers over the levels, spills them and
 // pays a lane read for each use, more than computing it again.

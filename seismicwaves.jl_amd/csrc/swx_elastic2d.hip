@@ -1,8 +1,9 @@
 // 2D isotropic elastic engine (displacement-stress, 4th-order staggered
 // space, 2nd-order time, C-PML, optional free surface on the top row) for a
-// batch of shots: two launches per time step (stresses from ucur, then
-// displacements), a receiver gather when traces are recorded, and the
-// gradient correlation fused into the adjoint stress launch.
+// batch of shots: one launch per time step (el_row_kernel: stresses from ucur,
+// displacements, the gradient correlation of the adjoint, and the receivers of
+// the level before), or two (stresses, then displacements) where the stresses
+// must be in memory.
 //
 // Reference semantics (paths relative to the reference root):
 //   step       src/models/elastic/backends/shared/elastic2D_iso_xPU.jl:1-448
@@ -54,7 +55,7 @@ struct TapView {
 template <typename T>
 struct ElArgs {
   int nx, nz, h, freetop;
-  int nbx, nbz, ch;             // z-marching launch: strips, chunks, rows per chunk
+  int nbx, nbz, ch, nshots;     // z-marching launch: strips, chunks, rows per chunk
   int tbx, tbz, xcd;            // block launches: tiles along x, z; XCD-aware tile map
   int order;                    // 1: the tiles outside [ibx0, ibx1] x [iby0, iby1] first
   int ibx0, ibx1, iby0, iby1;   // tiles clear of the C-PML strips and grid edges
@@ -78,6 +79,9 @@ struct ElArgs {
   T *hist; int64_t hslot; int hmode; int S; int cbase;
   // correlation (stress launch on the adjoint field)
   T *grad; int64_t gstride; int update; int corr_step; int corr_lim;
+  // receivers of level it-1, recorded by the first nrecb blocks per shot of a row march
+  TapView<T> r0, r1;
+  T *traces; const int64_t *off_tr; int maxrec, nrecb;
 };
 
 // Block -> (strip, chunk, shot) map giving each of the 8 XCDs a contiguous
@@ -1576,14 +1580,13 @@ __global__ __launch_bounds__(TX *TZ) void el_tile_kernel(ElArgs<T> a) {
 }
 
 // traces[it, comp, r] = sum over taps of coef * u (record_receivers2D_* and
-// the per-receiver reduction, elastic2D_iso_xPU.jl:108-118, :216-231).
+// the per-receiver reduction, elastic2D_iso_xPU.jl:108-118, :216-231), q = 2 r + comp.
 template <typename T>
-__global__ void el_record_kernel(const T *u, int64_t N, TapView<T> r0, TapView<T> r1, const int *nt_shot,
-                                 const int64_t *off_tr, T *traces, int it, int maxrec) {
-  const int s = blockIdx.y;
+__device__ __forceinline__ void el_record(const T *u, int64_t N, const TapView<T> &r0, const TapView<T> &r1,
+                                          const int *nt_shot, const int64_t *off_tr, T *traces, int it, int maxrec,
+                                          int s, int q) {
   const int nts = nt_shot[s];
   if (it > nts) return;
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
   const int comp = q & 1, r = q >> 1;
   const int p0 = r0.poff[s], np = r0.poff[s + 1] - p0;
   if (r >= np || r >= maxrec) return;
@@ -1592,6 +1595,499 @@ __global__ void el_record_kernel(const T *u, int64_t N, TapView<T> r0, TapView<T
   T acc = 0;
   for (int k = t.pptr[p0 + r]; k < t.pptr[p0 + r + 1]; k++) acc += t.pcoef[k] * f[t.pcell[k]];
   traces[off_tr[s] + (it - 1) + (int64_t)nts * (comp + 2 * r)] = acc;
+}
+template <typename T>
+__global__ void el_record_kernel(const T *u, int64_t N, TapView<T> r0, TapView<T> r1, const int *nt_shot,
+                                 const int64_t *off_tr, T *traces, int it, int maxrec) {
+  el_record(u, N, r0, r1, nt_shot, off_tr, traces, it, maxrec, blockIdx.y, blockIdx.x * blockDim.x + threadIdx.x);
+}
+
+// ---------------------------------------------------------------------------
+// Row march (el_row_kernel)
+//
+// A wave owns up to 58 columns of a window of 64 and marches down z over a
+// chunk of rows: the stresses of row j from ucur rows j-2 .. j+2, then the
+// displacements of row j-2 from stress rows j-4 .. j.  Everything stays in
+// the wave's registers: z neighbours in rows kept from the iterations before,
+// x neighbours in the adjacent lanes (zero beyond the first and last column,
+// as the derivative rules have it).  The row is the same for all lanes, so the
+// free surface, the grid's first and last rows and the z C-PML strips are
+// decided once per row, and every field of row j+2 is in flight while row j is
+// stepped.  Points that act on displacements are applied by el_inject_kernel,
+// moment tensors from a list in LDS.  Statements are those of
+// el_stress_kernel and el_disp_kernel: results are bitwise the same.
+//
+// Against the tile step (el_tile_kernel: 64 x 16 tiles with two barriers, both
+// u and the stresses staged in LDS, the stresses of a 68 x 20 region computed
+// for a tile) it loads a row of u once per wave and recomputes 6 of 64 columns
+// and 4 rows per chunk.  us per step, tile / row march: 813 x 407, 4 shots,
+// float32, forward 45 / 27; 1500 x 600, 12 shots, float32, forward 130 / 101
+// and adjoint 346 / 306 (88 bytes per cell of fields, history and gradients:
+// 3.1 TB/s); 331 x 257, 3 shots, float64, forward 34 / 20, adjoint 29 / 29.
+// What bounds it: the waves in the strips, which issue three (two axes) times
+// the instructions of an interior one per row, and in double precision the
+// adjoint's registers (one wave per SIMD).
+constexpr int ER_OWN = 58, ER_W = 4;      // columns per window, waves per block
+constexpr int ER_ROWS = 56;               // most rows per chunk (64 lanes hold the coefficients of the rows loaded)
+constexpr int ER_TAPS = 128;              // most moment-tensor taps per wave
+
+template <typename T>
+struct ElRow {
+  T ux, uz, l, m, mh, ox, oz, rx, rz;
+  T hx, hz, h0x, h0z, h2x, h2z, g[5];     // correlation: level corr_step-1 (hx, hz), its neighbours in time, gradients
+  T p[8];                                 // C-PML memory variables
+};
+
+// Moment-tensor taps on the stress cells of a wave: f0 then f1, by cell
+template <typename T>
+struct ElTaps {
+  int key[ER_TAPS];                       // 64 * row of the chunk + lane
+  T c0[ER_TAPS], c1[ER_TAPS], f[ER_TAPS];
+};
+
+// Taps of family t on rows jr .. jr+63 (row jr + lane held by a lane: rows
+// [b, e) of the cell table) and columns X0 .. X0+63, appended to L from n on.
+template <typename T, bool SHEAR>
+__device__ __forceinline__ int el_row_taps(const ElArgs<T> &a, const TapView<T> &t, int s, int nts, int jr, int X0,
+                                           int u0, int u1, ElTaps<T> &L, int n) {
+  const int lane = threadIdx.x & (TX - 1);
+  const T *tf = a.tf + a.off_tf[s] + (a.it - 1);
+  const T *M = a.mom + 3 * (int64_t)a.off_mom[s];
+  const int e0 = t.eptr[u0], e1 = t.eptr[u1];
+  for (int eb = e0; eb < e1; eb += TX) {
+    const int e = eb + lane;
+    bool in = e < e1;
+    int key = 0;
+    if (in) {
+      int lo = u0, hi = u1 - 1;           // unique cell of entry e
+      while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (t.eptr[mid] <= e) lo = mid;
+        else hi = mid - 1;
+      }
+      const int64_t c = t.cell[lo];
+      const int j = (int)(c / a.nx) + 1, col = (int)(c % a.nx) + 1 - X0;
+      in = col >= 0 && col < TX;
+      key = (j - jr) * TX + col;
+    }
+    const uint64_t w = __ballot(in);
+    const int q = n + __builtin_popcountll(w & ((uint64_t(1) << lane) - 1));
+    if (in && q < ER_TAPS) {
+      const int p = t.epoint[e];
+      const T x = t.ecoef[e];
+      L.key[q] = key;
+      L.c0[q] = M[3 * p + (SHEAR ? 2 : 0)] * x;
+      L.c1[q] = SHEAR ? T(0) : M[3 * p + 1] * x;
+      L.f[q] = tf[(int64_t)nts * p];
+    }
+    n = min(n + __builtin_popcountll(w), ER_TAPS);
+  }
+  return n;
+}
+
+// XS: the window reaches a strip or a side; ZS: the chunk's rows do.
+template <typename T, bool XS, bool ZS, bool ADJ>
+__device__ __forceinline__ void el_row_march(const ElArgs<T> &a, int s, int nts, int X0, int Z0, int Z1, bool own,
+                                             const ElTaps<T> *L, int n0, int n1) {
+  constexpr unsigned E = sizeof(T);
+  const int nx = a.nx, nz = a.nz, h = a.h;
+  const int lane = threadIdx.x & (TX - 1), i = X0 + lane;
+  const bool ft = a.freetop != 0;
+  const int64_t N = a.N;
+  const unsigned row = (unsigned)nx * E, vi = (unsigned)(min(i, nx) - 1) * E;
+  const T *ucx = a.ucur + (int64_t)s * 2 * N, *ucz = ucx + N;
+  T *unx = a.unew + (int64_t)s * 2 * N, *unz = unx + N;
+  const T *pso = a.psi_o + (int64_t)s * a.psi_stride;
+  T *psn = a.psi_n + (int64_t)s * a.psi_stride;
+  const T *cb = a.cpml + (int64_t)s * a.cstride;
+  const AxisCoef<T> cx = axis_coef(cb, h, 0), cz = axis_coef(cb, h, 1);
+  const bool colx = i <= nx - 1, colz = i <= nx;             // columns of the ux, uz grids
+  const bool nrmx = i >= 2 && i <= nx - 1;
+  // x strips: entries and coefficients of the column
+  const int kf = XS && colz ? strip_full(i, nx, h) : 0, kh = XS && colz ? strip_half(i - 1, nx - 1, h) : 0;
+  const unsigned of = (unsigned)max(kf - 1, 0), oh = (unsigned)max(kh - 1, 0);
+  T xb = 0, xa = 0, xbh = 0, xah = 0;
+  if (XS && kh) {
+    xb = cx.b(kh - 1);
+    xa = cx.a(kh - 1);
+  }
+  if (XS && kf) {
+    xbh = cx.bh(kf - 1);
+    xah = cx.ah(kf - 1);
+  }
+  // z strips: lane m holds the entries and coefficients of row jr + m
+  const int jr = Z0 - 2;
+  T zb = 0, za = 0, zbh = 0, zah = 0;
+  uint64_t zf = 0, zh = 0;                                   // rows in a full, half strip
+  if (ZS) {
+    const int j = jr + lane;
+    const bool in = j >= 1 && j <= nz;
+    const int k1 = in ? strip_half(j - 1, nz - 1, h) : 0, k2 = in ? strip_full(j, nz, h) : 0;
+    if (k1) {
+      zb = cz.b(k1 - 1);
+      za = cz.a(k1 - 1);
+    }
+    if (k2) {
+      zbh = cz.bh(k2 - 1);
+      zah = cz.ah(k2 - 1);
+    }
+    zh = __ballot(k1 != 0);
+    zf = __ballot(k2 != 0);
+  }
+  auto clampz = [&](int j) { return (unsigned)(min(max(j, 1), nz) - 1); };
+  auto zfull = [&](int j) { return (unsigned)(strip_full(j, nz, h) - 1); };
+  auto zhalf = [&](int j) { return (unsigned)(strip_half(j - 1, nz - 1, h) - 1); };
+  const T *p0_ = pso + a.psioff[0], *p1_ = pso + a.psioff[1], *p2_ = pso + a.psioff[2], *p3_ = pso + a.psioff[3],
+          *p4_ = pso + a.psioff[4], *p5_ = pso + a.psioff[5], *p6_ = pso + a.psioff[6], *p7_ = pso + a.psioff[7];
+  const int64_t dp = psn - pso;                              // the written parity
+  const unsigned wf = (unsigned)(2 * h) * E, wh = (unsigned)(2 * h + 2) * E, row1 = (unsigned)(nx - 1) * E;
+  const unsigned vi1 = (unsigned)(min(i, nx - 1) - 1) * E;   // column of the (nx-1)-wide variables
+  // correlation
+  const T *h1x_ = nullptr, *h1z_ = nullptr, *h0x_ = nullptr, *h0z_ = nullptr, *h2x_ = nullptr, *h2z_ = nullptr;
+  T *g_[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
+  if (ADJ) {
+    h0x_ = a.hist + (int64_t)(a.corr_step - a.cbase - 1) * a.hslot + (int64_t)s * 2 * N;
+    h1x_ = h0x_ + a.hslot;
+    h2x_ = h1x_ + a.hslot;
+    h0z_ = h0x_ + N;
+    h1z_ = h1x_ + N;
+    h2z_ = h2x_ + N;
+    for (int q = 0; q < 5; q++) g_[q] = a.grad + (int64_t)s * a.gstride + q * N;
+  }
+  // history of the level
+  const int sb = a.hmode == 1 ? (nts / a.S) * a.S : a.cbase;
+  const bool keep = !ADJ && a.hmode && a.it > sb, first = keep && a.hmode == 1 && a.it == sb + 1;
+  T *hs_ = keep ? a.hist + (int64_t)s * 2 * N : nullptr;
+  T *hn_ = keep ? hs_ + (int64_t)(a.it - sb + 1) * a.hslot : nullptr;
+
+  auto load = [&](int j) {
+    ElRow<T> q;
+    const unsigned r0 = clampz(j) * row + vi, rd = clampz(j - 2) * row + vi;
+    const unsigned r1 = clampz(j + 1) * row + vi, r2 = clampz(j + 2) * row + vi;
+    q.ux = ld_off(ucx, r2);
+    q.uz = ld_off(ucz, r1);
+    q.l = ld_off(a.lam, r0);
+    q.m = ld_off(a.mu, r0);
+    q.mh = ld_off(a.muhh, r0);
+    q.ox = ld_off(unx, rd);
+    q.oz = ld_off(unz, rd);
+    q.rx = ld_off(a.rdx, rd);
+    q.rz = ld_off(a.rdz, rd);
+    if (ADJ) {
+      q.hx = ld_off(h1x_, r2);
+      q.hz = ld_off(h1z_, r1);
+      q.h0x = ld_off(h0x_, r0);
+      q.h0z = ld_off(h0z_, r0);
+      q.h2x = ld_off(h2x_, r0);
+      q.h2z = ld_off(h2z_, r0);
+#pragma unroll
+      for (int f = 0; f < 5; f++) q.g[f] = ld_off(g_[f], r0);
+    }
+    if (XS) {
+      const unsigned js = clampz(j), jd = min(clampz(j - 2), (unsigned)(nz - 2));
+      q.p[4] = ld_off(p4_, js * wh + oh * E);
+      q.p[1] = ld_off(p1_, jd * wh + oh * E);
+      if (h > 0) {
+        q.p[5] = ld_off(p5_, min(js, (unsigned)(nz - 2)) * wf + of * E);
+        q.p[0] = ld_off(p0_, clampz(j - 2) * wf + of * E);
+      }
+    }
+    if (ZS) {
+      const int m = j - jr;
+      if (zh >> m & 1) q.p[7] = ld_off(p7_, zhalf(j) * row + vi);
+      if (zf >> m & 1) q.p[6] = ld_off(p6_, zfull(j) * row1 + vi1);
+      if (m >= 2 && (zh >> (m - 2) & 1)) q.p[3] = ld_off(p3_, zhalf(j - 2) * row1 + vi1);
+      if (m >= 2 && (zf >> (m - 2) & 1)) q.p[2] = ld_off(p2_, zfull(j - 2) * row + vi);
+    }
+    return q;
+  };
+  auto inx = [&](T v, int j) {        // a value of the ux grid, zero outside
+    if (XS) v = colx ? v : T(0);
+    if (ZS) v = j >= 1 && j <= nz ? v : T(0);
+    return v;
+  };
+  auto inz = [&](T v, int j) {        // of the uz grid
+    if (XS) v = colz ? v : T(0);
+    if (ZS) v = j >= 1 && j <= nz - 1 ? v : T(0);
+    return v;
+  };
+  // rows of ux (j-2 .. j+2) and uz (j-2 .. j+1), of the correlated level, and of the stresses
+  T xm2 = 0, xm1, x0, x1, x2, zm2, zm1, z0, z1;
+  T am1 = 0, a0 = 0, a1 = 0, a2 = 0, bm2 = 0, bm1 = 0, b0 = 0, b1 = 0;
+  T sxx2 = 0, sxx1 = 0, sxx0 = 0, szz3 = 0, szz2 = 0, szz1 = 0, szz0 = 0;
+  T sxz4 = 0, sxz3 = 0, sxz2 = 0, sxz1 = 0, sxz0 = 0;
+  {
+    auto at = [&](const T *f, int j) { return ld_off(f, clampz(j) * row + vi); };
+    xm1 = inx(at(ucx, jr - 2), jr - 2);
+    x0 = inx(at(ucx, jr - 1), jr - 1);
+    x1 = inx(at(ucx, jr), jr);
+    x2 = inx(at(ucx, jr + 1), jr + 1);
+    zm1 = inz(at(ucz, jr - 2), jr - 2);
+    z0 = inz(at(ucz, jr - 1), jr - 1);
+    z1 = inz(at(ucz, jr), jr);
+    if (ADJ) {
+      a0 = inx(at(h1x_, jr - 1), jr - 1);
+      a1 = inx(at(h1x_, jr), jr);
+      a2 = inx(at(h1x_, jr + 1), jr + 1);
+      bm1 = inz(at(h1z_, jr - 2), jr - 2);
+      b0 = inz(at(h1z_, jr - 1), jr - 1);
+      b1 = inz(at(h1z_, jr), jr);
+    }
+  }
+  int t0 = 0, t1 = n0;                // next taps of the normal, shear stresses
+  auto step = [&](int j, const ElRow<T> &q) {
+    const int m = j - jr;
+    xm2 = xm1; xm1 = x0; x0 = x1; x1 = x2; x2 = inx(q.ux, j + 2);
+    zm2 = zm1; zm1 = z0; z0 = z1; z1 = inz(q.uz, j + 1);
+    const bool rown = j >= Z0 && j < Z1;
+    const bool jn = !ZS || (j >= (ft ? 1 : 2) && j <= nz - 1), js = !ZS || (j >= 1 && j <= nz - 1);
+    const bool nrm = jn && (!XS || nrmx), shr = js && (!XS || colx);
+    const T l = q.l, mu = q.m;
+    // ---- stresses of row j ----
+    T dux, duz, duzx, duxz;
+    {
+      const T f1 = lane_before(x0), f2 = lane_before(f1);
+      dux = d4<T>(f2, f1, x0, lane_after(x0), a.idx);
+      const T e1 = lane_after(z0), e2 = lane_after(e1);
+      duzx = d4<T>(lane_before(z0), z0, e1, e2, a.idx);
+    }
+    if (ZS && ft && j <= 2) {
+      duz = j == 1 ? (-l / (l + T(2) * mu)) * dux : d4<T>(zm1, zm1, z0, z1, a.idz);
+      duxz = j == 1 ? d4<T>(x1, x0, x1, x2, a.idz) : d4<T>(xm1, x0, x1, x2, a.idz);
+    } else {
+      duz = d4<T>(zm2, zm1, z0, z1, a.idz);
+      duxz = d4<T>(xm1, x0, x1, x2, a.idz);
+    }
+    T dxc = dux, dzc = duz, c1 = duzx, c2 = duxz;
+    if (XS) {
+      const T pn = xb * q.p[4] + xa * dux;
+      if (kh) dxc = dux + pn;
+      if (own && rown && kh && nrm) st_off(const_cast<T *>(p4_) + dp, (unsigned)(j - 1) * wh + oh * E, pn);
+      if (h > 0) {
+        const T pm = xbh * q.p[5] + xah * duzx;
+        if (kf) c1 = duzx + pm;
+        if (own && rown && kf && shr) st_off(const_cast<T *>(p5_) + dp, (unsigned)(j - 1) * wf + of * E, pm);
+      }
+    }
+    if (ZS && (zh >> m & 1)) {
+      const T pn = lane_value(zb, m) * q.p[7] + lane_value(za, m) * duz;
+      dzc = duz + pn;
+      if (own && rown && nrm) st_off(const_cast<T *>(p7_) + dp, zhalf(j) * row + vi, pn);
+    }
+    if (ZS && (zf >> m & 1)) {
+      const T pn = lane_value(zbh, m) * q.p[6] + lane_value(zah, m) * duxz;
+      c2 = duxz + pn;
+      if (own && rown && shr) st_off(const_cast<T *>(p6_) + dp, zfull(j) * row1 + vi, pn);
+    }
+    T vxx = (l + T(2) * mu) * dxc + l * dzc;
+    T vzz = l * dxc + (l + T(2) * mu) * dzc;
+    if (ZS) vzz = j == 1 ? T(0) : vzz;
+    T vxz = q.mh * (c1 + c2);
+    if (!ADJ) {
+      while (t0 < n0 && L->key[t0] < (m + 1) * TX) {
+        if ((L->key[t0] & (TX - 1)) == lane) {
+          vxx += L->c0[t0] * L->f[t0];
+          vzz += L->c1[t0] * L->f[t0];
+        }
+        t0++;
+      }
+      while (t1 < n1 && L->key[t1] < (m + 1) * TX) {
+        if ((L->key[t1] & (TX - 1)) == lane) vxz += L->c0[t1] * L->f[t1];
+        t1++;
+      }
+    }
+    if (XS || ZS) {
+      vxx = nrm ? vxx : T(0);
+      vzz = nrm ? vzz : T(0);
+      vxz = shr ? vxz : T(0);
+    }
+    sxx2 = sxx1; sxx1 = sxx0; sxx0 = vxx;
+    szz3 = szz2; szz2 = szz1; szz1 = szz0; szz0 = vzz;
+    sxz4 = sxz3; sxz3 = sxz2; sxz2 = sxz1; sxz1 = sxz0; sxz0 = vxz;
+    // ---- correlation at the stress cells of row j (correlate_gradient_xPU.jl:1-82) ----
+    if (ADJ) {
+      am1 = a0; a0 = a1; a1 = a2; a2 = inx(q.hx, j + 2);
+      bm2 = bm1; bm1 = b0; b0 = b1; b1 = inz(q.hz, j + 1);
+      const T f1 = lane_before(a0), f2 = lane_before(f1);
+      const T exx = d4<T>(f2, f1, a0, lane_after(a0), a.idx);
+      const T e1 = lane_after(b0), e2 = lane_after(e1);
+      const T ezx = d4<T>(lane_before(b0), b0, e1, e2, a.idx);
+      T ezz, exz_;
+      if (ZS && ft && j <= 2) {
+        ezz = j == 1 ? (-l / (l + T(2) * mu)) * exx : d4<T>(bm1, bm1, b0, b1, a.idz);
+        exz_ = j == 1 ? d4<T>(a1, a0, a1, a2, a.idz) : d4<T>(am1, a0, a1, a2, a.idz);
+      } else {
+        ezz = d4<T>(bm2, bm1, b0, b1, a.idz);
+        exz_ = d4<T>(am1, a0, a1, a2, a.idz);
+      }
+      if (own && rown) {
+        const unsigned r0 = (unsigned)(j - 1) * row + vi;
+        const bool top = ZS && ft && j == 1;
+        const T v = x0 * (q.h0x - T(2) * a0 + q.h2x) * a.idt2;
+        if (!XS || colx) st_off(g_[0], r0, q.g[0] + (top ? v / T(2) : v));
+        if (!ZS || j <= nz - 1) st_off(g_[1], r0, q.g[1] + z0 * (q.h0z - T(2) * b0 + q.h2z) * a.idt2);
+        if (nrm) {
+          const T dv = exx + ezz, dva = dux + duz;
+          if (top) {
+            st_off(g_[2], r0, q.g[2] + dv * dva / T(2));
+            st_off(g_[3], r0, q.g[3] + (exx * dux + ezz * duz));
+          } else {
+            st_off(g_[2], r0, q.g[2] + dv * dva);
+            st_off(g_[3], r0, q.g[3] + T(2) * (exx * dux + ezz * duz));
+          }
+        }
+        if (shr) {
+          const T exz = (ezx + exz_) / T(2);
+          const T exza = (duzx + duxz) / T(2);
+          st_off(g_[4], r0, q.g[4] + T(2) * (exz * exza + exz * exza));
+        }
+      }
+    }
+    // ---- displacements of row jd ----
+    if (m < 4) return;
+    const int jd = j - 2;
+    const unsigned rd = (unsigned)(jd - 1) * row + vi;
+    const bool hx = own && (!XS || colx), hz = own && (!ZS || jd <= nz - 1);
+    T nux, nuz;
+    {
+      const T e1 = lane_after(sxx2), e2 = lane_after(e1);
+      const T d1 = d4<T>(lane_before(sxx2), sxx2, e1, e2, a.idx);
+      T d2;
+      if (ZS && ft && jd <= 2) d2 = jd == 1 ? d4<T>(-sxz1, -sxz2, sxz2, sxz1, a.idz) : d4<T>(-sxz3, sxz3, sxz2, sxz1, a.idz);
+      else d2 = d4<T>(sxz4, sxz3, sxz2, sxz1, a.idz);
+      T c1 = d1, c2 = d2;
+      if (XS && h > 0) {
+        const T pn = xbh * q.p[0] + xah * d1;
+        if (kf) c1 = d1 + pn;
+        if (hx && kf) st_off(const_cast<T *>(p0_) + dp, (unsigned)(jd - 1) * wf + of * E, pn);
+      }
+      if (ZS && (zh >> (m - 2) & 1)) {
+        const T pn = lane_value(zb, m - 2) * q.p[3] + lane_value(za, m - 2) * d2;
+        if (hx) st_off(const_cast<T *>(p3_) + dp, zhalf(jd) * row1 + vi, pn);
+        c2 = d2 + pn;
+      }
+      nux = T(2) * xm2 - q.ox + q.rx * (c1 + c2);
+    }
+    {
+      const T f1 = lane_before(sxz2), f2 = lane_before(f1);
+      const T d1 = d4<T>(f2, f1, sxz2, lane_after(sxz2), a.idx);
+      T d2;
+      if (ZS && ft && jd == 1) d2 = d4<T>(-szz1, szz2, szz1, szz0, a.idz);
+      else d2 = d4<T>(szz3, szz2, szz1, szz0, a.idz);
+      T c1 = d1, c2 = d2;
+      if (XS) {
+        const T pn = xb * q.p[1] + xa * d1;
+        if (kh) c1 = d1 + pn;
+        if (hz && kh) st_off(const_cast<T *>(p1_) + dp, (unsigned)(jd - 1) * wh + oh * E, pn);
+      }
+      if (ZS && (zf >> (m - 2) & 1)) {
+        const T pn = lane_value(zbh, m - 2) * q.p[2] + lane_value(zah, m - 2) * d2;
+        if (hz) st_off(const_cast<T *>(p2_) + dp, zfull(jd) * row + vi, pn);
+        c2 = d2 + pn;
+      }
+      nuz = T(2) * zm2 - q.oz + q.rz * (c1 + c2);
+    }
+    if (hx) st_off(unx, rd, nux);
+    if (hz) st_off(unz, rd, nuz);
+    if (!ADJ && keep) {
+      if (XS) nux = colx ? nux : T(0);
+      if (ZS) nuz = jd <= nz - 1 ? nuz : T(0);
+      if (own) {
+        st_off(hn_, rd, nux);
+        st_off(hn_ + N, rd, nuz);
+        if (first) {
+          st_off(hs_, rd, XS && !colx ? T(0) : q.ox);
+          st_off(hs_ + N, rd, ZS && jd > nz - 1 ? T(0) : q.oz);
+          st_off(hs_ + a.hslot, rd, xm2);
+          st_off(hs_ + a.hslot + N, rd, zm2);
+        }
+      }
+    }
+  };
+  // three row buffers in turn: rows j+1 and j+2 are in flight while row j is
+  // stepped
+  const int je = Z1 + 2;
+  ElRow<T> A = load(jr), B = load(jr + 1);
+  for (int j = jr; j < je; j += 3) {
+    const ElRow<T> C = load(j + 2);
+    step(j, A);
+    if (j + 1 >= je) break;
+    A = load(j + 3);
+    step(j + 1, B);
+    if (j + 2 >= je) break;
+    B = load(j + 4);
+    step(j + 2, C);
+  }
+}
+
+template <typename T, bool ADJ>
+__global__ __launch_bounds__(TX *ER_W) void el_row_kernel(ElArgs<T> a) {
+  __shared__ ElTaps<T> taps[ADJ ? 1 : ER_W];
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / TX), lane = threadIdx.x & (TX - 1);
+  const int nrec = ADJ ? 0 : a.nrecb * a.nshots;
+  if (!ADJ && (int)blockIdx.x < nrec) {      // receivers of the level before
+    const int s = blockIdx.x / a.nrecb, b = blockIdx.x - s * a.nrecb;
+    el_record(a.ucur, a.N, a.r0, a.r1, a.nt_shot, a.off_tr, a.traces, a.it - 1, a.maxrec, s,
+              b * (int)blockDim.x + (int)threadIdx.x);
+    return;
+  }
+  const int t = xcd_tile_el(blockIdx.x - nrec, gridDim.x - nrec) * ER_W + w;
+  const int bx = t % a.nbx, r = t / a.nbx, bz = r % a.nbz, s = r / a.nbz;
+  if (s >= a.nshots) return;
+  const int nts = a.nt_shot[s];
+  if (a.it > nts || (!ADJ && nts <= a.act_min)) return;
+  const int nx = a.nx, nz = a.nz, h = a.h;
+  const int X0 = bx * ER_OWN + 1, Z0 = bz * a.ch + 1, Z1 = min(Z0 + a.ch, nz + 1);
+  const bool own = X0 + lane <= nx && lane >= (bx ? 3 : 0) && lane < (bx < a.nbx - 1 ? TX - 3 : TX);
+  int n0 = 0, n1 = 0;
+  if (!ADJ && a.kind == 1) {
+    const int jr = Z0 - 2, j0 = max(jr, 1) - 1, j1 = min(Z1 + 1, nz);
+    const int64_t o = (int64_t)s * (a.nrows + 1);
+    ElTaps<T> &L = taps[ADJ ? 0 : w];
+    const int u0 = a.f0.rows[o + j0], u1 = a.f0.rows[o + j1], v0 = a.f1.rows[o + j0], v1 = a.f1.rows[o + j1];
+    if (u0 < u1) n0 = el_row_taps<T, false>(a, a.f0, s, nts, jr, X0, u0, u1, L, 0);
+    n1 = n0;
+    if (v0 < v1) n1 = el_row_taps<T, true>(a, a.f1, s, nts, jr, X0, v0, v1, L, n0);
+    n0 = __builtin_amdgcn_readfirstlane(n0);
+    n1 = __builtin_amdgcn_readfirstlane(n1);
+    __builtin_amdgcn_wave_barrier();
+  }
+  const bool corr = ADJ && a.corr_step > 0 && a.corr_step <= nts && a.corr_step <= a.corr_lim;
+  const int lo = max(3, h + 2);
+  const bool xs = X0 < lo || X0 + TX - 1 > min(nx - 2, nx - h - 2);
+  const bool zs = Z0 - 2 < lo || Z1 + 1 > min(nz - 2, nz - h - 2);
+  const ElTaps<T> *L = &taps[ADJ ? 0 : w];
+  auto run = [&](auto xsc, auto zsc) {
+    if (ADJ && corr) el_row_march<T, xsc(), zsc(), true>(a, s, nts, X0, Z0, Z1, own, L, 0, 0);
+    else el_row_march<T, xsc(), zsc(), false>(a, s, nts, X0, Z0, Z1, own, L, n0, n1);
+  };
+  if (xs && zs) run(std::true_type{}, std::true_type{});
+  else if (xs) run(std::true_type{}, std::false_type{});
+  else if (zs) run(std::false_type{}, std::true_type{});
+  else run(std::false_type{}, std::false_type{});
+}
+
+// Injection into the displacements that el_row_kernel has stepped
+// (elastic2D_iso_xPU.jl:96-106), one thread per cell and component, and their
+// copy in the history.
+template <typename T>
+__global__ void el_inject_kernel(ElArgs<T> a) {
+  const int s = blockIdx.y;
+  const int nts = a.nt_shot[s];
+  if (a.it > nts || nts <= a.act_min) return;
+  const int comp = blockIdx.z;
+  const TapView<T> &t = comp ? a.f1 : a.f0;
+  const int *rows = t.rows + (int64_t)s * (a.nrows + 1);
+  const int u = rows[0] + blockIdx.x * blockDim.x + threadIdx.x;
+  if (u >= rows[a.nrows]) return;
+  const int64_t c = t.cell[u], o = (int64_t)s * 2 * a.N + comp * a.N + c;
+  const T *tf = a.tf + a.off_tf[s] + (a.it - 1);
+  const T r = (comp ? a.rdz : a.rdx)[c];
+  T v = a.unew[o];
+  for (int e = t.eptr[u]; e < t.eptr[u + 1]; e++) v += t.ecoef[e] * tf[(int64_t)nts * (a.ncomp * t.epoint[e] + comp)] * r;
+  a.unew[o] = v;
+  const int sb = a.hmode == 1 ? (nts / a.S) * a.S : a.cbase;
+  if (a.hmode && a.it > sb) a.hist[(int64_t)(a.it - sb + 1) * a.hslot + o] = v;
 }
 
 // dt^2 / rho on a padded slab (the spare column or row holds rho = 0 and
@@ -1605,6 +2101,7 @@ __global__ void el_rdt_kernel(T *out, const T *rho, int64_t n, T dt2) {
 // Host-side tap table of one family for a batch of shots.
 struct TapTable {
   DevBuf cell, eptr, epoint, ecoef, rows, poff, pptr, pcell, pcoef;
+  int max_ucell = 0;   // most unique cells of a shot
   template <typename T>
   TapView<T> view() const {
     return TapView<T>{cell.as<int64_t>(), eptr.as<int>(),   epoint.as<int>(), ecoef.as<T>(), rows.as<int>(),
@@ -1639,6 +2136,7 @@ void build_taps(TapTable &t, int nshots, const int *npts, const swx_taps *const 
     }
     poff.push_back(poff.back() + npts[s]);
     const int u0 = (int)cell.size();
+    t.max_ucell = std::max(s ? t.max_ucell : 0, (int)g.size());
     for (auto &kv : g) {
       cell.push_back(kv.first);
       for (auto &pe : kv.second) {
@@ -1845,13 +2343,17 @@ class El2dEngine final : public Engine {
     nsh_ = nshots;
     nt_ = pt.nt;
     ntmax_ = *std::max_element(nt_.begin(), nt_.end());
+    for (int k = 0; k < 2; k++) max_ucell_[k] = std::max(taps_[2 * k].max_ucell, taps_[2 * k + 1].max_ucell);
+    const bool was = rows_ok_;
+    choose_rows(nshots, nsrc.data(), shots);
+    if (rows_ok_ != was) var_fwd_ = var_adj_ = -1;
   }
 
   void forward(bool save) override {
     SWX_REQUIRE(model_set_, SWX_ESTATE, "swx_set_model must be called before running");
     if (var_fwd_ < 0) {
       // tuning launches run on the state before it is cleared below
-      var_fwd_ = tune("SWX_EL2D_VARIANT_FWD", [&](int v) { step_fwd_v(v, 1, 0, 0, 0, nullptr); }, true);
+      var_fwd_ = tune("SWX_EL2D_VARIANT_FWD", [&](int v) { step_fwd_v(v, 1, 0, 0, 0, nullptr); });
     }
     zero_forward_state(true);
     if (save) SWX_HIP(hipMemsetAsync(hist_.get(), 0, hist_.bytes(), c_.stream));
@@ -1891,7 +2393,7 @@ class El2dEngine final : public Engine {
       // are in range, and the adjoint state and gradients are cleared below
       const int cbt = (int)(ceil_div(ntmax_, S_) - 1) * S_;
       const int itt = ntmax_ - 1 > cbt ? ntmax_ - 1 : ntmax_;
-      var_adj_ = tune("SWX_EL2D_VARIANT_ADJ", [&](int v) { step_adj_v(v, itt, cbt); }, false);
+      var_adj_ = tune("SWX_EL2D_VARIANT_ADJ", [&](int v) { step_adj_v(v, itt, cbt); });
     }
     SWX_HIP(hipMemsetAsync(au_.get(), 0, au_.bytes(), c_.stream));
     SWX_HIP(hipMemsetAsync(asig_.get(), 0, asig_.bytes(), c_.stream));
@@ -2062,7 +2564,7 @@ class El2dEngine final : public Engine {
 
   void step_fwd(int it, int act_min, int hmode, int cbase, T *traces) {
     // with snapshots the stresses must be in HBM: no fused variant
-    const bool fused = var_fwd_ == 2 || var_fwd_ > 100;
+    const bool fused = var_fwd_ >= 2;
     step_fwd_v(c_.snap_every > 0 && fused ? 1 : var_fwd_, it, act_min, hmode, cbase, traces);
   }
   void step_adj(int it, int cbase) { step_adj_v(var_adj_, it, cbase); }
@@ -2087,16 +2589,75 @@ class El2dEngine final : public Engine {
     SWX_HIP(hipGetLastError());
   }
 
+  // Row march: rows per chunk so that the waves of the batch are resident at
+  // once (from 5 rows on: a chunk loads 7 and steps the stresses of 4 more),
+  // and whether the row march takes the plan's shots at all: its byte offsets
+  // have 32 bits, a wave lists at most ER_TAPS moment-tensor taps of a family
+  // pair, and stress cells that accumulate moment tensors need the stresses in
+  // memory.
+  void choose_rows(int nshots, const int *nsrc, const swx_elastic_shot_desc *shots) {
+    int cus = 0, dev = 0;
+    SWX_HIP(hipGetDevice(&dev));
+    SWX_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    const int64_t cols = windows() * nshots;
+    for (int adj = 0; adj < 2; adj++) {
+      int per_cu = 0;
+      if (adj)
+        SWX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, el_row_kernel<T, true>, TX * ER_W, 0));
+      else
+        SWX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, el_row_kernel<T, false>, TX * ER_W, 0));
+      const int64_t chunks = std::max<int64_t>((int64_t)per_cu * ER_W * cus / cols, 1);
+      row_ch_[adj] = (int)std::clamp<int64_t>(ceil_div(nz_, chunks), 5, ER_ROWS);
+      if (const char *v = std::getenv("SWX_EL2D_ROWS")) row_ch_[adj] = std::clamp(std::atoi(v), 1, ER_ROWS);
+    }
+    rows_ok_ = std::max(N_, psi_stride_) * (int64_t)sizeof(T) < (int64_t(1) << 32) && !edge_taps_;
+    if (kind_ != SWX_SRC_MOMENT_TENSOR) return;
+    const int ch = row_ch_[0], nbx = (int)windows(), nbz = (int)ceil_div(nz_, ch);
+    std::vector<int> count;
+    for (int s = 0; s < nshots && rows_ok_; s++) {
+      count.assign((size_t)nbx * nbz, 0);
+      for (int f = 0; f < 2; f++)
+        for (int k = 0; k < shots[s].src[f].ptr[nsrc[s]]; k++) {
+          const int i = (int)shots[s].src[f].ij[2 * (int64_t)k], j = (int)shots[s].src[f].ij[2 * (int64_t)k + 1];
+          for (int bx = std::max((i - TX) / ER_OWN, 0); bx < nbx && bx * ER_OWN + 1 <= i; bx++)
+            for (int bz = std::max((j - 2 - ch) / ch, 0); bz < nbz && bz * ch - 1 <= j; bz++)
+              if (++count[(size_t)bz * nbx + bx] > ER_TAPS) rows_ok_ = false;
+        }
+    }
+  }
+  int64_t windows() const { return std::max<int64_t>(ceil_div(nx_ - 6, ER_OWN), 1); }
+
+  // a step of the row march; what the points add to the displacements follows
+  // in a launch of its own
+  template <bool ADJ>
+  void launch_rows(ElArgs<T> a, int kind) {
+    a.nbx = (int)windows();
+    a.ch = row_ch_[ADJ];
+    a.nbz = (int)ceil_div(nz_, a.ch);
+    a.nshots = nsh_;
+    const unsigned g = (unsigned)ceil_div((int64_t)a.nbx * a.nbz * nsh_, ER_W) + (unsigned)(a.nrecb * nsh_);
+    c_.ktimer.begin(c_.stream);
+    el_row_kernel<T, ADJ><<<g, TX * ER_W, 0, c_.stream>>>(a);
+    c_.ktimer.end(c_.stream, kind);
+    SWX_HIP(hipGetLastError());
+    const int most = ADJ ? max_ucell_[1] : max_ucell_[0];
+    if (a.kind == 2 && most > 0) {
+      dim3 b((unsigned)ceil_div(most, 64), (unsigned)nsh_, 2);
+      el_inject_kernel<T><<<b, 64, 0, c_.stream>>>(a);
+      SWX_HIP(hipGetLastError());
+    }
+  }
+
   // Variants: 0 = stress and displacement steps each as an interior-block
   // launch plus an other-block launch, 1 = the same steps with both kinds of
   // blocks in one launch each, 2 = both steps in one launch on 64 x R tiles
   // with the stresses in LDS, 102/104 = one z-marching launch on 128/256-
-  // column strips.  The tuner times 0, 1 and 2, and the z-marching variants
-  // when kMarchInTuner is set; the environment can pin any.
+  // column strips, 3 = the row march.  3 is taken where choose_rows allows it;
+  // elsewhere the tuner times 0, 1 and 2, and the z-marching variants when
+  // kMarchInTuner is set.  The environment can pin any.
   static constexpr bool kMarchInTuner = false;
   template <typename F>
-  int tune(const char *env, F step, bool forward) {
-    (void)forward;
+  int tune(const char *env, F step) {
     std::vector<int> cands = {0, 1, 2};
     if (kMarchInTuner) {
       cands.push_back(102);
@@ -2105,12 +2666,15 @@ class El2dEngine final : public Engine {
     if (const char *v = std::getenv(env)) {
       const int t = std::atoi(v);
       if (t == 0 || t == 1 || t == 2 || t == 102 || t == 104) return t;
+      if (t == 3 && rows_ok_) return t;
+    } else if (rows_ok_) {
+      return 3;
     }
     return cands[fastest_candidate(c_.stream, (int)cands.size(), [&](int k) { step(cands[k]); })];
   }
 
   void step_fwd_v(int v, int it, int act_min, int hmode, int cbase, T *traces) {
-    if (v == 2 || v > 100) {
+    if (v >= 2) {
       ElArgs<T> a = base_args(it);
       a.ucur = U(u_, it - 1);
       a.unew = U(u_, it);
@@ -2125,6 +2689,19 @@ class El2dEngine final : public Engine {
       a.kind = kind_ == SWX_SRC_MOMENT_TENSOR ? 1 : 2;
       a.hmode = c_.d.gradient ? hmode : 0;
       a.cbase = cbase;
+      if (v == 3) {
+        if (traces && it > 1) {   // the receivers of level it-1 ride on this launch
+          a.r0 = taps_[2].view<T>();
+          a.r1 = taps_[3].view<T>();
+          a.traces = traces;
+          a.off_tr = c_.pts.d_off_tr.as<int64_t>();
+          a.maxrec = maxrec_;
+          a.nrecb = (int)ceil_div(2 * maxrec_, TX * ER_W);
+        }
+        launch_rows<false>(a, 0);
+        if (it == ntmax_) record(it, traces);
+        return;
+      }
       if (a.kind == 1 && edge_taps_) {
         dim3 g((unsigned)ceil_div(std::max(max_ucell0_, 1), 64), (unsigned)nsh_);
         el_edge_inject_kernel<T><<<g, 64, 0, c_.stream>>>(a);
@@ -2175,7 +2752,7 @@ class El2dEngine final : public Engine {
   }
 
   void step_adj_v(int v, int it, int cbase) {
-    if (v == 2 || v > 100) {
+    if (v >= 2) {
       ElArgs<T> a = base_args(it);
       a.ucur = U(au_, it + 1);
       a.unew = U(au_, it);
@@ -2191,6 +2768,10 @@ class El2dEngine final : public Engine {
       a.tf = c_.pts.d_res.as<T>();
       a.off_tf = c_.pts.d_off_tr.as<int64_t>();
       a.ncomp = 2;
+      if (v == 3) {
+        launch_rows<true>(a, 1);
+        return;
+      }
       if (v == 2) {
         a.tbx = (int)ceil_div(nx_, TX);
         a.tbz = (int)ceil_div(nz_, ElTile<T>::rows);
@@ -2254,6 +2835,9 @@ class El2dEngine final : public Engine {
   int kind_ = SWX_SRC_MOMENT_TENSOR, maxrec_ = 0;
   bool edge_taps_ = false;
   int max_ucell0_ = 0;
+  int max_ucell_[2] = {0, 0};      // most cells of a shot with source, receiver taps
+  int row_ch_[2] = {5, 5};         // rows per chunk of the row march, forward and adjoint
+  bool rows_ok_ = false;
   int var_fwd_ = -1, var_adj_ = -1;
   // XCD-aware tile map of the block launches (env SWX_EL2D_XCD=0 turns it off)
   bool xcd_ = [] {
