@@ -55,7 +55,7 @@ struct TapView {
 template <typename T>
 struct ElArgs {
   int nx, nz, h, freetop;
-  int nbx, nbz, ch, nshots;     // z-marching launch: strips, chunks, rows per chunk
+  int nbx, nbz, ch;             // z-marching launch: strips, chunks, rows per chunk
   int tbx, tbz, xcd;            // block launches: tiles along x, z; XCD-aware tile map
   int order;                    // 1: the tiles outside [ibx0, ibx1] x [iby0, iby1] first
   int ibx0, ibx1, iby0, iby1;   // tiles clear of the C-PML strips and grid edges
@@ -82,6 +82,7 @@ struct ElArgs {
   // receivers of level it-1, recorded by the first nrecb blocks per shot of a row march
   TapView<T> r0, r1;
   T *traces; const int64_t *off_tr; int maxrec, nrecb;
+  const int4 *tiles; int ntiles, nslow, nbx_rows, nshots;   // row march: tiles of a shot, the first nslow in strips
 };
 
 // Block -> (strip, chunk, shot) map giving each of the 8 XCDs a contiguous
@@ -1621,12 +1622,13 @@ __global__ void el_record_kernel(const T *u, int64_t N, TapView<T> r0, TapView<T
 // u and the stresses staged in LDS, the stresses of a 68 x 20 region computed
 // for a tile) it loads a row of u once per wave and recomputes 6 of 64 columns
 // and 4 rows per chunk.  us per step, tile / row march: 813 x 407, 4 shots,
-// float32, forward 45 / 27; 1500 x 600, 12 shots, float32, forward 130 / 101
-// and adjoint 346 / 306 (88 bytes per cell of fields, history and gradients:
-// 3.1 TB/s); 331 x 257, 3 shots, float64, forward 34 / 20, adjoint 29 / 29.
-// What bounds it: the waves in the strips, which issue three (two axes) times
-// the instructions of an interior one per row, and in double precision the
-// adjoint's registers (one wave per SIMD).
+// float32, forward 45 / 22; 1500 x 600, 12 shots, float32, forward 130 / 88 and
+// adjoint 346 / 267; 331 x 257, 3 shots, float64, forward 34 / 19, adjoint 29 /
+// 28.  What bounds it: at 1500 x 600 memory (24 and 88 bytes per cell of fields,
+// history and gradients and 20 of the model, which the shots share in the last
+// cache: 5.4 and 4.4 TB/s with them); on small grids the corners' waves, which
+// issue three times the instructions of an interior one per row, and in double
+// precision the adjoint's registers (one wave per SIMD).
 constexpr int ER_OWN = 58, ER_W = 4;      // columns per window, waves per block
 constexpr int ER_ROWS = 56;               // most rows per chunk (64 lanes hold the coefficients of the rows loaded)
 constexpr int ER_TAPS = 128;              // most moment-tensor taps per wave
@@ -2031,14 +2033,20 @@ __global__ __launch_bounds__(TX *ER_W) void el_row_kernel(ElArgs<T> a) {
               b * (int)blockDim.x + (int)threadIdx.x);
     return;
   }
-  const int t = xcd_tile_el(blockIdx.x - nrec, gridDim.x - nrec) * ER_W + w;
-  const int bx = t % a.nbx, r = t / a.nbx, bz = r % a.nbz, s = r / a.nbz;
+  // the strips' tiles of all shots first (they take longest per row), then the
+  // interior ones, both dealt to the XCDs in contiguous runs
+  const int gslow = (a.nslow * a.nshots + ER_W - 1) / ER_W, b = (int)blockIdx.x - nrec;
+  const bool slow = b < gslow;
+  const int per = slow ? a.nslow : a.ntiles - a.nslow;
+  const int t = (slow ? xcd_tile_el(b, gslow) : xcd_tile_el(b - gslow, (int)gridDim.x - nrec - gslow)) * ER_W + w;
+  const int s = t / per;
   if (s >= a.nshots) return;
+  const int4 tile = a.tiles[(slow ? 0 : a.nslow) + t - s * per];   // window, rows [y, z)
   const int nts = a.nt_shot[s];
   if (a.it > nts || (!ADJ && nts <= a.act_min)) return;
   const int nx = a.nx, nz = a.nz, h = a.h;
-  const int X0 = bx * ER_OWN + 1, Z0 = bz * a.ch + 1, Z1 = min(Z0 + a.ch, nz + 1);
-  const bool own = X0 + lane <= nx && lane >= (bx ? 3 : 0) && lane < (bx < a.nbx - 1 ? TX - 3 : TX);
+  const int bx = tile.x, X0 = bx * ER_OWN + 1, Z0 = tile.y, Z1 = tile.z;
+  const bool own = X0 + lane <= nx && lane >= (bx ? 3 : 0) && lane < (bx < a.nbx_rows - 1 ? TX - 3 : TX);
   int n0 = 0, n1 = 0;
   if (!ADJ && a.kind == 1) {
     const int jr = Z0 - 2, j0 = max(jr, 1) - 1, j1 = min(Z1 + 1, nz);
@@ -2589,39 +2597,91 @@ class El2dEngine final : public Engine {
     SWX_HIP(hipGetLastError());
   }
 
-  // Row march: rows per chunk so that the waves of the batch are resident at
-  // once (from 5 rows on: a chunk loads 7 and steps the stresses of 4 more),
-  // and whether the row march takes the plan's shots at all: its byte offsets
-  // have 32 bits, a wave lists at most ER_TAPS moment-tensor taps of a family
-  // pair, and stress cells that accumulate moment tensors need the stresses in
-  // memory.
+  // Row march: the tiles of a shot, and whether it takes the plan's shots at
+  // all: its byte offsets have 32 bits, a wave lists at most ER_TAPS
+  // moment-tensor taps of a family pair, and stress cells that accumulate
+  // moment tensors need the stresses in memory.
+  //
+  // Rows per chunk: a wave in a strip takes COST times as long per row (x
+  // strips, z strips, both: instructions of the loops), so it gets fewer of
+  // them and starts first.  A corner's wave has at least 3 rows (a chunk steps
+  // the stresses of 4 more), which gives an interior one 16 (12 in the adjoint);
+  // chunks grow from there until the waves of the batch are resident at once,
+  // up to 40 (24) rows.  us per step with 16 / 24 / 40 / 56 rows, 1500 x 600, 12
+  // shots, float32: forward 102 / 95 / 88 / 91, adjoint 268 / 267 / 280 / 290;
+  // with the same 40 rows everywhere and in grid order 101 and 306.  813 x 407, 4
+  // shots, forward: 22 with 16 rows, 25 with 40, 27 with 5 rows everywhere.
   void choose_rows(int nshots, const int *nsrc, const swx_elastic_shot_desc *shots) {
+    static constexpr double COST[2][2] = {{1.0, 2.3}, {1.5, 2.9}};      // [x strip][z strip]
+    const int lo = std::max(3, h_ + 2), za = lo + 2, zb = std::min(nz_ - 2, nz_ - h_ - 2) - 1;
+    const int nbx = (int)windows();
+    auto xs = [&](int bx) {
+      const int X0 = bx * ER_OWN + 1;
+      return X0 < lo || X0 + TX - 1 > std::min(nx_ - 2, nx_ - h_ - 2);
+    };
     int cus = 0, dev = 0;
     SWX_HIP(hipGetDevice(&dev));
     SWX_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    const int64_t cols = windows() * nshots;
+    const char *pin = std::getenv("SWX_EL2D_ROWS");
+    std::vector<int4> fwd;
     for (int adj = 0; adj < 2; adj++) {
       int per_cu = 0;
       if (adj)
         SWX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, el_row_kernel<T, true>, TX * ER_W, 0));
       else
         SWX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, el_row_kernel<T, false>, TX * ER_W, 0));
-      const int64_t chunks = std::max<int64_t>((int64_t)per_cu * ER_W * cus / cols, 1);
-      row_ch_[adj] = (int)std::clamp<int64_t>(ceil_div(nz_, chunks), 5, ER_ROWS);
-      if (const char *v = std::getenv("SWX_EL2D_ROWS")) row_ch_[adj] = std::clamp(std::atoi(v), 1, ER_ROWS);
+      std::vector<int4> slow, rest;
+      const int most = pin ? std::clamp(std::atoi(pin), 1, ER_ROWS) : adj ? 24 : 40;
+      for (int ch = pin ? most : adj ? 12 : 16; ch <= most; ch++) {
+        slow.clear();
+        rest.clear();
+        // rows [r0, r1) of every window, by the strips they are in
+        auto add = [&](int r0, int r1, bool z) {
+          for (int x = 0; x < 2; x++) {
+            const int c = pin ? ch : std::max((int)((ch + 4) / COST[x][z]) - 4, 3);
+            const int n = r1 > r0 ? (int)ceil_div(r1 - r0, c) : 0;
+            for (int k = 0; k < n; k++)
+              for (int bx = 0; bx < nbx; bx++)
+                if (xs(bx) == (x != 0))
+                  (x || z ? slow : rest).push_back({bx, r0 + (int)((int64_t)(r1 - r0) * k / n),
+                                                    r0 + (int)((int64_t)(r1 - r0) * (k + 1) / n), 2 * x + z});
+          }
+        };
+        if (zb > za) {
+          add(1, za, true);
+          add(zb, nz_ + 1, true);
+          add(za, zb, false);
+        } else {
+          add(1, nz_ + 1, true);
+        }
+        if ((int64_t)(slow.size() + rest.size()) * nshots <= (int64_t)per_cu * ER_W * cus) break;
+      }
+      // the corners' tiles first
+      std::stable_sort(slow.begin(), slow.end(), [](const int4 &p, const int4 &q) {
+        return COST[p.w >> 1][p.w & 1] > COST[q.w >> 1][q.w & 1];
+      });
+      nslow_[adj] = (int)slow.size();
+      slow.insert(slow.end(), rest.begin(), rest.end());
+      ntiles_[adj] = (int)slow.size();
+      tiles_[adj].alloc(slow.size() * sizeof(int4));
+      SWX_HIP(hipMemcpyAsync(tiles_[adj].get(), slow.data(), slow.size() * sizeof(int4), hipMemcpyHostToDevice,
+                             c_.stream));
+      SWX_HIP(hipStreamSynchronize(c_.stream));
+      if (!adj) fwd = slow;
     }
     rows_ok_ = std::max(N_, psi_stride_) * (int64_t)sizeof(T) < (int64_t(1) << 32) && !edge_taps_;
     if (kind_ != SWX_SRC_MOMENT_TENSOR) return;
-    const int ch = row_ch_[0], nbx = (int)windows(), nbz = (int)ceil_div(nz_, ch);
-    std::vector<int> count;
+    std::vector<std::vector<int>> of(nbx);      // tiles of a window
+    for (size_t t = 0; t < fwd.size(); t++) of[fwd[t].x].push_back((int)t);
+    std::vector<int> count(fwd.size());
     for (int s = 0; s < nshots && rows_ok_; s++) {
-      count.assign((size_t)nbx * nbz, 0);
+      std::fill(count.begin(), count.end(), 0);
       for (int f = 0; f < 2; f++)
         for (int k = 0; k < shots[s].src[f].ptr[nsrc[s]]; k++) {
           const int i = (int)shots[s].src[f].ij[2 * (int64_t)k], j = (int)shots[s].src[f].ij[2 * (int64_t)k + 1];
           for (int bx = std::max((i - TX) / ER_OWN, 0); bx < nbx && bx * ER_OWN + 1 <= i; bx++)
-            for (int bz = std::max((j - 2 - ch) / ch, 0); bz < nbz && bz * ch - 1 <= j; bz++)
-              if (++count[(size_t)bz * nbx + bx] > ER_TAPS) rows_ok_ = false;
+            for (int t : of[bx])
+              if (j >= fwd[t].y - 2 && j <= fwd[t].z + 1 && ++count[t] > ER_TAPS) rows_ok_ = false;
         }
     }
   }
@@ -2631,11 +2691,13 @@ class El2dEngine final : public Engine {
   // in a launch of its own
   template <bool ADJ>
   void launch_rows(ElArgs<T> a, int kind) {
-    a.nbx = (int)windows();
-    a.ch = row_ch_[ADJ];
-    a.nbz = (int)ceil_div(nz_, a.ch);
+    a.tiles = tiles_[ADJ].as<int4>();
+    a.ntiles = ntiles_[ADJ];
+    a.nslow = nslow_[ADJ];
+    a.nbx_rows = (int)windows();
     a.nshots = nsh_;
-    const unsigned g = (unsigned)ceil_div((int64_t)a.nbx * a.nbz * nsh_, ER_W) + (unsigned)(a.nrecb * nsh_);
+    const unsigned g = (unsigned)(ceil_div((int64_t)a.nslow * nsh_, ER_W) +
+                                  ceil_div((int64_t)(a.ntiles - a.nslow) * nsh_, ER_W) + (int64_t)a.nrecb * nsh_);
     c_.ktimer.begin(c_.stream);
     el_row_kernel<T, ADJ><<<g, TX * ER_W, 0, c_.stream>>>(a);
     c_.ktimer.end(c_.stream, kind);
@@ -2836,7 +2898,8 @@ class El2dEngine final : public Engine {
   bool edge_taps_ = false;
   int max_ucell0_ = 0;
   int max_ucell_[2] = {0, 0};      // most cells of a shot with source, receiver taps
-  int row_ch_[2] = {5, 5};         // rows per chunk of the row march, forward and adjoint
+  DevBuf tiles_[2];                // of the row march, forward and adjoint
+  int ntiles_[2] = {0, 0}, nslow_[2] = {0, 0};
   bool rows_ok_ = false;
   int var_fwd_ = -1, var_adj_ = -1;
   // XCD-aware tile map of the block launches (env SWX_EL2D_XCD=0 turns it off)
