@@ -319,8 +319,8 @@ def alg_bytes(physics, n, halo, e, nts, S, variant=(0, 0)):
             # and written once per step.  A variant with two launches per step
             # (stress, displacement) is priced at the same bytes per step.
             # (one launch per step: the z-marching variants > 100 and the
-            # fused tile step 2)
-            march_f, march_a = variant[0] > 100 or variant[0] == 2, variant[1] > 100 or variant[1] == 2
+            # fused tile step 2 and the row march 3)
+            march_f, march_a = variant[0] > 100 or variant[0] in (2, 3), variant[1] > 100 or variant[1] in (2, 3)
             last = nt - (nt // S) * S
             rep = (nt // S) * (S - 1)
             est = _el_strip_cells(n, halo) * 2 * e
@@ -328,6 +328,18 @@ def alg_bytes(physics, n, halo, e, nts, S, variant=(0, 0)):
             fwd_n += (1 if march_f else 2) * (nt + rep)
             adj_b += nt * 27 * e * N + nt * est
             adj_n += (1 if march_a else 2) * nt
+            continue
+        if physics == "vd2d" and 500 < variant[0] % 1000 < 600:
+            # n levels per launch: a launch reads p, vx, vz, m0, m1x, m1z and
+            # writes p, vx, vz once (9e); + w p-history (1e) per stored step.
+            # Launches end at multiples of S; an adjoint step as below.
+            lv = variant[0] - 500
+            nl = sum(-(-(min((k + 1) * S, nt) - k * S) // lv) for k in range(-(-nt // S)))
+            nl += (nt // S) * -(-(S - 1) // lv)
+            fwd_b += nl * (9 * e * N + strip) + (last + rep) * e * N
+            fwd_n += nl
+            adj_b += nt * (14 if vd_groups[1] > 1 else 17) * e * N + nt * strip
+            adj_n += nt
             continue
         if physics == "vd2d" and (vd_groups[0] > 1 or vd_groups[1] > 1):
             # two shots per block (4xx) or shot groups in the block order
@@ -427,6 +439,8 @@ def kernel_names(physics, variant):
     if physics == "vd2d":
         def name(kind, v):
             v %= 1000      # the thousands give the shot groups of the block order
+            if v > 500:    # several levels per launch
+                return f"vd2d_stepn_kernel<float, 4, 16> ({v - 500} levels per launch)"
             if v >= 400:   # two shots per block, one launch
                 return f"vd2d_{kind}_pair_kernel<float, {v - 400}>"
             if v >= 300:   # interior and other tiles in one launch

@@ -26,7 +26,7 @@
 
 #include <hip/hip_ext.h>
 
-#include "swx_device.hpp"
+#include "swx_levels.hpp"
 #include "swx_internal.hpp"
 
 namespace swx {
@@ -311,10 +311,6 @@ __global__ __launch_bounds__(TX *TZ) void cd2d_step_kernel(Cd2dStepArgs<T> a) {
 //   f32 1000 x 1000:      forward 7.9 -> 3.9, adjoint + replay  15.9 -> 7.2
 //   f64 12 x 397 x 253:   forward  15 -> 6.2, adjoint + replay    33 -> 13
 
-constexpr int SN_MAX = 8;        // most levels per launch
-constexpr int SN_SLOTS = 126;    // staged point values per level
-constexpr int SN_RECS = 254;     // receivers whose traces are kept
-
 template <typename T>
 struct Cd2dStepNArgs {
   Cd2dStepArgs<T> a;   // a.it: first level; a.pnew: the last level stepped
@@ -323,15 +319,9 @@ struct Cd2dStepNArgs {
 };
 
 template <typename T, int R, int NW>
-struct Cd2dNLds {
+struct Cd2dNLds : LevelPoints<T, NW * R> {
   T first[2][NW][TX], last[2][NW][TX], lastz[2][NW][TX];   // rows 0 and R-1 of p, row R-1 of psi_z
   T cz[NW * R + 1][4];         // z C-PML coefficients b_h, a_h, b, a of the rows, from the one before
-  short inj[NW * R][TX];       // staged values of a cell's points: slot + 1 and, above bit 7, their number;
-                               // 0: no point, -1: not staged
-  short rec[NW * R][TX];       // a cell's entries of col: first + 1 and, above bit 8, their number; 0, -1 alike
-  T val[SN_MAX][SN_SLOTS];
-  int col[SN_RECS];            // traces of the window's receivers
-  int used, rused;             // slots and entries taken
 };
 
 // Registers of one thread: R cells of a column.
@@ -341,46 +331,6 @@ struct Cd2dNRegs {
   T psx[R], xix[R], psz[R], xiz[R];
 };
 
-// Window of a block and what its threads own.
-struct Cd2dNWin {
-  int i, j0, w, lane;
-  bool own;            // column owned
-  int rows;            // rows of this wave owned (bit r: row r)
-  int jin, kzr, xzr;   // rows inside the grid's z edges, with a psi_z / a xi_z
-  int imask, rmask;    // rows that hold injected points / receivers
-};
-
-// Injection of the level with index m (of the nl staged ones) and number l at
-// row r: p += value (times the factor in the adjoint), in list order.
-template <typename T, int R, int NW, bool ADJ>
-__device__ __forceinline__ void cd2d_n_inject(const Cd2dStepArgs<T> &a, const Cd2dNLds<T, R, NW> &L,
-                                              const Cd2dNWin &W, int s, int nts, int r, int m, int l, T f, T &pnv,
-                                              T &inj) {
-  const int e = L.inj[W.w * R + r][W.lane];
-  if (e == 0) return;
-  auto add = [&](T v) {
-    if (ADJ) {
-      pnv += v * f;
-    } else {
-      pnv += v;
-      inj += v;
-    }
-  };
-  if (e > 0) {
-    const T *v = L.val[m] + (e & 127) - 1;
-#pragma clang loop unroll(disable)
-    for (int k = 0; k < e >> 7; k++) add(v[k]);
-    return;
-  }
-  const int *ptr = ADJ ? a.pt.urec_ptr : a.pt.usrc_ptr, *list = ADJ ? a.pt.urec_list : a.pt.usrc_list;
-  const T *tf = (ADJ ? a.res + a.pt.off_tr[s] : a.srctf + a.pt.off_tf[s]) + (l - 1);
-  const int j = W.j0 + r;
-  const int u = find_point(ADJ ? a.pt.rrow : a.pt.srow, ADJ ? a.pt.urec_cell : a.pt.usrc_cell, a.pt.nrows, s, j,
-                           (int64_t)j * a.nx + W.i);
-#pragma clang loop unroll(disable)
-  for (int k = ptr[u]; k < ptr[u + 1]; k++) add(tf[(int64_t)nts * list[k]]);
-}
-
 // One level on a thread's R cells.  XS: the window reaches an x strip or x
 // edge; ZS: the wave's rows reach a z strip or z edge.  up / dn: values of
 // the row before the first / after the last, zup: old psi_z of the row
@@ -388,7 +338,7 @@ __device__ __forceinline__ void cd2d_n_inject(const Cd2dStepArgs<T> &a, const Cd
 // injection).
 template <typename T, int R, int NW, bool ADJ, bool XS, bool ZS>
 __device__ __forceinline__ void cd2d_n_level(const Cd2dStepArgs<T> &a, const Cd2dNLds<T, R, NW> &L,
-                                             const Cd2dNWin &W, int kx, const T *xc, T up, T dn, T zup,
+                                             const LevelWin &W, int kx, const T *xc, T up, T dn, T zup,
                                              Cd2dNRegs<T, R> &G, T *dv) {
   const int nx = a.nx, h = a.h, i = W.i;
   const bool xin = !XS || (i >= 1 && i <= nx - 2);
@@ -457,70 +407,6 @@ __device__ __forceinline__ void cd2d_n_level(const Cd2dStepArgs<T> &a, const Cd2
   }
 }
 
-// Points of the wave's rows: the cells' entries in LDS, and (injected points)
-// their values of the levels la, la + dir, .. (nl of them).
-template <typename T, int R, int NW, bool ADJ>
-__device__ __forceinline__ void cd2d_n_points(const Cd2dStepArgs<T> &a, Cd2dNLds<T, R, NW> &L, Cd2dNWin &W, int s,
-                                              int nts, int X0, int la, int nl) {
-  const int64_t ro = (int64_t)s * (a.pt.nrows + 1);
-  const int *irow = (ADJ ? a.pt.rrow : a.pt.srow) + ro, *rrow = a.pt.rrow + ro;
-  const int64_t *icell = ADJ ? a.pt.urec_cell : a.pt.usrc_cell;
-  const int *iptr = ADJ ? a.pt.urec_ptr : a.pt.usrc_ptr, *ilist = ADJ ? a.pt.urec_list : a.pt.usrc_list;
-  const T *tf = ADJ ? a.res + a.pt.off_tr[s] : a.srctf + a.pt.off_tf[s];
-  // bounds of the rows' points, one row per lane
-  const int jl = min(W.j0 + min(W.lane, R), a.nz);
-  const int ib = irow[min(jl, a.nz)], rb = (!ADJ && a.traces) ? rrow[min(jl, a.nz)] : 0;
-  W.imask = W.rmask = 0;
-#pragma unroll
-  for (int r = 0; r < R; r++) {
-    if (__shfl(ib, r) != __shfl(ib, r + 1)) W.imask |= 1 << r;
-    if (__shfl(rb, r) != __shfl(rb, r + 1)) W.rmask |= 1 << r;
-  }
-  W.imask = __builtin_amdgcn_readfirstlane(W.imask);
-  W.rmask = __builtin_amdgcn_readfirstlane(W.rmask);
-  if (!(W.imask | W.rmask)) return;
-  for (int r = 0; r < R; r++) {
-    const int64_t c0 = (int64_t)(W.j0 + r) * a.nx + X0;
-    if (W.imask >> r & 1) {
-      L.inj[W.w * R + r][W.lane] = 0;
-      __builtin_amdgcn_wave_barrier();
-      const int q1 = __shfl(ib, r + 1);
-      for (int q = __shfl(ib, r) + W.lane; q < q1; q += TX) {
-        const int64_t o = icell[q] - c0;
-        if (o < 0 || o >= TX) continue;
-        const int k0 = iptr[q], cnt = iptr[q + 1] - k0;
-        const int slot = cnt <= SN_SLOTS ? atomicAdd(&L.used, cnt) : SN_SLOTS;
-        if (slot + cnt > SN_SLOTS) {
-          L.inj[W.w * R + r][o] = -1;
-          continue;
-        }
-        for (int k = 0; k < cnt; k++) {
-          const T *v = tf + (int64_t)nts * ilist[k0 + k] + (la - 1);
-          for (int m = 0; m < nl; m++) L.val[m][slot + k] = v[ADJ ? -m : m];
-        }
-        L.inj[W.w * R + r][o] = (short)((slot + 1) | cnt << 7);
-      }
-    }
-    if (W.rmask >> r & 1) {
-      L.rec[W.w * R + r][W.lane] = 0;
-      __builtin_amdgcn_wave_barrier();
-      const int q1 = __shfl(rb, r + 1);
-      for (int q = __shfl(rb, r) + W.lane; q < q1; q += TX) {
-        const int64_t o = a.pt.urec_cell[q] - c0;
-        if (o < 0 || o >= TX) continue;
-        const int k0 = a.pt.urec_ptr[q], cnt = a.pt.urec_ptr[q + 1] - k0;
-        const int first = cnt <= 127 ? atomicAdd(&L.rused, cnt) : SN_RECS;
-        if (first + cnt > SN_RECS) {
-          L.rec[W.w * R + r][o] = -1;
-          continue;
-        }
-        for (int k = 0; k < cnt; k++) L.col[first + k] = a.pt.urec_list[k0 + k];
-        L.rec[W.w * R + r][o] = (short)((first + 1) | cnt << 8);
-      }
-    }
-  }
-}
-
 // Forward / replay levels it .. it+n-1, or (ADJ) adjoint levels it .. it-n+1
 // with their injection and their correlation with the forward history.
 template <typename T, int R, int NW, bool ADJ>
@@ -536,7 +422,7 @@ __global__ __launch_bounds__(NW *TX, sizeof(T) == 4 ? 4 : 2) void cd2d_stepn_ker
   const int nts = a.nt_shot[s];
   const int n = A.n, nx = a.nx, nz = a.nz, h = a.h;
   const int X0 = bx * (TX - 2 * n), Z0 = by * (H - 2 * n);
-  Cd2dNWin W;
+  LevelWin W;
   W.lane = threadIdx.x & (TX - 1);
   W.w = __builtin_amdgcn_readfirstlane(threadIdx.x / TX);
   W.i = X0 + W.lane;
@@ -628,7 +514,7 @@ __global__ __launch_bounds__(NW *TX, sizeof(T) == 4 ? 4 : 2) void cd2d_stepn_ker
   }
   // (loaded here: a load in the level loop would wait for the wave's stores)
   const int64_t otr = a.pt.off_tr[s];
-  cd2d_n_points<T, R, NW, ADJ>(a, L, W, s, nts, X0, la, nl);
+  level_points<T, R, ADJ>(a, L, W, s, nts, X0, la, nl);
   if (threadIdx.x <= H) {
     const int j = Z0 - 1 + (int)threadIdx.x;
     int kz = -1;
@@ -670,7 +556,7 @@ __global__ __launch_bounds__(NW *TX, sizeof(T) == 4 ? 4 : 2) void cd2d_stepn_ker
         if (W.imask >> r & 1) {
           T inj = 0;
           const T before = G.pc[r];      // of an edge cell: its level before last
-          cd2d_n_inject<T, R, NW, ADJ>(a, L, W, s, nts, r, m, l, G.fa[r], G.pc[r], inj);
+          level_inject<T, R, ADJ>(a, L, W, s, nts, r, m, l, G.fa[r], G.pc[r], inj);
           if (!ADJ) {
             const bool interior = W.i >= 1 && W.i <= nx - 2 && (W.jin >> r & 1);
             dval[r] = interior ? dval[r] + inj : (before - T(2) * G.po[r]) + G.pc[r];

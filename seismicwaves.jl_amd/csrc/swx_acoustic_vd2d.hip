@@ -36,7 +36,7 @@
 #include <algorithm>
 #include <cstdlib>
 
-#include "swx_device.hpp"
+#include "swx_levels.hpp"
 #include "swx_internal.hpp"
 
 namespace swx {
@@ -849,6 +849,302 @@ __global__ __launch_bounds__(NB) void vd2d_fwd2_kernel(Vd2dArgs<T> a) {
   p_phase(a.it + 1, true, true);   // p^{it+1} on P2
   __syncthreads();
   v_phase(true, true);          // v^{it+1} on the tile, to HBM
+}
+
+// ---------------------------------------------------------------------------
+// Several forward / replay levels per launch (vd2d_stepn_kernel).
+//
+// A block of NW waves holds a 64 x (NW R) window of pressure, velocities and
+// model factors in registers (lane = column, R rows per wave) and steps it n
+// times.  A level reaches three cells to every side (pressure from velocities
+// two cells before and one after, velocities from the new pressure one before
+// and two after), so the block owns, and writes, the cells at least 3 n from
+// the window's sides (all cells up to a side that is the grid's).  x
+// neighbours come from the adjacent lanes, z neighbours from the thread's own
+// rows; the last two and the first velocity row of each wave, then the last
+// and the first two pressure rows, pass through LDS: two barriers per level.
+// The C-PML memory variables of the strip cells step along in registers; point
+// values of the n levels are staged in LDS once.  Cell updates are spelled as
+// in vd2d_fwd_general_tile: results are bitwise those of n single steps.
+//
+// Bound by latency on small grids (701 x 403 float32: 19 us for 5 levels, 9.7 us
+// for one of the tile steps) and by instruction issue on large ones, where the
+// windows step 1.9 (3 levels) times the owned cells (1000 x 700, 8 shots
+// float32: 49 -> 38 us per level; 2000 x 800, 32 shots: 349 -> 315).
+template <typename T, int R, int NW>
+struct Vd2dNLds : LevelPoints<T, NW * R> {
+  T vz[3][NW][TX];             // rows R-2, R-1 and 0 of vz
+  T p[3][NW][TX];              // rows R-1, 0 and 1 of the new pressure
+  T cz[NW * R][4];             // z C-PML coefficients b, a (pressure), b_h, a_h (velocity) of the rows
+};
+
+// Registers of one thread: R cells of a column.
+template <typename T, int R>
+struct Vd2dNRegs {
+  T p[R], vx[R], vz[R], m0[R], m1x[R], m1z[R];
+  T xix[R], xiz[R], psx[R], psz[R];
+};
+
+// Pressure of one level; vu2, vu1: vz of the two rows before the wave's, vd of
+// the one after.  XS: the window reaches an x strip or side; ZS: the wave's
+// rows reach a z strip or side.
+template <typename T, int R, int NW, bool XS, bool ZS>
+__device__ __forceinline__ void vd2d_n_pressure(const Vd2dArgs<T> &a, const Vd2dNLds<T, R, NW> &L, const LevelWin &W,
+                                                bool xst, const T *xc, T vu2, T vu1, T vd, Vd2dNRegs<T, R> &G) {
+  const bool xin = !XS || (W.i >= 1 && W.i <= a.nx - 2);
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    const T x0 = G.vx[r], x1 = lane_before(x0), x2 = lane_before(x1);
+    T dvx = d4(x2, x1, x0, lane_after(x0)) * a.idx;
+    T dvz = d4(r > 1 ? G.vz[r > 1 ? r - 2 : 0] : r > 0 ? vu1 : vu2, r > 0 ? G.vz[r > 0 ? r - 1 : 0] : vu1, G.vz[r],
+               r + 1 < R ? G.vz[r + 1 < R ? r + 1 : r] : vd) * a.idz;
+    const bool interior = xin && (!ZS || (W.jin >> r & 1));
+    if (XS) {
+      const T xi = xc[0] * G.xix[r] + xc[1] * dvx;
+      if (xst && interior) {
+        G.xix[r] = xi;
+        dvx = dvx + xi;
+      }
+    }
+    if (ZS) {
+      if (W.xzr >> r & 1) {
+        const T *c = L.cz[W.w * R + r];
+        const T xi = c[0] * G.xiz[r] + c[1] * dvz;
+        if (interior) {
+          G.xiz[r] = xi;
+          dvz = dvz + xi;
+        }
+      }
+    }
+    const T pv = G.p[r] - G.m0[r] * (dvx + dvz);
+    G.p[r] = interior ? pv : G.p[r];
+  }
+}
+
+// Velocities of one level; pu: new pressure of the row before the wave's, pd1,
+// pd2 of the two after.
+template <typename T, int R, int NW, bool XS, bool ZS>
+__device__ __forceinline__ void vd2d_n_velocity(const Vd2dArgs<T> &a, const Vd2dNLds<T, R, NW> &L, const LevelWin &W,
+                                                bool pst, const T *xc, T pu, T pd1, T pd2, Vd2dNRegs<T, R> &G) {
+  const bool xv = !XS || W.i <= a.nx - 2, xg = !XS || W.i <= a.nx - 1;
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    const T p0 = G.p[r], p1 = lane_after(p0), p2 = lane_after(p1);
+    T dx = d4(lane_before(p0), p0, p1, p2) * a.idx;
+    T dz = d4(r > 0 ? G.p[r > 0 ? r - 1 : 0] : pu, p0, r + 1 < R ? G.p[r + 1 < R ? r + 1 : r] : pd1,
+              r + 2 < R ? G.p[r + 2 < R ? r + 2 : r] : r + 1 < R ? pd1 : pd2) * a.idz;
+    if (XS) {
+      const T ps = xc[2] * G.psx[r] + xc[3] * dx;
+      if (pst) {
+        G.psx[r] = ps;
+        dx = dx + ps;
+      }
+    }
+    if (ZS) {
+      if (W.kzr >> r & 1) {
+        const T *c = L.cz[W.w * R + r];
+        const T ps = c[2] * G.psz[r] + c[3] * dz;
+        G.psz[r] = ps;
+        dz = dz + ps;
+      }
+    }
+    const T vx = G.vx[r] - G.m1x[r] * dx, vz = G.vz[r] - G.m1z[r] * dz;
+    G.vx[r] = xv && (!ZS || (W.jg >> r & 1)) ? vx : G.vx[r];
+    G.vz[r] = xg && (!ZS || (W.jv >> r & 1)) ? vz : G.vz[r];
+  }
+}
+
+template <typename T, int R, int NW>
+__global__ __launch_bounds__(NW *TX, sizeof(T) == 4 ? 4 : 2) void vd2d_stepn_kernel(Vd2dArgs<T> a, int n) {
+  __shared__ Vd2dNLds<T, R, NW> L;
+  constexpr int H = NW * R;
+  if (threadIdx.x == 0) L.used = L.rused = 0;
+  __syncthreads();
+  const int b = xcd_tile(blockIdx.x, gridDim.x);
+  const int t = b / a.nbx;
+  const int bx = b - t * a.nbx, by = t % a.nbz, s = t / a.nbz;
+  const int nts = a.nt_shot[s];
+  const int nx = a.nx, nz = a.nz, h = a.h;
+  const int X0 = bx * (TX - 6 * n), Z0 = by * (H - 6 * n);
+  LevelWin W;
+  W.lane = threadIdx.x & (TX - 1);
+  W.w = __builtin_amdgcn_readfirstlane(threadIdx.x / TX);
+  W.i = X0 + W.lane;
+  W.j0 = Z0 + W.w * R;
+  W.own = W.i < nx && W.lane >= (bx ? 3 * n : 0) && W.lane < (bx < a.nbx - 1 ? TX - 3 * n : TX);
+  W.rows = W.jin = W.kzr = W.xzr = W.jg = W.jv = 0;
+  const int own0 = by ? Z0 + 3 * n : 0, own1 = by < a.nbz - 1 ? Z0 + H - 3 * n : nz;
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    const int j = W.j0 + r;
+    if (j >= own0 && j < own1) W.rows |= 1 << r;
+    if (j < nz) W.jg |= 1 << r;
+    if (j <= nz - 2) W.jv |= 1 << r;
+    if (j >= 1 && j <= nz - 2) {
+      W.jin |= 1 << r;
+      if (j <= h || j >= nz - h - 1) W.xzr |= 1 << r;
+    }
+    if (j < h || (j >= nz - h - 1 && j <= nz - 2)) W.kzr |= 1 << r;
+  }
+  const int64_t so = (int64_t)s * a.N;
+  const bool xs = X0 <= max(h, 1) || X0 + TX - 1 >= nx - h - 1;
+  const bool zs = W.j0 <= max(h, 1) || W.j0 + R - 1 >= nz - h - 1;
+  // strip entries of the column: pressure (xi), velocity (psi)
+  const bool xst = W.i >= 1 && W.i <= nx - 2 && (W.i <= h || W.i >= nx - h - 1);
+  const bool pst = W.i < h || (W.i >= nx - h - 1 && W.i <= nx - 2);
+  const int kxi = xst ? (W.i <= h ? W.i : W.i - nx + 2 * h + 2) : 0, kps = pst ? (W.i < h ? W.i : W.i + 1 - nx + 2 * h) : 0;
+
+  // Fields and factors, zero outside their grids (the derivative rule).
+  Vd2dNRegs<T, R> G;
+  const unsigned ic = min(W.i, nx - 1);
+  auto row = [&](const T *p, int r) { return p + (int64_t)min(W.j0 + r, nz - 1) * nx; };
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    G.p[r] = row(a.p_o + so, r)[ic];
+    G.vx[r] = row(a.vx_o + so, r)[ic];
+    G.vz[r] = row(a.vz_o + so, r)[ic];
+    G.m0[r] = row(a.m0, r)[ic];
+    G.m1x[r] = row(a.m1x, r)[ic];
+    G.m1z[r] = row(a.m1z, r)[ic];
+    G.xix[r] = G.xiz[r] = G.psx[r] = G.psz[r] = T(0);
+  }
+  auto zxi = [&](int r) { return W.j0 + r <= h ? W.j0 + r : W.j0 + r - nz + 2 * h + 2; };
+  auto zps = [&](int r) { return W.j0 + r < h ? W.j0 + r : W.j0 + r + 1 - nz + 2 * h; };
+  T xc[4] = {T(0), T(0), T(0), T(0)};
+  if (xs && h > 0) {
+    const AxisCoef<T> cx = axis_coef(a.cpml + (int64_t)s * a.cstride, h, 0);
+    const T c0 = cx.b(kxi), c1 = cx.a(kxi), c2 = cx.bh(kps), c3 = cx.ah(kps);
+    xc[0] = c0;
+    xc[1] = c1;
+    xc[2] = c2;
+    xc[3] = c3;
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      const int64_t j = min(W.j0 + r, nz - 1);
+      G.xix[r] = (a.xix_o + (int64_t)s * a.sxx + j * (2 * h + 2))[(unsigned)kxi];
+      G.psx[r] = (a.psx_o + (int64_t)s * a.spx + j * (2 * h))[(unsigned)kps];
+    }
+  }
+  if (zs) {
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      if (W.xzr >> r & 1) G.xiz[r] = (a.xiz_o + (int64_t)s * a.sxz + (int64_t)zxi(r) * nx)[ic];
+      if (W.kzr >> r & 1) G.psz[r] = (a.psz_o + (int64_t)s * a.spz + (int64_t)zps(r) * nx)[ic];
+    }
+  }
+  // Levels of this shot: up to nts.  Tested after the loads above were issued,
+  // so that they do not wait for nts.
+  const int nl = min(n, nts - a.it + 1);
+  if (nl <= 0 || nts <= a.act_min) return;
+  if (xs || zs) {
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      const bool g = W.i < nx && (W.jg >> r & 1);
+      G.p[r] = g ? G.p[r] : T(0);
+      G.vx[r] = g && W.i <= nx - 2 ? G.vx[r] : T(0);
+      G.vz[r] = g && (W.jv >> r & 1) ? G.vz[r] : T(0);
+    }
+  }
+  const int64_t otr = a.pt.off_tr[s];     // (here: a load in the level loop would wait for the wave's stores)
+  level_points<T, R, false>(a, L, W, s, nts, X0, a.it, nl);
+  if (threadIdx.x < H) {
+    const int j = Z0 + (int)threadIdx.x;
+    const AxisCoef<T> cz = axis_coef(a.cpml + (int64_t)s * a.cstride, h, 1);
+    T *q = L.cz[threadIdx.x];
+    const bool x = j >= 1 && j <= nz - 2 && (j <= h || j >= nz - h - 1), v = j < h || (j >= nz - h - 1 && j <= nz - 2);
+    const int kx = j <= h ? j : j - nz + 2 * h + 2, kv = j < h ? j : j + 1 - nz + 2 * h;
+    q[0] = x ? cz.b(kx) : T(0);
+    q[1] = x ? cz.a(kx) : T(0);
+    q[2] = v ? cz.bh(kv) : T(0);
+    q[3] = v ? cz.ah(kv) : T(0);
+  }
+  const int seg0 = store_base(a.smode, 1 << 30, nts, a.S, a.cbase);    // level l > seg0 >= 0 goes to slot l - seg0
+
+#pragma clang loop unroll(disable)
+  for (int m = 0; m < nl; m++) {
+    opaque(W.j0);
+    opaque(W.rows);
+    opaque(W.jin);
+    opaque(W.kzr);
+    opaque(W.xzr);
+    opaque(W.jg);
+    opaque(W.jv);
+    opaque(W.imask);
+    opaque(W.rmask);
+    const int l = a.it + m;
+    const int wu = W.w > 0 ? W.w - 1 : 0, wd = W.w < NW - 1 ? W.w + 1 : NW - 1;
+    L.vz[0][W.w][W.lane] = G.vz[R - 2];
+    L.vz[1][W.w][W.lane] = G.vz[R - 1];
+    L.vz[2][W.w][W.lane] = G.vz[0];
+    __syncthreads();
+    {
+      // (beyond the window: zero, what the grid's own sides need)
+      T vu2 = L.vz[0][wu][W.lane], vu1 = L.vz[1][wu][W.lane], vd = L.vz[2][wd][W.lane];
+      if (W.w == 0) vu2 = vu1 = T(0);
+      if (W.w == NW - 1) vd = T(0);
+      if (seg0 >= 0 && a.smode == 1 && l == seg0 + 1 && W.own) {
+#pragma unroll
+        for (int r = 0; r < R; r++)
+          if (W.rows >> r & 1) (a.pbuf + so + (int64_t)(W.j0 + r) * nx)[ic] = G.p[r];
+      }
+      if (xs) vd2d_n_pressure<T, R, NW, true, true>(a, L, W, xst, xc, vu2, vu1, vd, G);
+      else if (zs) vd2d_n_pressure<T, R, NW, false, true>(a, L, W, xst, xc, vu2, vu1, vd, G);
+      else vd2d_n_pressure<T, R, NW, false, false>(a, L, W, xst, xc, vu2, vu1, vd, G);
+    }
+    if (W.imask | W.rmask) {
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        if (W.imask >> r & 1) {
+          T inj = 0;
+          level_inject<T, R, false>(a, L, W, s, nts, r, m, l, T(0), G.p[r], inj);
+        }
+        if ((W.rmask & W.rows) >> r & 1 && W.own) {
+          const int e = L.rec[W.w * R + r][W.lane];
+          T *tr = a.traces + otr + (l - 1);
+          if (e > 0) {
+#pragma clang loop unroll(disable)
+            for (int k = 0; k < e >> 8; k++) tr[(int64_t)nts * L.col[(e & 255) - 1 + k]] = G.p[r];
+          } else if (e < 0) {
+            const int j = W.j0 + r;
+            const int u = find_point(a.pt.rrow, a.pt.urec_cell, a.pt.nrows, s, j, (int64_t)j * nx + W.i);
+#pragma clang loop unroll(disable)
+            for (int k = a.pt.urec_ptr[u]; k < a.pt.urec_ptr[u + 1]; k++)
+              tr[(int64_t)nts * a.pt.urec_list[k]] = G.p[r];
+          }
+        }
+      }
+    }
+    L.p[0][W.w][W.lane] = G.p[R - 1];
+    L.p[1][W.w][W.lane] = G.p[0];
+    L.p[2][W.w][W.lane] = G.p[1];
+    __syncthreads();
+    T pu = L.p[0][wu][W.lane], pd1 = L.p[1][wd][W.lane], pd2 = L.p[2][wd][W.lane];
+    if (W.w == 0) pu = T(0);
+    if (W.w == NW - 1) pd1 = pd2 = T(0);
+    if (xs) vd2d_n_velocity<T, R, NW, true, true>(a, L, W, pst, xc, pu, pd1, pd2, G);
+    else if (zs) vd2d_n_velocity<T, R, NW, false, true>(a, L, W, pst, xc, pu, pd1, pd2, G);
+    else vd2d_n_velocity<T, R, NW, false, false>(a, L, W, pst, xc, pu, pd1, pd2, G);
+    if (seg0 >= 0 && l > seg0 && W.own) {
+      T *hs = a.pbuf + (int64_t)(l - seg0) * a.pslot + so;
+#pragma unroll
+      for (int r = 0; r < R; r++)
+        if (W.rows >> r & 1) st_nt(hs + (int64_t)(W.j0 + r) * nx + ic, G.p[r]);
+    }
+  }
+
+  if (!W.own) return;
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    if (!(W.rows >> r & 1)) continue;
+    const int64_t j = W.j0 + r, o = so + j * nx;
+    (a.p_n + o)[ic] = G.p[r];
+    if (W.i <= nx - 2) (a.vx_n + o)[ic] = G.vx[r];
+    if (j <= nz - 2) (a.vz_n + o)[ic] = G.vz[r];
+    if (xst) (a.xix_n + (int64_t)s * a.sxx + j * (2 * h + 2))[(unsigned)kxi] = G.xix[r];
+    if (pst) (a.psx_n + (int64_t)s * a.spx + j * (2 * h))[(unsigned)kps] = G.psx[r];
+    if (W.xzr >> r & 1) (a.xiz_n + (int64_t)s * a.sxz + (int64_t)zxi(r) * nx)[ic] = G.xiz[r];
+    if (W.kzr >> r & 1) (a.psz_n + (int64_t)s * a.spz + (int64_t)zps(r) * nx)[ic] = G.psz[r];
+  }
 }
 
 // Forward / replay step marching down z.  A block owns a strip of 64*W
@@ -1763,6 +2059,7 @@ class Vd2dEngine final : public Engine {
   void forward(bool save) override {
     SWX_REQUIRE(model_set_, SWX_ESTATE, "swx_set_model must be called before running");
     zero(st_);
+    if (!tz_fwd_ || is_stepn(tz_fwd_)) tz_fwd_ = choose_steps();
     if (!tz_fwd_) {
       const Vd2dArgs<T> a1 = fwd_args(1, 0, save && c_.d.gradient ? 1 : 0, 0, c_.pts.d_traces.as<T>());
       tz_fwd_ = tune("SWX_VD2D_TILE_FWD",
@@ -1771,13 +2068,14 @@ class Vd2dEngine final : public Engine {
     }
     for (int it = 1; it <= ntmax_;) {
       progress("forward step", it, ntmax_);
-      // a two-step launch never steps over a checkpoint or snapshot level
-      const int n = steps_per_launch(tz_fwd_) == 2 && it % S_ != 0 && it + 1 <= ntmax_ && c_.snap_every == 0 ? 2
-                                                                                                             : 1;
+      // a launch of several steps never steps over a checkpoint or snapshot level
+      int n = std::min(steps_per_launch(tz_fwd_), ntmax_ - it + 1);
+      if (save && nck_ > 0) n = std::min(n, S_ - (it - 1) % S_);
+      if (c_.snap_every > 0) n = std::min(n, c_.snap_every - (it - 1) % c_.snap_every);
       fwd_step(it, n, 0, save && c_.d.gradient ? 1 : 0, 0, c_.pts.d_traces.as<T>());
-      if (n == 1) take_snapshots(c_, *this, it);
       it += n;
       const int last = it - 1;
+      take_snapshots(c_, *this, last);
       if (save && last % S_ == 0) {
         const int k = last / S_;
         if (k >= 1 && k <= nck_) ckpt_copy(k, last, true);
@@ -1815,7 +2113,7 @@ class Vd2dEngine final : public Engine {
                                                        c_.pts.d_nt.as<int>(), act);
         SWX_HIP(hipGetLastError());
         for (int it = cb + 1; it <= cb + S_ - 1;) {
-          const int n = steps_per_launch(tz_fwd_) == 2 && it + 1 <= cb + S_ - 1 ? 2 : 1;
+          const int n = std::min(steps_per_launch(tz_fwd_), cb + S_ - it);
           fwd_step(it, n, act, 2, cb, nullptr);
           it += n;
         }
@@ -1886,7 +2184,8 @@ class Vd2dEngine final : public Engine {
   // read level it-1 and write level it into the other buffer; a two-step
   // launch also writes into the other buffer, so it toggles flip_.
   int slot(int k) const { return ((k % 2) + 2 + flip_) % 2; }
-  static int steps_per_launch(int code) { return code >= 200 && code < 300 ? 2 : 1; }
+  static bool is_stepn(int code) { return code > 500 && code < 600; }
+  static int steps_per_launch(int code) { return is_stepn(code) ? code - 500 : code >= 200 && code < 300 ? 2 : 1; }
   // a 2-D tile code and its shot-group codes (code + 1000 k, groups of 2^k
   // shots, k = 1..3) whose group divides the batch
   std::vector<int> with_groups(int code) const {
@@ -1990,6 +2289,18 @@ class Vd2dEngine final : public Engine {
     }
     SWX_HIP(hipGetLastError());
   }
+  static constexpr int NR = 4, NWV = sizeof(T) == 4 ? 16 : 8;   // rows per wave, waves per block of vd2d_stepn_kernel
+  static constexpr int NMAX = std::min(SN_MAX, (NR * NWV - 1) / 6);          // most levels of a window
+  int64_t stepn_blocks(int n) const {
+    return std::max<int64_t>(ceil_div(nx_ - 6 * n, TX - 6 * n), 1) *
+           std::max<int64_t>(ceil_div(nz_ - 6 * n, NR * NWV - 6 * n), 1) * nsh_;
+  }
+  void launch_stepn(Vd2dArgs<T> a, int n) {
+    a.nbx = (int)std::max<int64_t>(ceil_div(nx_ - 6 * n, TX - 6 * n), 1);
+    a.nbz = (int)std::max<int64_t>(ceil_div(nz_ - 6 * n, NR * NWV - 6 * n), 1);
+    vd2d_stepn_kernel<T, NR, NWV><<<(unsigned)stepn_blocks(n), TX * NWV, 0, c_.stream>>>(a, n);
+    SWX_HIP(hipGetLastError());
+  }
   void launch_adj(Vd2dArgs<T> a, int tz) {
     a.sgrp = 1 << (tz / 1000);
     tz %= 1000;
@@ -2036,18 +2347,18 @@ class Vd2dEngine final : public Engine {
     return a;
   }
 
-  // n = 2: steps it and it+1 in one launch (two-step kernel variants)
+  // steps it .. it+n-1 in one launch
   void fwd_step(int it, int n, int act_min, int smode, int cbase, T *traces) {
     const Vd2dArgs<T> a = fwd_args(it, act_min, smode, cbase, traces);
     c_.ktimer.begin(c_.stream);
-    if (n == 2) {
-      launch_fwd(a, tz_fwd_);
-      flip_ ^= 1;
+    if (is_stepn(tz_fwd_)) {
+      launch_stepn(a, n);
     } else {
       // the last step before a checkpoint (or of a replay) runs the
       // single-step kernel of the same tile height
-      launch_fwd(a, steps_per_launch(tz_fwd_) == 2 ? tz_fwd_ - 200 : tz_fwd_);
+      launch_fwd(a, steps_per_launch(tz_fwd_) == 2 && n == 1 ? tz_fwd_ - 200 : tz_fwd_);
     }
+    if (n % 2 == 0) flip_ ^= 1;
     c_.ktimer.end(c_.stream, 0);
   }
 
@@ -2056,6 +2367,33 @@ class Vd2dEngine final : public Engine {
     c_.ktimer.begin(c_.stream);
     launch_adj(a, tz_adj_);
     c_.ktimer.end(c_.stream, 1);
+  }
+
+  // Levels per launch (code 500 + levels), or 0: one, with a tuned tile.  A
+  // launch of few windows costs a level's latency whatever their number, up to
+  // one block per CU, so that the most levels whose windows still number at
+  // most 256 are the best; beyond, 3 (float32) or 3 and then 2 (float64: windows
+  // of half the height) balance the launches against the windows' halos, and
+  // large float64 grids gain nothing.  us per level, best tile / 2 / 3 / 4 / 5 / 6
+  // levels:
+  //   f32  300 x 200, 4 shots     9.9 / 6.7 / 5.2 / 4.5 / 3.9 / 3.7
+  //   f32  701 x 403              9.7 / 6.6 / 5.1 / 4.4 / 3.8 / -
+  //   f32  401 x 301, 8 shots      15 /  11 / 9.2 / 9.7 / 9.3 / 13
+  //   f32  1000 x 700, 8 shots     49 /  40 /  38 /  41 /  49 / 62
+  //   f32  2000 x 800, 32 shots   349 / 354 / 315 / 344 / 401 / 530
+  //   f64  331 x 257              9.6 / 7.0 / 5.5 / 4.6 / 12
+  //   f64  331 x 257, 8 shots    17.4 / 15.5 / 14.5 / 21 / 70
+  //   f64  1000 x 1000           21.1 / 17.5 / 20.3 / 30 / 110
+  //   f64  1000 x 700, 8 shots     88 /  89 /  97 / 150
+  int choose_steps() const {
+    if (const char *v = std::getenv("SWX_VD2D_TILE_FWD")) {
+      const int t = std::atoi(v);
+      return t > 500 && t <= 500 + NMAX ? t : 0;
+    }
+    for (int n = sizeof(T) == 4 ? 6 : 4; n > 3; n--)
+      if (stepn_blocks(n) <= 256) return 500 + n;
+    if (sizeof(T) == 4 || stepn_blocks(3) <= 1024) return 503;
+    return stepn_blocks(2) <= 3072 ? 502 : 0;
   }
 
   // Tuner candidates: the 2-D tile heights 8/16/32 as an interior-tile launch
