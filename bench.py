@@ -332,14 +332,22 @@ def alg_bytes(physics, n, halo, e, nts, S, variant=(0, 0)):
         if physics == "vd2d" and 500 < variant[0] % 1000 < 600:
             # n levels per launch: a launch reads p, vx, vz, m0, m1x, m1z and
             # writes p, vx, vz once (9e); + w p-history (1e) per stored step.
-            # Launches end at multiples of S; an adjoint step as below.
-            lv = variant[0] - 500
-            nl = sum(-(-(min((k + 1) * S, nt) - k * S) // lv) for k in range(-(-nt // S)))
-            nl += (nt // S) * -(-(S - 1) // lv)
+            # An adjoint launch also reads and writes the gradients (6e) and
+            # reads one history level per level (1e).  Launches end at
+            # multiples of S.
+            def launches(lv):
+                return sum(-(-(min((k + 1) * S, nt) - k * S) // lv) for k in range(-(-nt // S)))
+
+            nl = launches(variant[0] - 500) + (nt // S) * -(-(S - 1) // (variant[0] - 500))
             fwd_b += nl * (9 * e * N + strip) + (last + rep) * e * N
             fwd_n += nl
-            adj_b += nt * (14 if vd_groups[1] > 1 else 17) * e * N + nt * strip
-            adj_n += nt
+            if 500 < variant[1] < 600:
+                la = launches(variant[1] - 500)
+                adj_b += la * (15 * e * N + strip) + nt * e * N
+                adj_n += la
+            else:
+                adj_b += nt * (14 if vd_groups[1] > 1 else 17) * e * N + nt * strip
+                adj_n += nt
             continue
         if physics == "vd2d" and (vd_groups[0] > 1 or vd_groups[1] > 1):
             # two shots per block (4xx) or shot groups in the block order
@@ -440,7 +448,7 @@ def kernel_names(physics, variant):
         def name(kind, v):
             v %= 1000      # the thousands give the shot groups of the block order
             if v > 500:    # several levels per launch
-                return f"vd2d_stepn_kernel<float, 4, 16> ({v - 500} levels per launch)"
+                return f"vd2d_stepn_kernel<float, 4, 16, {'true' if kind == 'adj' else 'false'}> ({v - 500} levels per launch)"
             if v >= 400:   # two shots per block, one launch
                 return f"vd2d_{kind}_pair_kernel<float, {v - 400}>"
             if v >= 300:   # interior and other tiles in one launch

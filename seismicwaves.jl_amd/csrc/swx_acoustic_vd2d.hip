@@ -852,7 +852,7 @@ __global__ __launch_bounds__(NB) void vd2d_fwd2_kernel(Vd2dArgs<T> a) {
 }
 
 // ---------------------------------------------------------------------------
-// Several forward / replay levels per launch (vd2d_stepn_kernel).
+// Several levels per launch (vd2d_stepn_kernel).
 //
 // A block of NW waves holds a 64 x (NW R) window of pressure, velocities and
 // model factors in registers (lane = column, R rows per wave) and steps it n
@@ -870,7 +870,9 @@ __global__ __launch_bounds__(NB) void vd2d_fwd2_kernel(Vd2dArgs<T> a) {
 // Bound by latency on small grids (701 x 403 float32: 19 us for 5 levels, 9.7 us
 // for one of the tile steps) and by instruction issue on large ones, where the
 // windows step 1.9 (3 levels) times the owned cells (1000 x 700, 8 shots
-// float32: 49 -> 38 us per level; 2000 x 800, 32 shots: 349 -> 315).
+// float32: 49 -> 38 us per level; 2000 x 800, 32 shots: 349 -> 315).  The adjoint
+// keeps the three gradients of its cells in registers too and reads one
+// history level per level: 701 x 403 10.9 -> 4.9 us, 2000 x 800, 32 shots 585 -> 538.
 template <typename T, int R, int NW>
 struct Vd2dNLds : LevelPoints<T, NW * R> {
   T vz[3][NW][TX];             // rows R-2, R-1 and 0 of vz
@@ -954,8 +956,36 @@ __device__ __forceinline__ void vd2d_n_velocity(const Vd2dArgs<T> &a, const Vd2d
   }
 }
 
-template <typename T, int R, int NW>
-__global__ __launch_bounds__(NW *TX, sizeof(T) == 4 ? 4 : 2) void vd2d_stepn_kernel(Vd2dArgs<T> a, int n) {
+// Correlation of one adjoint level (correlate_gradient_xPU.jl:12-21,
+// acoustic2D_VD_xPU.jl:180-198): cur, prev: the replayed pressure of the level
+// and the one before, rows from the one before the thread's to two after.
+// EDGE: the window or the rows reach a side of the grid.
+template <typename T, int R, bool EDGE>
+__device__ __forceinline__ void vd2d_n_correlate(const Vd2dArgs<T> &a, const LevelWin &W, const T *cur, const T *prev,
+                                                 const Vd2dNRegs<T, R> &G, T *g0, T *g1x, T *g1z) {
+  T c[R + 3];
+#pragma unroll
+  for (int q = 0; q < R + 3; q++) {
+    const int j = W.j0 - 1 + q;
+    c[q] = EDGE && (W.i > a.nx - 1 || j < 0 || j > a.nz - 1) ? T(0) : cur[q];
+  }
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    const T pcv = c[r + 1];
+    g0[r] = g0[r] - (G.p[r] * (pcv - prev[r + 1]) * a.idt);
+    const T p1 = lane_after(pcv);
+    const T dpx = d4(lane_before(pcv), pcv, p1, lane_after(p1)) * a.idx;
+    g1x[r] = g1x[r] + G.vx[r] * dpx;
+    const T dpz = d4(c[r], pcv, c[r + 2], c[r + 3]) * a.idz;
+    g1z[r] = g1z[r] + G.vz[r] * dpz;
+  }
+}
+
+// Forward / replay levels it .. it+n-1, or (ADJ) adjoint levels it .. it-n+1:
+// velocities from the old pressure, then the pressure, residual injection and
+// the correlation with the replayed pressure, which is loaded a level ahead.
+template <typename T, int R, int NW, bool ADJ>
+__global__ __launch_bounds__(NW *TX, sizeof(T) == 4 ? NW / 4 : 2) void vd2d_stepn_kernel(Vd2dArgs<T> a, int n) {
   __shared__ Vd2dNLds<T, R, NW> L;
   constexpr int H = NW * R;
   if (threadIdx.x == 0) L.used = L.rused = 0;
@@ -1032,10 +1062,31 @@ __global__ __launch_bounds__(NW *TX, sizeof(T) == 4 ? 4 : 2) void vd2d_stepn_ker
       if (W.kzr >> r & 1) G.psz[r] = (a.psz_o + (int64_t)s * a.spz + (int64_t)zps(r) * nx)[ic];
     }
   }
-  // Levels of this shot: up to nts.  Tested after the loads above were issued,
-  // so that they do not wait for nts.
-  const int nl = min(n, nts - a.it + 1);
+  T g0[ADJ ? R : 1], g1x[ADJ ? R : 1], g1z[ADJ ? R : 1];
+  if constexpr (ADJ) {
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      g0[r] = row(a.g0 + so, r)[ic];
+      g1x[r] = row(a.g1x + so, r)[ic];
+      g1z[r] = row(a.g1z + so, r)[ic];
+    }
+  }
+  // Levels of this shot: a forward one ends at nts, an adjoint one starts there
+  // (from zero fields).  Tested after the loads above were issued, so that
+  // they do not wait for nts.
+  const int la = ADJ ? min(a.it, nts) : a.it;
+  const int nl = ADJ ? la - (a.it - n) : min(n, nts - a.it + 1);
   if (nl <= 0 || nts <= a.act_min) return;
+  T d0[ADJ ? R + 3 : 1], d1[ADJ ? R + 3 : 1];      // replayed pressure of a level, rows j0-1 .. j0+R+1
+  auto fetch = [&](T *d, int l) {
+    const T *slot = a.pbuf + (int64_t)(max(l, a.cbase) - a.cbase) * a.pslot + so;
+#pragma unroll
+    for (int q = 0; q < R + 3; q++) d[q] = (slot + (int64_t)min(max(W.j0 - 1 + q, 0), nz - 1) * nx)[ic];
+  };
+  if constexpr (ADJ) {
+    fetch(d0, la);
+    fetch(d1, la - 1);
+  }
   if (xs || zs) {
 #pragma unroll
     for (int r = 0; r < R; r++) {
@@ -1046,7 +1097,7 @@ __global__ __launch_bounds__(NW *TX, sizeof(T) == 4 ? 4 : 2) void vd2d_stepn_ker
     }
   }
   const int64_t otr = a.pt.off_tr[s];     // (here: a load in the level loop would wait for the wave's stores)
-  level_points<T, R, false>(a, L, W, s, nts, X0, a.it, nl);
+  level_points<T, R, ADJ>(a, L, W, s, nts, X0, la, nl);
   if (threadIdx.x < H) {
     const int j = Z0 + (int)threadIdx.x;
     const AxisCoef<T> cz = axis_coef(a.cpml + (int64_t)s * a.cstride, h, 1);
@@ -1058,62 +1109,25 @@ __global__ __launch_bounds__(NW *TX, sizeof(T) == 4 ? 4 : 2) void vd2d_stepn_ker
     q[2] = v ? cz.bh(kv) : T(0);
     q[3] = v ? cz.ah(kv) : T(0);
   }
-  const int seg0 = store_base(a.smode, 1 << 30, nts, a.S, a.cbase);    // level l > seg0 >= 0 goes to slot l - seg0
+  // level l > seg0 >= 0 goes to slot l - seg0
+  const int seg0 = ADJ ? -1 : store_base(a.smode, 1 << 30, nts, a.S, a.cbase);
 
-#pragma clang loop unroll(disable)
-  for (int m = 0; m < nl; m++) {
-    opaque(W.j0);
-    opaque(W.rows);
-    opaque(W.jin);
-    opaque(W.kzr);
-    opaque(W.xzr);
-    opaque(W.jg);
-    opaque(W.jv);
-    opaque(W.imask);
-    opaque(W.rmask);
-    const int l = a.it + m;
+  auto pressure = [&] {
     const int wu = W.w > 0 ? W.w - 1 : 0, wd = W.w < NW - 1 ? W.w + 1 : NW - 1;
     L.vz[0][W.w][W.lane] = G.vz[R - 2];
     L.vz[1][W.w][W.lane] = G.vz[R - 1];
     L.vz[2][W.w][W.lane] = G.vz[0];
     __syncthreads();
-    {
-      // (beyond the window: zero, what the grid's own sides need)
-      T vu2 = L.vz[0][wu][W.lane], vu1 = L.vz[1][wu][W.lane], vd = L.vz[2][wd][W.lane];
-      if (W.w == 0) vu2 = vu1 = T(0);
-      if (W.w == NW - 1) vd = T(0);
-      if (seg0 >= 0 && a.smode == 1 && l == seg0 + 1 && W.own) {
-#pragma unroll
-        for (int r = 0; r < R; r++)
-          if (W.rows >> r & 1) (a.pbuf + so + (int64_t)(W.j0 + r) * nx)[ic] = G.p[r];
-      }
-      if (xs) vd2d_n_pressure<T, R, NW, true, true>(a, L, W, xst, xc, vu2, vu1, vd, G);
-      else if (zs) vd2d_n_pressure<T, R, NW, false, true>(a, L, W, xst, xc, vu2, vu1, vd, G);
-      else vd2d_n_pressure<T, R, NW, false, false>(a, L, W, xst, xc, vu2, vu1, vd, G);
-    }
-    if (W.imask | W.rmask) {
-#pragma unroll
-      for (int r = 0; r < R; r++) {
-        if (W.imask >> r & 1) {
-          T inj = 0;
-          level_inject<T, R, false>(a, L, W, s, nts, r, m, l, T(0), G.p[r], inj);
-        }
-        if ((W.rmask & W.rows) >> r & 1 && W.own) {
-          const int e = L.rec[W.w * R + r][W.lane];
-          T *tr = a.traces + otr + (l - 1);
-          if (e > 0) {
-#pragma clang loop unroll(disable)
-            for (int k = 0; k < e >> 8; k++) tr[(int64_t)nts * L.col[(e & 255) - 1 + k]] = G.p[r];
-          } else if (e < 0) {
-            const int j = W.j0 + r;
-            const int u = find_point(a.pt.rrow, a.pt.urec_cell, a.pt.nrows, s, j, (int64_t)j * nx + W.i);
-#pragma clang loop unroll(disable)
-            for (int k = a.pt.urec_ptr[u]; k < a.pt.urec_ptr[u + 1]; k++)
-              tr[(int64_t)nts * a.pt.urec_list[k]] = G.p[r];
-          }
-        }
-      }
-    }
+    // (beyond the window: zero, what the grid's own sides need)
+    T vu2 = L.vz[0][wu][W.lane], vu1 = L.vz[1][wu][W.lane], vd = L.vz[2][wd][W.lane];
+    if (W.w == 0) vu2 = vu1 = T(0);
+    if (W.w == NW - 1) vd = T(0);
+    if (xs) vd2d_n_pressure<T, R, NW, true, true>(a, L, W, xst, xc, vu2, vu1, vd, G);
+    else if (zs) vd2d_n_pressure<T, R, NW, false, true>(a, L, W, xst, xc, vu2, vu1, vd, G);
+    else vd2d_n_pressure<T, R, NW, false, false>(a, L, W, xst, xc, vu2, vu1, vd, G);
+  };
+  auto velocity = [&] {
+    const int wu = W.w > 0 ? W.w - 1 : 0, wd = W.w < NW - 1 ? W.w + 1 : NW - 1;
     L.p[0][W.w][W.lane] = G.p[R - 1];
     L.p[1][W.w][W.lane] = G.p[0];
     L.p[2][W.w][W.lane] = G.p[1];
@@ -1124,11 +1138,77 @@ __global__ __launch_bounds__(NW *TX, sizeof(T) == 4 ? 4 : 2) void vd2d_stepn_ker
     if (xs) vd2d_n_velocity<T, R, NW, true, true>(a, L, W, pst, xc, pu, pd1, pd2, G);
     else if (zs) vd2d_n_velocity<T, R, NW, false, true>(a, L, W, pst, xc, pu, pd1, pd2, G);
     else vd2d_n_velocity<T, R, NW, false, false>(a, L, W, pst, xc, pu, pd1, pd2, G);
-    if (seg0 >= 0 && l > seg0 && W.own) {
-      T *hs = a.pbuf + (int64_t)(l - seg0) * a.pslot + so;
+  };
+  // injection and (forward) recording of level l, number m
+  auto points = [&](int m, int l) {
+    if (!(W.imask | W.rmask)) return;
 #pragma unroll
-      for (int r = 0; r < R; r++)
-        if (W.rows >> r & 1) st_nt(hs + (int64_t)(W.j0 + r) * nx + ic, G.p[r]);
+    for (int r = 0; r < R; r++) {
+      if (W.imask >> r & 1) {
+        T inj = 0;
+        level_inject<T, R, ADJ>(a, L, W, s, nts, r, m, l, G.m0[r], G.p[r], inj);
+      }
+      if (!ADJ && (W.rmask & W.rows) >> r & 1 && W.own) {
+        const int e = L.rec[W.w * R + r][W.lane];
+        T *tr = a.traces + otr + (l - 1);
+        if (e > 0) {
+#pragma clang loop unroll(disable)
+          for (int k = 0; k < e >> 8; k++) tr[(int64_t)nts * L.col[(e & 255) - 1 + k]] = G.p[r];
+        } else if (e < 0) {
+          const int j = W.j0 + r;
+          const int u = find_point(a.pt.rrow, a.pt.urec_cell, a.pt.nrows, s, j, (int64_t)j * nx + W.i);
+#pragma clang loop unroll(disable)
+          for (int k = a.pt.urec_ptr[u]; k < a.pt.urec_ptr[u + 1]; k++)
+            tr[(int64_t)nts * a.pt.urec_list[k]] = G.p[r];
+        }
+      }
+    }
+  };
+  auto fresh = [&] {
+    opaque(W.j0);
+    opaque(W.rows);
+    opaque(W.jin);
+    opaque(W.kzr);
+    opaque(W.xzr);
+    opaque(W.jg);
+    opaque(W.jv);
+    opaque(W.imask);
+    opaque(W.rmask);
+  };
+  if constexpr (ADJ) {
+    auto level = [&](int m, T *cur, const T *prev) {
+      fresh();
+      velocity();
+      pressure();
+      points(m, la - m);
+      if (xs || zs) vd2d_n_correlate<T, R, true>(a, W, cur, prev, G, g0, g1x, g1z);
+      else vd2d_n_correlate<T, R, false>(a, W, cur, prev, G, g0, g1x, g1z);
+      fetch(cur, la - m - 2);
+    };
+#pragma clang loop unroll(disable)
+    for (int m = 0; m < nl; m += 2) {
+      level(m, d0, d1);
+      if (m + 1 < nl) level(m + 1, d1, d0);
+    }
+  } else {
+#pragma clang loop unroll(disable)
+    for (int m = 0; m < nl; m++) {
+      fresh();
+      const int l = a.it + m;
+      if (seg0 >= 0 && a.smode == 1 && l == seg0 + 1 && W.own) {
+#pragma unroll
+        for (int r = 0; r < R; r++)
+          if (W.rows >> r & 1) (a.pbuf + so + (int64_t)(W.j0 + r) * nx)[ic] = G.p[r];
+      }
+      pressure();
+      points(m, l);
+      velocity();
+      if (seg0 >= 0 && l > seg0 && W.own) {
+        T *hs = a.pbuf + (int64_t)(l - seg0) * a.pslot + so;
+#pragma unroll
+        for (int r = 0; r < R; r++)
+          if (W.rows >> r & 1) st_nt(hs + (int64_t)(W.j0 + r) * nx + ic, G.p[r]);
+      }
     }
   }
 
@@ -1144,6 +1224,11 @@ __global__ __launch_bounds__(NW *TX, sizeof(T) == 4 ? 4 : 2) void vd2d_stepn_ker
     if (pst) (a.psx_n + (int64_t)s * a.spx + j * (2 * h))[(unsigned)kps] = G.psx[r];
     if (W.xzr >> r & 1) (a.xiz_n + (int64_t)s * a.sxz + (int64_t)zxi(r) * nx)[ic] = G.xiz[r];
     if (W.kzr >> r & 1) (a.psz_n + (int64_t)s * a.spz + (int64_t)zps(r) * nx)[ic] = G.psz[r];
+    if constexpr (ADJ) {
+      (a.g0 + o)[ic] = g0[r];
+      if (W.i <= nx - 2) (a.g1x + o)[ic] = g1x[r];
+      if (j <= nz - 2) (a.g1z + o)[ic] = g1z[r];
+    }
   }
 }
 
@@ -2059,7 +2144,7 @@ class Vd2dEngine final : public Engine {
   void forward(bool save) override {
     SWX_REQUIRE(model_set_, SWX_ESTATE, "swx_set_model must be called before running");
     zero(st_);
-    if (!tz_fwd_ || is_stepn(tz_fwd_)) tz_fwd_ = choose_steps();
+    if (!tz_fwd_ || is_stepn(tz_fwd_)) tz_fwd_ = choose_steps("SWX_VD2D_TILE_FWD");
     if (!tz_fwd_) {
       const Vd2dArgs<T> a1 = fwd_args(1, 0, save && c_.d.gradient ? 1 : 0, 0, c_.pts.d_traces.as<T>());
       tz_fwd_ = tune("SWX_VD2D_TILE_FWD",
@@ -2085,6 +2170,7 @@ class Vd2dEngine final : public Engine {
 
   void adjoint(bool per_shot) override {
     const int Kmax = (int)ceil_div(ntmax_, S_);
+    if (!tz_adj_ || is_stepn(tz_adj_)) tz_adj_ = choose_steps("SWX_VD2D_TILE_ADJ");
     if (!tz_adj_) {
       // timed on a step every shot takes part in (the shortest shot's last
       // step); the history slots it reads are in range, their contents do
@@ -2123,7 +2209,11 @@ class Vd2dEngine final : public Engine {
         SWX_HIP(hipGetLastError());
       }
       const int top = std::min(cb + S_, ntmax_);
-      for (int it = top; it >= cb + 1; it--) adj_step(it, cb);
+      for (int it = top; it >= cb + 1;) {
+        const int n = is_stepn(tz_adj_) ? std::min(steps_per_launch(tz_adj_), it - cb) : 1;
+        adj_step(it, n, cb);
+        it -= n;
+      }
     }
     dim3 g((unsigned)std::min<int64_t>(ceil_div(N_, 256), 4096));
     for (int f = 0; f < 3; f++)
@@ -2177,7 +2267,7 @@ class Vd2dEngine final : public Engine {
 
   void zero(DevBuf *b) {
     for (int k = 0; k < 3; k++) SWX_HIP(hipMemsetAsync(b[k].get(), 0, b[k].bytes(), c_.stream));
-    if (b == st_) flip_ = 0;
+    (b == st_ ? flip_ : aflip_) = 0;
   }
 
   // Forward state buffer (0/1) holding time level k.  Single-step launches
@@ -2295,10 +2385,11 @@ class Vd2dEngine final : public Engine {
     return std::max<int64_t>(ceil_div(nx_ - 6 * n, TX - 6 * n), 1) *
            std::max<int64_t>(ceil_div(nz_ - 6 * n, NR * NWV - 6 * n), 1) * nsh_;
   }
-  void launch_stepn(Vd2dArgs<T> a, int n) {
+  void launch_stepn(Vd2dArgs<T> a, int n, bool adj) {
     a.nbx = (int)std::max<int64_t>(ceil_div(nx_ - 6 * n, TX - 6 * n), 1);
     a.nbz = (int)std::max<int64_t>(ceil_div(nz_ - 6 * n, NR * NWV - 6 * n), 1);
-    vd2d_stepn_kernel<T, NR, NWV><<<(unsigned)stepn_blocks(n), TX * NWV, 0, c_.stream>>>(a, n);
+    if (adj) vd2d_stepn_kernel<T, NR, NWV, true><<<(unsigned)stepn_blocks(n), TX * NWV, 0, c_.stream>>>(a, n);
+    else vd2d_stepn_kernel<T, NR, NWV, false><<<(unsigned)stepn_blocks(n), TX * NWV, 0, c_.stream>>>(a, n);
     SWX_HIP(hipGetLastError());
   }
   void launch_adj(Vd2dArgs<T> a, int tz) {
@@ -2342,7 +2433,7 @@ class Vd2dEngine final : public Engine {
     return a;
   }
   Vd2dArgs<T> adj_args(int it, int cbase) const {
-    Vd2dArgs<T> a = args(ad_, it, (it + 1) & 1, it & 1);
+    Vd2dArgs<T> a = args(ad_, it, (it + 1 + aflip_) & 1, (it + aflip_) & 1);
     a.cbase = cbase;
     return a;
   }
@@ -2352,7 +2443,7 @@ class Vd2dEngine final : public Engine {
     const Vd2dArgs<T> a = fwd_args(it, act_min, smode, cbase, traces);
     c_.ktimer.begin(c_.stream);
     if (is_stepn(tz_fwd_)) {
-      launch_stepn(a, n);
+      launch_stepn(a, n, false);
     } else {
       // the last step before a checkpoint (or of a replay) runs the
       // single-step kernel of the same tile height
@@ -2362,10 +2453,13 @@ class Vd2dEngine final : public Engine {
     c_.ktimer.end(c_.stream, 0);
   }
 
-  void adj_step(int it, int cbase) {
+  // adjoint steps it .. it-n+1 in one launch
+  void adj_step(int it, int n, int cbase) {
     const Vd2dArgs<T> a = adj_args(it, cbase);
     c_.ktimer.begin(c_.stream);
-    launch_adj(a, tz_adj_);
+    if (is_stepn(tz_adj_)) launch_stepn(a, n, true);
+    else launch_adj(a, tz_adj_);
+    if (n % 2 == 0) aflip_ ^= 1;
     c_.ktimer.end(c_.stream, 1);
   }
 
@@ -2385,8 +2479,16 @@ class Vd2dEngine final : public Engine {
   //   f64  331 x 257, 8 shots    17.4 / 15.5 / 14.5 / 21 / 70
   //   f64  1000 x 1000           21.1 / 17.5 / 20.3 / 30 / 110
   //   f64  1000 x 700, 8 shots     88 /  89 /  97 / 150
-  int choose_steps() const {
-    if (const char *v = std::getenv("SWX_VD2D_TILE_FWD")) {
+  // and of the adjoint with its replay:
+  //   f32  300 x 200, 4 shots    15.9 / 12.2 / 10.3 / 9.2 / 8.6 / 8.4
+  //   f32  701 x 403             15.8 / 12.1 / 10.2 / 9.3 / 8.9
+  //   f32  1000 x 700, 8 shots    111 / 112 / 103 / 103 / 110 / 126
+  //   f32  2000 x 800, 32 shots   901 / 933 / 854 / 853 / 910
+  //   f64  331 x 257             17.2 / 11.8 / 10.0 / 9.2 / 19
+  //   f64  1000 x 1000             50 /  41 /  44 /  56
+  //   f64  1000 x 700, 8 shots    214 / 211 / 219 / 285
+  int choose_steps(const char *env) const {
+    if (const char *v = std::getenv(env)) {
       const int t = std::atoi(v);
       return t > 500 && t <= 500 + NMAX ? t : 0;
     }
@@ -2466,7 +2568,7 @@ class Vd2dEngine final : public Engine {
     return best;
   }
   int tz_fwd_ = 0, tz_adj_ = 0;
-  int flip_ = 0;
+  int flip_ = 0, aflip_ = 0;
 
   // checkpoint k (k = 1 .. floor(nt_max/S), all shots): p, vx, vz, psi_x,
   // psi_z, xi_x, xi_z at parity cb&1
