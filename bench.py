@@ -338,11 +338,11 @@ def alg_bytes(physics, n, halo, e, nts, S, variant=(0, 0)):
             def launches(lv):
                 return sum(-(-(min((k + 1) * S, nt) - k * S) // lv) for k in range(-(-nt // S)))
 
-            nl = launches(variant[0] - 500) + (nt // S) * -(-(S - 1) // (variant[0] - 500))
+            nl = launches(variant[0] % 10) + (nt // S) * -(-(S - 1) // (variant[0] % 10))
             fwd_b += nl * (9 * e * N + strip) + (last + rep) * e * N
             fwd_n += nl
             if 500 < variant[1] < 600:
-                la = launches(variant[1] - 500)
+                la = launches(variant[1] % 10)
                 adj_b += la * (15 * e * N + strip) + nt * e * N
                 adj_n += la
             else:
@@ -448,7 +448,8 @@ def kernel_names(physics, variant):
         def name(kind, v):
             v %= 1000      # the thousands give the shot groups of the block order
             if v > 500:    # several levels per launch
-                return f"vd2d_stepn_kernel<float, 4, 16, {'true' if kind == 'adj' else 'false'}> ({v - 500} levels per launch)"
+                shape = "8, 8, true" if kind == "adj" else "6, 16, false" if v > 510 else "4, 16, false"
+                return f"vd2d_stepn_kernel<float, {shape}> ({v % 10} levels per launch)"
             if v >= 400:   # two shots per block, one launch
                 return f"vd2d_{kind}_pair_kernel<float, {v - 400}>"
             if v >= 300:   # interior and other tiles in one launch

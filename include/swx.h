@@ -156,8 +156,8 @@ typedef struct {
   int64_t n_kernel[2];
   /* Launch shapes the plan's autotuner chose (or the environment pinned):
    * VD [forward, adjoint] tile codes (8/16/32 interior + other launches,
-   * 308/316/332 one launch, 102/104 z-marching strips, 500 + n: n levels per
-   * launch; + 1000 k: shots in groups of 2^k in the block order); elastic [forward, adjoint] variant
+   * 308/316/332 one launch, 102/104 z-marching strips, 500 + n and 510 + n: n
+   * levels per launch; + 1000 k: shots in groups of 2^k in the block order); elastic [forward, adjoint] variant
    * codes (0/1 stress and displacement launches, 2 one fused launch, 3 row
    * march); CD 2D
    * [window shapes (or, with one level per launch, rows per thread), most

@@ -869,10 +869,11 @@ __global__ __launch_bounds__(NB) void vd2d_fwd2_kernel(Vd2dArgs<T> a) {
 //
 // Bound by latency on small grids (701 x 403 float32: 19 us for 5 levels, 9.7 us
 // for one of the tile steps) and by instruction issue on large ones, where the
-// windows step 1.9 (3 levels) times the owned cells (1000 x 700, 8 shots
-// float32: 49 -> 38 us per level; 2000 x 800, 32 shots: 349 -> 315).  The adjoint
-// keeps the three gradients of its cells in registers too and reads one
-// history level per level: 701 x 403 10.9 -> 4.9 us, 2000 x 800, 32 shots 585 -> 538.
+// windows step 1.7 (6 x 16 rows, 4 levels: 2.1) times the owned cells: 1000 x
+// 700, 8 shots float32 49 -> 33 us per level; 2000 x 800, 32 shots 349 -> 270.
+// The adjoint keeps the three gradients of its cells in registers too and
+// reads one history level per level: 701 x 403 10.9 -> 5.1 us, 2000 x 800, 32
+// shots 585 -> 530 (8 x 8 rows; 601 with 4 x 16, where six registers spill).
 template <typename T, int R, int NW>
 struct Vd2dNLds : LevelPoints<T, NW * R> {
   T vz[3][NW][TX];             // rows R-2, R-1 and 0 of vz
@@ -985,7 +986,7 @@ __device__ __forceinline__ void vd2d_n_correlate(const Vd2dArgs<T> &a, const Lev
 // velocities from the old pressure, then the pressure, residual injection and
 // the correlation with the replayed pressure, which is loaded a level ahead.
 template <typename T, int R, int NW, bool ADJ>
-__global__ __launch_bounds__(NW *TX, sizeof(T) == 4 ? NW / 4 : 2) void vd2d_stepn_kernel(Vd2dArgs<T> a, int n) {
+__global__ __launch_bounds__(NW *TX, NW / 4) void vd2d_stepn_kernel(Vd2dArgs<T> a, int n) {
   __shared__ Vd2dNLds<T, R, NW> L;
   constexpr int H = NW * R;
   if (threadIdx.x == 0) L.used = L.rused = 0;
@@ -2144,7 +2145,7 @@ class Vd2dEngine final : public Engine {
   void forward(bool save) override {
     SWX_REQUIRE(model_set_, SWX_ESTATE, "swx_set_model must be called before running");
     zero(st_);
-    if (!tz_fwd_ || is_stepn(tz_fwd_)) tz_fwd_ = choose_steps("SWX_VD2D_TILE_FWD");
+    if (!tz_fwd_ || is_stepn(tz_fwd_)) tz_fwd_ = choose_steps("SWX_VD2D_TILE_FWD", false);
     if (!tz_fwd_) {
       const Vd2dArgs<T> a1 = fwd_args(1, 0, save && c_.d.gradient ? 1 : 0, 0, c_.pts.d_traces.as<T>());
       tz_fwd_ = tune("SWX_VD2D_TILE_FWD",
@@ -2170,7 +2171,7 @@ class Vd2dEngine final : public Engine {
 
   void adjoint(bool per_shot) override {
     const int Kmax = (int)ceil_div(ntmax_, S_);
-    if (!tz_adj_ || is_stepn(tz_adj_)) tz_adj_ = choose_steps("SWX_VD2D_TILE_ADJ");
+    if (!tz_adj_ || is_stepn(tz_adj_)) tz_adj_ = choose_steps("SWX_VD2D_TILE_ADJ", true);
     if (!tz_adj_) {
       // timed on a step every shot takes part in (the shortest shot's last
       // step); the history slots it reads are in range, their contents do
@@ -2275,7 +2276,7 @@ class Vd2dEngine final : public Engine {
   // launch also writes into the other buffer, so it toggles flip_.
   int slot(int k) const { return ((k % 2) + 2 + flip_) % 2; }
   static bool is_stepn(int code) { return code > 500 && code < 600; }
-  static int steps_per_launch(int code) { return is_stepn(code) ? code - 500 : code >= 200 && code < 300 ? 2 : 1; }
+  static int steps_per_launch(int code) { return is_stepn(code) ? code % 10 : code >= 200 && code < 300 ? 2 : 1; }
   // a 2-D tile code and its shot-group codes (code + 1000 k, groups of 2^k
   // shots, k = 1..3) whose group divides the batch
   std::vector<int> with_groups(int code) const {
@@ -2379,18 +2380,31 @@ class Vd2dEngine final : public Engine {
     }
     SWX_HIP(hipGetLastError());
   }
-  static constexpr int NR = 4, NWV = sizeof(T) == 4 ? 16 : 8;   // rows per wave, waves per block of vd2d_stepn_kernel
-  static constexpr int NMAX = std::min(SN_MAX, (NR * NWV - 1) / 6);          // most levels of a window
-  int64_t stepn_blocks(int n) const {
+  // Windows of vd2d_stepn_kernel: rows per wave and waves per block of shape 0
+  // (forward, few windows), 1 (forward, many) and 2 (adjoint), all 64 columns
+  // wide; as high as registers allow for the number of waves.
+  struct Shape {
+    int r, nw;
+  };
+  static constexpr Shape SHAPES[3] = {{4, sizeof(T) == 4 ? 16 : 8}, {6, sizeof(T) == 4 ? 16 : 8},
+                                      {sizeof(T) == 4 ? 8 : 4, 8}};
+  static constexpr int NMAX = std::min(SN_MAX, (SHAPES[0].r * SHAPES[0].nw - 1) / 6);   // most levels of a window
+  int64_t stepn_blocks(int shape, int n) const {
     return std::max<int64_t>(ceil_div(nx_ - 6 * n, TX - 6 * n), 1) *
-           std::max<int64_t>(ceil_div(nz_ - 6 * n, NR * NWV - 6 * n), 1) * nsh_;
+           std::max<int64_t>(ceil_div(nz_ - 6 * n, SHAPES[shape].r * SHAPES[shape].nw - 6 * n), 1) * nsh_;
   }
-  void launch_stepn(Vd2dArgs<T> a, int n, bool adj) {
+  template <int S, bool ADJ>
+  void launch_shape(Vd2dArgs<T> a, int n) {
+    constexpr int R = SHAPES[S].r, NW = SHAPES[S].nw;
     a.nbx = (int)std::max<int64_t>(ceil_div(nx_ - 6 * n, TX - 6 * n), 1);
-    a.nbz = (int)std::max<int64_t>(ceil_div(nz_ - 6 * n, NR * NWV - 6 * n), 1);
-    if (adj) vd2d_stepn_kernel<T, NR, NWV, true><<<(unsigned)stepn_blocks(n), TX * NWV, 0, c_.stream>>>(a, n);
-    else vd2d_stepn_kernel<T, NR, NWV, false><<<(unsigned)stepn_blocks(n), TX * NWV, 0, c_.stream>>>(a, n);
+    a.nbz = (int)std::max<int64_t>(ceil_div(nz_ - 6 * n, R * NW - 6 * n), 1);
+    vd2d_stepn_kernel<T, R, NW, ADJ><<<(unsigned)stepn_blocks(S, n), TX * NW, 0, c_.stream>>>(a, n);
     SWX_HIP(hipGetLastError());
+  }
+  void launch_stepn(const Vd2dArgs<T> &a, int n, bool adj) {
+    if (adj) launch_shape<2, true>(a, n);
+    else if (tz_fwd_ > 510) launch_shape<1, false>(a, n);
+    else launch_shape<0, false>(a, n);
   }
   void launch_adj(Vd2dArgs<T> a, int tz) {
     a.sgrp = 1 << (tz / 1000);
@@ -2463,39 +2477,42 @@ class Vd2dEngine final : public Engine {
     c_.ktimer.end(c_.stream, 1);
   }
 
-  // Levels per launch (code 500 + levels), or 0: one, with a tuned tile.  A
-  // launch of few windows costs a level's latency whatever their number, up to
-  // one block per CU, so that the most levels whose windows still number at
-  // most 256 are the best; beyond, 3 (float32) or 3 and then 2 (float64: windows
-  // of half the height) balance the launches against the windows' halos, and
-  // large float64 grids gain nothing.  us per level, best tile / 2 / 3 / 4 / 5 / 6
-  // levels:
-  //   f32  300 x 200, 4 shots     9.9 / 6.7 / 5.2 / 4.5 / 3.9 / 3.7
-  //   f32  701 x 403              9.7 / 6.6 / 5.1 / 4.4 / 3.8 / -
-  //   f32  401 x 301, 8 shots      15 /  11 / 9.2 / 9.7 / 9.3 / 13
-  //   f32  1000 x 700, 8 shots     49 /  40 /  38 /  41 /  49 / 62
-  //   f32  2000 x 800, 32 shots   349 / 354 / 315 / 344 / 401 / 530
-  //   f64  331 x 257              9.6 / 7.0 / 5.5 / 4.6 / 12
-  //   f64  331 x 257, 8 shots    17.4 / 15.5 / 14.5 / 21 / 70
-  //   f64  1000 x 1000           21.1 / 17.5 / 20.3 / 30 / 110
-  //   f64  1000 x 700, 8 shots     88 /  89 /  97 / 150
-  // and of the adjoint with its replay:
-  //   f32  300 x 200, 4 shots    15.9 / 12.2 / 10.3 / 9.2 / 8.6 / 8.4
-  //   f32  701 x 403             15.8 / 12.1 / 10.2 / 9.3 / 8.9
-  //   f32  1000 x 700, 8 shots    111 / 112 / 103 / 103 / 110 / 126
-  //   f32  2000 x 800, 32 shots   901 / 933 / 854 / 853 / 910
-  //   f64  331 x 257             17.2 / 11.8 / 10.0 / 9.2 / 19
-  //   f64  1000 x 1000             50 /  41 /  44 /  56
-  //   f64  1000 x 700, 8 shots    214 / 211 / 219 / 285
-  int choose_steps(const char *env) const {
+  // Levels per launch (code 500 + levels; 510 + levels: shape 1), or 0: one,
+  // with a tuned tile.  A launch of few windows costs a level's latency whatever
+  // their number, up to one block per CU, so that the most levels whose windows
+  // still number at most 256 are the best.  Beyond, the halos count: the forward
+  // takes the taller windows of shape 1, and 4 levels (float32) or 3 (float64,
+  // half the rows) balance them against the launches; the adjoint, which its
+  // registers hold to the height of shape 0, takes 3, and in float64 2 and at
+  // last single steps.  us per level, forward: best tile / 3 / 4 / 5 / 6 levels /
+  // shape 1 with 3 / 4 / 5:
+  //   f32  300 x 200, 4 shots     9.9 / 5.2 / 4.5 / 3.9 / 3.7 / 6.1 / 5.2 / 4.5
+  //   f32  701 x 403              9.7 / 5.1 / 4.4 / 3.8 /   - / 6.1 / 5.1 / 4.5
+  //   f32  1000 x 1000           14.6 / 8.5 / 9.8 /  11 /   - /  10 / 8.6 / 8.0
+  //   f32  800 x 600, 3 shots    18.1 /  12 /  13 /   - /   - /  11 / 9.9 /  11
+  //   f32  1000 x 700, 8 shots     49 /  38 /  41 /  49 /   - /  33 /  33 /  36
+  //   f32  2000 x 800, 32 shots   349 / 315 / 344 / 401 / 530 / 296 / 270 / 291
+  //   f64  331 x 257              9.6 / 5.4 / 4.5 /  12 /   - / 5.9 / 5.1 / 4.5
+  //   f64  331 x 257, 8 shots    17.4 /  15 /  21 /  70 /   - /  11 /  12 /  14
+  //   f64  1000 x 1000           20.8 /  20 /  30 / 110 /   - /  15 /  17 /  21
+  //   f64  1000 x 700, 8 shots     86 /  97 / 151 /   - /   - /  71 /  78 / 102
+  // Adjoint with replay (forward as chosen above): tile / 2 / 3 / 4 levels
+  //   f32  701 x 403             15.8 /  14 /  11 / 9.8   (5: 9.0)
+  //   f32  2000 x 800, 32 shots   864 / 830 / 751 / 746
+  //   f64  331 x 257             17.2 /  12 /  10 / 9.1
+  //   f64  1000 x 1000             47 /  38 /  41 /  53
+  //   f64  1000 x 700, 8 shots    202 / 201 / 207 / 273
+  int choose_steps(const char *env, bool adj) const {
     if (const char *v = std::getenv(env)) {
       const int t = std::atoi(v);
-      return t > 500 && t <= 500 + NMAX ? t : 0;
+      return (t / 10 == 50 || (t / 10 == 51 && !adj)) && t % 10 >= 1 && t % 10 <= NMAX ? t : 0;
     }
-    for (int n = sizeof(T) == 4 ? 6 : 4; n > 3; n--)
-      if (stepn_blocks(n) <= 256) return 500 + n;
-    if (sizeof(T) == 4 || stepn_blocks(3) <= 1024) return 503;
-    return stepn_blocks(2) <= 3072 ? 502 : 0;
+    const bool f32 = sizeof(T) == 4;
+    for (int n = f32 ? 6 : 4; n > 3; n--)
+      if (stepn_blocks(0, n) <= 256) return 500 + n;
+    if (!adj) return f32 ? 514 : 513;
+    if (f32 || stepn_blocks(2, 3) <= 1024) return 503;
+    return stepn_blocks(2, 2) <= 3072 ? 502 : 0;
   }
 
   // Tuner candidates: the 2-D tile heights 8/16/32 as an interior-tile launch

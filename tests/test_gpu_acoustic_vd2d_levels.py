@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 
 
 def _run(monkeypatch, tile, dtype, n, halo, nts, nrec, cf, seed):
-    for name in ("SWX_VD2D_TILE_FWD", "SWX_VD2D_TILE_ADJ"):
+    for name in ("SWX_VD2D_TILE_FWD", "SWX_VD2D_TILE_ADJ"):      # 51n: forward only
         if tile is None:
             monkeypatch.delenv(name, raising=False)
         else:
@@ -52,7 +52,7 @@ def test_levels_per_launch_agree_bitwise(monkeypatch, dtype, n, halo, nts, nrec)
     args = (dtype, n, halo, nts, nrec, 13, 5 + n[0])
     ref = _run(monkeypatch, 316, *args)
     assert all(np.max(np.abs(v)) > 0 for v in ref[0].values()) and all(np.max(np.abs(s)) > 0 for s in ref[2])
-    for tile in [None, 501, 502, 503, 505] + ([508] if dtype == np.float32 else []):
+    for tile in [None, 501, 502, 503, 505, 511, 512, 515] + ([508, 518] if dtype == np.float32 else []):
         print(f"[vd2d levels {tile} {np.dtype(dtype).name} {n} halo {halo} nrec {nrec}]", flush=True)
         g, mis, seis, snaps = _run(monkeypatch, tile, *args)
         assert mis == ref[1] and all(np.array_equal(g[k], ref[0][k]) for k in ref[0])
