@@ -2145,7 +2145,8 @@ class Vd2dEngine final : public Engine {
   void forward(bool save) override {
     SWX_REQUIRE(model_set_, SWX_ESTATE, "swx_set_model must be called before running");
     zero(st_);
-    if (!tz_fwd_ || is_stepn(tz_fwd_)) tz_fwd_ = choose_steps("SWX_VD2D_TILE_FWD", false);
+    if (const int n = choose_steps("SWX_VD2D_TILE_FWD", false)) tz_fwd_ = n;
+    else if (is_stepn(tz_fwd_)) tz_fwd_ = 0;
     if (!tz_fwd_) {
       const Vd2dArgs<T> a1 = fwd_args(1, 0, save && c_.d.gradient ? 1 : 0, 0, c_.pts.d_traces.as<T>());
       tz_fwd_ = tune("SWX_VD2D_TILE_FWD",
@@ -2171,7 +2172,8 @@ class Vd2dEngine final : public Engine {
 
   void adjoint(bool per_shot) override {
     const int Kmax = (int)ceil_div(ntmax_, S_);
-    if (!tz_adj_ || is_stepn(tz_adj_)) tz_adj_ = choose_steps("SWX_VD2D_TILE_ADJ", true);
+    if (const int n = choose_steps("SWX_VD2D_TILE_ADJ", true)) tz_adj_ = n;
+    else if (is_stepn(tz_adj_)) tz_adj_ = 0;
     if (!tz_adj_) {
       // timed on a step every shot takes part in (the shortest shot's last
       // step); the history slots it reads are in range, their contents do

@@ -2630,32 +2630,34 @@ class El2dEngine final : public Engine {
         SWX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, el_row_kernel<T, true>, TX * ER_W, 0));
       else
         SWX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, el_row_kernel<T, false>, TX * ER_W, 0));
-      std::vector<int4> slow, rest;
+      // chunks of len rows at base length ch
+      auto chunks = [&](int ch, int len, int x, int z) {
+        return len > 0 ? (int)ceil_div(len, pin ? ch : std::max((int)((ch + 4) / COST[x][z]) - 4, 3)) : 0;
+      };
+      // row ranges: top and bottom strips, between them; or all in strips
+      const bool inner = zb > za;
+      const int range[3][3] = {{1, inner ? za : nz_ + 1, 1}, {inner ? zb : 0, inner ? nz_ + 1 : 0, 1},
+                               {inner ? za : 0, inner ? zb : 0, 0}};
+      int nxs = 0;
+      for (int bx = 0; bx < nbx; bx++) nxs += xs(bx);
       const int most = pin ? std::clamp(std::atoi(pin), 1, ER_ROWS) : adj ? 24 : 40;
-      for (int ch = pin ? most : adj ? 12 : 16; ch <= most; ch++) {
-        slow.clear();
-        rest.clear();
-        // rows [r0, r1) of every window, by the strips they are in
-        auto add = [&](int r0, int r1, bool z) {
-          for (int x = 0; x < 2; x++) {
-            const int c = pin ? ch : std::max((int)((ch + 4) / COST[x][z]) - 4, 3);
-            const int n = r1 > r0 ? (int)ceil_div(r1 - r0, c) : 0;
-            for (int k = 0; k < n; k++)
-              for (int bx = 0; bx < nbx; bx++)
-                if (xs(bx) == (x != 0))
-                  (x || z ? slow : rest).push_back({bx, r0 + (int)((int64_t)(r1 - r0) * k / n),
-                                                    r0 + (int)((int64_t)(r1 - r0) * (k + 1) / n), 2 * x + z});
-          }
-        };
-        if (zb > za) {
-          add(1, za, true);
-          add(zb, nz_ + 1, true);
-          add(za, zb, false);
-        } else {
-          add(1, nz_ + 1, true);
-        }
-        if ((int64_t)(slow.size() + rest.size()) * nshots <= (int64_t)per_cu * ER_W * cus) break;
+      int ch = pin ? most : adj ? 12 : 16;
+      for (; ch < most; ch++) {
+        int64_t n = 0;
+        for (const auto &r : range)
+          n += (int64_t)nxs * chunks(ch, r[1] - r[0], 1, r[2]) + (int64_t)(nbx - nxs) * chunks(ch, r[1] - r[0], 0, r[2]);
+        if (n * nshots <= (int64_t)per_cu * ER_W * cus) break;
       }
+      std::vector<int4> slow, rest;
+      for (const auto &r : range)
+        for (int x = 0; x < 2; x++) {
+          const int len = r[1] - r[0], n = chunks(ch, len, x, r[2]);
+          for (int k = 0; k < n; k++)
+            for (int bx = 0; bx < nbx; bx++)
+              if (xs(bx) == (x != 0))
+                (x || r[2] ? slow : rest).push_back({bx, r[0] + (int)((int64_t)len * k / n),
+                                                     r[0] + (int)((int64_t)len * (k + 1) / n), 2 * x + r[2]});
+        }
       // the corners' tiles first
       std::stable_sort(slow.begin(), slow.end(), [](const int4 &p, const int4 &q) {
         return COST[p.w >> 1][p.w & 1] > COST[q.w >> 1][q.w & 1];
