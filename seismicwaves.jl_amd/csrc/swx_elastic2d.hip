@@ -1631,7 +1631,7 @@ __global__ void el_record_kernel(const T *u, int64_t N, TapView<T> r0, TapView<T
 // precision the adjoint's registers (one wave per SIMD).
 constexpr int ER_OWN = 58, ER_W = 4;      // columns per window, waves per block
 constexpr int ER_ROWS = 56;               // most rows per chunk (64 lanes hold the coefficients of the rows loaded)
-constexpr int ER_TAPS = 128;              // most moment-tensor taps per wave
+constexpr int ER_TAPS = 256;              // most moment-tensor taps per wave (two sources of 8 x 8 taps per stress grid)
 
 template <typename T>
 struct ElRow {
