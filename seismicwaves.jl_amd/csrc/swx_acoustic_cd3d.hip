@@ -606,7 +606,7 @@ __global__ __launch_bounds__(TX *TY) void cd3d_step_kernel(Cd3dArgs<T> a) {
 // float64 47 / 28 and 49 / 39; 300 x 280 x 200 float32 199 / 123 and 217 / 184;
 // 600 x 600 x 400 float32 1009 / 812 (4.2 TB/s of the 24 bytes per cell that
 // it cannot do without) and 1307 / 1315.  What bounds the march at 300 x 280 x
-// 200: 0.5 of the wave cycles wait on memory at 4 waves per SIMD, the address
+// 200 (counters of its form without the LDS exchange): 0.5 of the wave cycles wait on memory at 4 waves per SIMD, the address
 // units are busy 0.65 of the time (rows start at any alignment, so that a
 // window touches three cache lines instead of two), and a quarter of the cells
 // have strips to step besides.
