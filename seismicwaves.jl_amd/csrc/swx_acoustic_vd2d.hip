@@ -869,7 +869,7 @@ __global__ __launch_bounds__(NB) void vd2d_fwd2_kernel(Vd2dArgs<T> a) {
 //
 // Bound by latency on small grids (701 x 403 float32: 19 us for 5 levels, 9.7 us
 // for one of the tile steps) and by instruction issue on large ones, where the
-// windows step 1.7 (6 x 16 rows, 4 levels: 2.1) times the owned cells: 1000 x
+// windows step 2.1 times the owned cells (96 rows, 4 levels): 1000 x
 // 700, 8 shots float32 49 -> 33 us per level; 2000 x 800, 32 shots 349 -> 270.
 // The adjoint keeps the three gradients of its cells in registers too and
 // reads one history level per level: 701 x 403 10.9 -> 5.1 us, 2000 x 800, 32
