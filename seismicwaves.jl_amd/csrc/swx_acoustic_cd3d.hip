@@ -33,6 +33,7 @@
 
 #include "swx_device.hpp"
 #include "swx_internal.hpp"
+#include "swx_planes.hpp"
 
 namespace swx {
 namespace {
@@ -69,13 +70,6 @@ __device__ __forceinline__ int xcd_tile3(int b, int nb) {
   const int per = nb >> 3;
   if (b >= per * 8) return b;
   return (b & 7) * per + (b >> 3);
-}
-
-// strip index of the cell owning psi along an axis of size n (or -1)
-__device__ __forceinline__ int psi_owner(int i, int n, int h) {
-  if (i < h) return i;
-  if (i >= n - h - 1 && i <= n - 2) return i + 1 - n + 2 * h;
-  return -1;
 }
 
 // Interior column tile of the 3D step (cd3d_is_lean): no x/y C-PML strip or
@@ -716,7 +710,7 @@ __device__ __forceinline__ void cd3d_row_march(const Cd3dArgs<T> &a, int s, Cd3d
   const unsigned ppx = (unsigned)ny * (2 * h) * E, pxx = (unsigned)ny * (2 * h + 2) * E;
   const unsigned ppy = (unsigned)nx * (2 * h) * E, pxy = (unsigned)nx * (2 * h + 2) * E;
   const unsigned opy0 = w == 0 && ky > 0 ? oy - nx * E : 0, kpy0 = w == 0 && ky > 0 ? ppy : 0;
-  auto zentry = [&](int k) { return (unsigned)(k < h ? k : k + 1 - nz + 2 * h); };
+  auto zentry = [&](int k) { return (unsigned)z_entry(k, nz, h); };
   auto load = [&](int k_) {
     Cd3dPlane<T> q;
     const unsigned k = min(k_, nz - 1), kb = k * plane;
@@ -831,7 +825,7 @@ __device__ __forceinline__ void cd3d_row_march(const Cd3dArgs<T> &a, int s, Cd3d
     pm = pc;
   };
   // three plane buffers in turn: planes k+1 and k+2 are in flight while
-  // plane k is stepped
+  // plane k is stepped (the last ones are K1 .. K1 + RM_AHEAD - 1)
   Cd3dPlane<T> A = load(K0), B = load(K0 + 1);
   for (int k = K0; k < K1; k += 3) {
     const Cd3dPlane<T> C = load(k + 2);
@@ -910,7 +904,7 @@ __global__ __launch_bounds__(TX *RM_W) void cd3d_row_kernel(Cd3dArgs<T> a) {
   const int j = min(j0 + w, ny - 1);
   const bool own = j0 + w < ny && X0 + lane < nx && lane >= (bx ? 1 : 0) && lane < (bx < a.nbx - 1 ? TX - 1 : TX);
   const int K0 = bk * a.kch, K1 = min(K0 + a.kch, nz);
-  // planes of the chunk (at most 64) with points on the row
+  // planes of the chunk (at most RM_PLANES) with points on the row
   uint64_t points;
   {
     const int64_t ro = (int64_t)s * (a.pt.nrows + 1) + j + (int64_t)ny * min(K0 + lane, nz - 1);
@@ -1087,7 +1081,7 @@ class Cd3dEngine final : public Engine {
   int64_t bytes_checkpoints() const override { return ck_.bytes(); }
   int64_t bytes_replay() const override { return dbuf_.bytes(); }
   int segment() const override { return S_; }
-  void variants(int32_t v[2]) const override { v[0] = variant_; v[1] = kch_; }
+  void variants(int32_t v[2]) const override { v[0] = variant_; v[1] = planes(); }
 
  private:
   int64_t strip(int ax, int w) const {
@@ -1151,15 +1145,15 @@ class Cd3dEngine final : public Engine {
     }
   }
 
-  // blocks of one chunk of the row march, planes per chunk (64: the march's
-  // plane masks)
+  // planes per chunk of a launch, blocks of one chunk of the row march
+  int planes() const { return variant_ == 301 ? std::min(kch_, RM_PLANES) : kch_; }
   int64_t row_columns() const {
     return std::max<int64_t>(ceil_div(n_[0] - 2, TX - 2), 1) * ceil_div(n_[1], RM_W) * nsh_;
   }
   void launch_rows(Cd3dArgs<T> a) {
     a.nbx = (int)std::max<int64_t>(ceil_div(n_[0] - 2, TX - 2), 1);
     a.nby = (int)ceil_div(n_[1], RM_W);
-    a.kch = std::min(a.kch, 64);
+    a.kch = std::min(a.kch, RM_PLANES);
     a.nbk = (int)ceil_div(n_[2], a.kch);
     const unsigned nb = (unsigned)(row_columns() * a.nbk);
     if (a.corr) cd3d_row_kernel<T, true><<<nb, TX * RM_W, 0, c_.stream>>>(a);
