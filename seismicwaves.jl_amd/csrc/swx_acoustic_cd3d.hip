@@ -950,6 +950,19 @@ class Cd3dEngine final : public Engine {
       sxi_[ax] = strip(ax, 2 * h_ + 2);
     }
     cstride_ = 3 * (8 * h_ + 4);
+    // launch shape: 8 / 4 / 2 = one launch with 64 x 8 / 64 x 4 / 64 x 2
+    // tiles, 108 / 104 / 102 = interior tiles and the others in two launches,
+    // 208 / 204 / 202 = one launch with the LDS-staged interior march,
+    // 301 = row march
+    if (const char *v = std::getenv("SWX_CD3D_VARIANT")) {
+      const int c = std::atoi(v);
+      SWX_REQUIRE(((c % 100 == 8 || c % 100 == 4 || c % 100 == 2) && c > 0 && c < 300) || c == 301, SWX_EINVAL,
+                  "SWX_CD3D_VARIANT must be 8, 4, 2, 108, 104, 102, 208, 204, 202 or 301");
+      SWX_REQUIRE(c != 301 || rows_reach(), SWX_EINVAL,
+                  "SWX_CD3D_VARIANT=301: the row march takes fields below 4 GiB per shot");
+      variant_ = c;
+      variant_env_ = true;
+    }
     const int64_t e = sizeof(T);
     fact_.alloc(N_ * e);
     p_.alloc(3 * ns_ * N_ * e);
@@ -989,17 +1002,6 @@ class Cd3dEngine final : public Engine {
       kch_env_ = true;
     }
     if (const char *v = std::getenv("SWX_CD3D_LEAN")) lean_ = std::atoi(v) != 0;
-    // launch shape: 8 / 4 / 2 = one launch with 64 x 8 / 64 x 4 / 64 x 2
-    // tiles, 108 / 104 / 102 = interior tiles and the others in two launches,
-    // 208 / 204 / 202 = one launch with the LDS-staged interior march,
-    // 301 = row march
-    if (const char *v = std::getenv("SWX_CD3D_VARIANT")) {
-      const int c = std::atoi(v);
-      SWX_REQUIRE(((c % 100 == 8 || c % 100 == 4 || c % 100 == 2) && c > 0 && c < 300) || c == 301, SWX_EINVAL,
-                  "SWX_CD3D_VARIANT must be 8, 4, 2, 108, 104, 102, 208, 204, 202 or 301");
-      variant_ = c;
-      variant_env_ = true;
-    }
     zero_forward_state();
   }
 
@@ -1150,6 +1152,11 @@ class Cd3dEngine final : public Engine {
   int64_t row_columns() const {
     return std::max<int64_t>(ceil_div(n_[0] - 2, TX - 2), 1) * ceil_div(n_[1], RM_W) * nsh_;
   }
+  // do the march's 32-bit byte offsets reach over a shot's arrays?
+  bool rows_reach() const {
+    const int64_t widest = std::max({N_, sps_[0], sps_[1], sps_[2], sxi_[0], sxi_[1], sxi_[2]});
+    return widest * (int64_t)sizeof(T) < (int64_t(1) << 32);
+  }
   void launch_rows(Cd3dArgs<T> a) {
     a.nbx = (int)std::max<int64_t>(ceil_div(n_[0] - 2, TX - 2), 1);
     a.nby = (int)ceil_div(n_[1], RM_W);
@@ -1190,9 +1197,7 @@ class Cd3dEngine final : public Engine {
   // 24: fewer blocks to fill the last round; 300 x 280 x 200 float32 127, 123
   // and 128 us with 8, 12 and 24).
   void choose_shape(bool save, T *tr) {
-    const int64_t widest = std::max({N_, sps_[0], sps_[1], sps_[2], sxi_[0], sxi_[1], sxi_[2]});
-    const bool reach = widest * (int64_t)sizeof(T) < (int64_t(1) << 32);
-    if (!variant_env_ && reach) variant_ = 301;
+    if (!variant_env_ && rows_reach()) variant_ = 301;
     if (variant_ != 301) {
       if (!tuned_) tune_shape(save, tr);
     } else if (!kch_env_) {
