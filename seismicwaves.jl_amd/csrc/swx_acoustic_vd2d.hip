@@ -2247,7 +2247,7 @@ class Vd2dEngine final : public Engine {
   int64_t bytes_checkpoints() const override { return ck_.bytes(); }
   int64_t bytes_replay() const override { return pbuf_.bytes(); }
   int segment() const override { return S_; }
-  void variants(int32_t v[2]) const override { v[0] = tz_fwd_; v[1] = tz_adj_; }
+  void variants(int32_t v[2]) const override { v[0] = used(tz_fwd_); v[1] = used(tz_adj_); }
 
   // "pcur" and "vcur" = [vx, vz] (acou_forward.jl:116-120): level it is in
   // parity slot(it) right after its step
@@ -2289,6 +2289,11 @@ class Vd2dEngine final : public Engine {
       if (nsh_ % (1 << k) == 0 && nsh_ > (1 << k)) v.push_back(code + 1000 * k);
     return v;
   }
+
+  // A tile code as the batch in hand takes it: a code chosen for another batch
+  // may group the shots by a number that does not divide this one, and
+  // vd2d_tile_of would then send blocks to a shot beyond it.
+  int used(int code) const { return nsh_ % (1 << (code / 1000)) ? code % 1000 : code; }
 
   Vd2dArgs<T> args(const DevBuf *b, int it, int rpar, int wpar) const {
     Vd2dArgs<T> a{};
@@ -2341,7 +2346,7 @@ class Vd2dEngine final : public Engine {
   // Thousands of a 2-D tile code give the shot groups of the block order
   // (vd2d_tile_of): code + 1000 k takes groups of 2^k shots.
   void launch_fwd(Vd2dArgs<T> a, int tz) {
-    a.sgrp = 1 << (tz / 1000);
+    a.sgrp = 1 << (used(tz) / 1000);
     tz %= 1000;
     if (tz == 102 || tz == 104) {
       const unsigned g = grid_march(a, tz - 100);
@@ -2409,7 +2414,7 @@ class Vd2dEngine final : public Engine {
     else launch_shape<0, false>(a, n);
   }
   void launch_adj(Vd2dArgs<T> a, int tz) {
-    a.sgrp = 1 << (tz / 1000);
+    a.sgrp = 1 << (used(tz) / 1000);
     tz %= 1000;
     if (tz == 102 || tz == 104) {
       const unsigned g = grid_march(a, tz - 100);
