@@ -1019,7 +1019,9 @@ __global__ __launch_bounds__(NW *TX, NW / 4) void vd2d_stepn_kernel(Vd2dArgs<T> 
   }
   const int64_t so = (int64_t)s * a.N;
   const bool xs = X0 <= max(h, 1) || X0 + TX - 1 >= nx - h - 1;
-  const bool zs = W.j0 <= max(h, 1) || W.j0 + R - 1 >= nz - h - 1;
+  // (without strips too, two rows before the last one: the correlation reads
+  // the pressure two rows on, zero beyond the grid)
+  const bool zs = W.j0 <= max(h, 1) || W.j0 + R - 1 >= nz - max(h, 1) - 1;
   // strip entries of the column: pressure (xi), velocity (psi)
   const bool xst = W.i >= 1 && W.i <= nx - 2 && (W.i <= h || W.i >= nx - h - 1);
   const bool pst = W.i < h || (W.i >= nx - h - 1 && W.i <= nx - 2);
