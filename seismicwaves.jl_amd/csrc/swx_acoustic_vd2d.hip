@@ -2147,14 +2147,14 @@ class Vd2dEngine final : public Engine {
   void forward(bool save) override {
     SWX_REQUIRE(model_set_, SWX_ESTATE, "swx_set_model must be called before running");
     zero(st_);
-    if (const int n = choose_steps("SWX_VD2D_TILE_FWD", false)) tz_fwd_ = n;
-    else if (is_stepn(tz_fwd_)) tz_fwd_ = 0;
-    if (!tz_fwd_) {
+    tz_fwd_ = choose_steps("SWX_VD2D_TILE_FWD", false);
+    if (!tz_fwd_ && !tile_fwd_) {
       const Vd2dArgs<T> a1 = fwd_args(1, 0, save && c_.d.gradient ? 1 : 0, 0, c_.pts.d_traces.as<T>());
-      tz_fwd_ = tune("SWX_VD2D_TILE_FWD",
-                     candidates({8, 16, Tiles<T>::fwd_max, 308, 316, 300 + Tiles<T>::fwd_max}),
-                     [&](int tz) { launch_fwd(a1, tz); });
+      tile_fwd_ = tune("SWX_VD2D_TILE_FWD",
+                       candidates({8, 16, Tiles<T>::fwd_max, 308, 316, 300 + Tiles<T>::fwd_max}),
+                       [&](int tz) { launch_fwd(a1, tz); });
     }
+    if (!tz_fwd_) tz_fwd_ = tile_fwd_;
     for (int it = 1; it <= ntmax_;) {
       progress("forward step", it, ntmax_);
       // a launch of several steps never steps over a checkpoint or snapshot level
@@ -2174,16 +2174,16 @@ class Vd2dEngine final : public Engine {
 
   void adjoint(bool per_shot) override {
     const int Kmax = (int)ceil_div(ntmax_, S_);
-    if (const int n = choose_steps("SWX_VD2D_TILE_ADJ", true)) tz_adj_ = n;
-    else if (is_stepn(tz_adj_)) tz_adj_ = 0;
-    if (!tz_adj_) {
+    tz_adj_ = choose_steps("SWX_VD2D_TILE_ADJ", true);
+    if (!tz_adj_ && !tile_adj_) {
       // timed on a step every shot takes part in (the shortest shot's last
       // step); the history slots it reads are in range, their contents do
       // not matter, and the adjoint state and gradients are cleared below
       const int itt = *std::min_element(nt_.begin(), nt_.end());
       const Vd2dArgs<T> a1 = adj_args(itt, ((itt - 1) / S_) * S_);
-      tz_adj_ = tune("SWX_VD2D_TILE_ADJ", candidates({16, 316}), [&](int tz) { launch_adj(a1, tz); });
+      tile_adj_ = tune("SWX_VD2D_TILE_ADJ", candidates({16, 316}), [&](int tz) { launch_adj(a1, tz); });
     }
+    if (!tz_adj_) tz_adj_ = tile_adj_;
     zero(ad_);
     SWX_HIP(hipMemsetAsync(grad_.get(), 0, grad_.bytes(), c_.stream));
     const int64_t F = (int64_t)ns_ * N_;
@@ -2568,6 +2568,7 @@ class Vd2dEngine final : public Engine {
   template <typename F>
   int fastest(const std::vector<int> &cands, F launch) {
     if (cands.size() == 1) return cands.front();
+    progress("launch shapes timed", 1, 1);
     hipEvent_t e0, e1;
     SWX_HIP(hipEventCreate(&e0));
     SWX_HIP(hipEventCreate(&e1));
@@ -2593,7 +2594,8 @@ class Vd2dEngine final : public Engine {
     (void)hipEventDestroy(e1);
     return best;
   }
-  int tz_fwd_ = 0, tz_adj_ = 0;
+  int tz_fwd_ = 0, tz_adj_ = 0;          // codes of the batch in hand
+  int tile_fwd_ = 0, tile_adj_ = 0;      // timed once per plan, kept through batches that take several levels
   int flip_ = 0, aflip_ = 0;
 
   // checkpoint k (k = 1 .. floor(nt_max/S), all shots): p, vx, vz, psi_x,
