@@ -2352,16 +2352,16 @@ class El2dEngine final : public Engine {
     nt_ = pt.nt;
     ntmax_ = *std::max_element(nt_.begin(), nt_.end());
     for (int k = 0; k < 2; k++) max_ucell_[k] = std::max(taps_[2 * k].max_ucell, taps_[2 * k + 1].max_ucell);
-    const bool was = rows_ok_;
     choose_rows(nshots, nsrc.data(), shots);
-    if (rows_ok_ != was) var_fwd_ = var_adj_ = -1;
   }
 
   void forward(bool save) override {
     SWX_REQUIRE(model_set_, SWX_ESTATE, "swx_set_model must be called before running");
+    var_fwd_ = choose_variant("SWX_EL2D_VARIANT_FWD");
     if (var_fwd_ < 0) {
       // tuning launches run on the state before it is cleared below
-      var_fwd_ = tune("SWX_EL2D_VARIANT_FWD", [&](int v) { step_fwd_v(v, 1, 0, 0, 0, nullptr); });
+      if (tuned_fwd_ < 0) tuned_fwd_ = tune([&](int v) { step_fwd_v(v, 1, 0, 0, 0, nullptr); });
+      var_fwd_ = tuned_fwd_;
     }
     zero_forward_state(true);
     if (save) SWX_HIP(hipMemsetAsync(hist_.get(), 0, hist_.bytes(), c_.stream));
@@ -2394,15 +2394,17 @@ class El2dEngine final : public Engine {
   }
 
   void adjoint(bool per_shot) override {
-    if (var_adj_ < 0) {
+    var_adj_ = choose_variant("SWX_EL2D_VARIANT_ADJ");
+    if (var_adj_ < 0 && tuned_adj_ < 0) {
       // timed on a step of the last segment that correlates (its stress
       // launch correlates the step after it), so the candidates are timed
       // with the correlation's loads and stores; the history slots it reads
       // are in range, and the adjoint state and gradients are cleared below
       const int cbt = (int)(ceil_div(ntmax_, S_) - 1) * S_;
       const int itt = ntmax_ - 1 > cbt ? ntmax_ - 1 : ntmax_;
-      var_adj_ = tune("SWX_EL2D_VARIANT_ADJ", [&](int v) { step_adj_v(v, itt, cbt); });
+      tuned_adj_ = tune([&](int v) { step_adj_v(v, itt, cbt); });
     }
+    if (var_adj_ < 0) var_adj_ = tuned_adj_;
     SWX_HIP(hipMemsetAsync(au_.get(), 0, au_.bytes(), c_.stream));
     SWX_HIP(hipMemsetAsync(asig_.get(), 0, asig_.bytes(), c_.stream));
     SWX_HIP(hipMemsetAsync(apsi_.get(), 0, apsi_.bytes(), c_.stream));
@@ -2717,22 +2719,21 @@ class El2dEngine final : public Engine {
   // blocks in one launch each, 2 = both steps in one launch on 64 x R tiles
   // with the stresses in LDS, 102/104 = one z-marching launch on 128/256-
   // column strips, 3 = the row march.  3 is taken where choose_rows allows it;
-  // elsewhere the tuner times 0, 1 and 2, and the z-marching variants when
-  // kMarchInTuner is set.  The environment can pin any.
+  // elsewhere (-1) the tuner times 0, 1 and 2, and the z-marching variants when
+  // kMarchInTuner is set, once per plan.  The environment can pin any.
+  int choose_variant(const char *env) const {
+    const char *v = std::getenv(env);
+    if (!v) return rows_ok_ ? 3 : -1;
+    const int t = std::atoi(v);
+    return t == 0 || t == 1 || t == 2 || t == 102 || t == 104 || (t == 3 && rows_ok_) ? t : -1;
+  }
   static constexpr bool kMarchInTuner = false;
   template <typename F>
-  int tune(const char *env, F step) {
+  int tune(F step) {
     std::vector<int> cands = {0, 1, 2};
     if (kMarchInTuner) {
       cands.push_back(102);
       cands.push_back(104);
-    }
-    if (const char *v = std::getenv(env)) {
-      const int t = std::atoi(v);
-      if (t == 0 || t == 1 || t == 2 || t == 102 || t == 104) return t;
-      if (t == 3 && rows_ok_) return t;
-    } else if (rows_ok_) {
-      return 3;
     }
     return cands[fastest_candidate(c_.stream, (int)cands.size(), [&](int k) { step(cands[k]); })];
   }
@@ -2903,7 +2904,8 @@ class El2dEngine final : public Engine {
   DevBuf tiles_[2];                // of the row march, forward and adjoint
   int ntiles_[2] = {0, 0}, nslow_[2] = {0, 0};
   bool rows_ok_ = false;
-  int var_fwd_ = -1, var_adj_ = -1;
+  int var_fwd_ = -1, var_adj_ = -1;        // variants of the batch in hand
+  int tuned_fwd_ = -1, tuned_adj_ = -1;    // timed ones, kept through batches that take the row march
   // XCD-aware tile map of the block launches (env SWX_EL2D_XCD=0 turns it off)
   bool xcd_ = [] {
     const char *v = std::getenv("SWX_EL2D_XCD");

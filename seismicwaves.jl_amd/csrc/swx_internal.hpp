@@ -302,6 +302,7 @@ int choose_segment(int nt_max, int check_freq, int64_t slot_bytes, int64_t ckpt_
 template <typename F>
 int fastest_candidate(hipStream_t stream, int n, F launch) {
   if (n <= 1) return 0;
+  progress("launch shapes timed", 1, 1);
   hipEvent_t e0, e1;
   SWX_HIP(hipEventCreate(&e0));
   SWX_HIP(hipEventCreate(&e1));
