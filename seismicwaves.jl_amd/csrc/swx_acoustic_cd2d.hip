@@ -562,20 +562,8 @@ __global__ __launch_bounds__(NW *TX, sizeof(T) == 4 ? 4 : 2) void cd2d_stepn_ker
             dval[r] = interior ? dval[r] + inj : (before - T(2) * G.po[r]) + G.pc[r];
           }
         }
-        if (!ADJ && (W.rmask & W.rows) >> r & 1 && W.own) {
-          const int e = L.rec[W.w * R + r][W.lane];
-          T *tr = a.traces + otr + (l - 1);
-          if (e > 0) {
-#pragma clang loop unroll(disable)
-            for (int k = 0; k < e >> 8; k++) tr[(int64_t)nts * L.col[(e & 255) - 1 + k]] = G.pc[r];
-          } else if (e < 0) {
-            const int j = W.j0 + r;
-            const int u = find_point(a.pt.rrow, a.pt.urec_cell, a.pt.nrows, s, j, (int64_t)j * nx + W.i);
-#pragma clang loop unroll(disable)
-            for (int k = a.pt.urec_ptr[u]; k < a.pt.urec_ptr[u + 1]; k++)
-              tr[(int64_t)nts * a.pt.urec_list[k]] = G.pc[r];
-          }
-        }
+        if (!ADJ && (W.rmask & W.rows) >> r & 1 && W.own)
+          level_record<T, R>(a, L, W, nts, r, a.traces + otr + (l - 1), G.pc[r]);
       }
     }
     if constexpr (ADJ) {

@@ -1151,20 +1151,8 @@ __global__ __launch_bounds__(NW *TX, NW / 4) void vd2d_stepn_kernel(Vd2dArgs<T> 
         T inj = 0;
         level_inject<T, R, ADJ>(a, L, W, s, nts, r, m, l, G.m0[r], G.p[r], inj);
       }
-      if (!ADJ && (W.rmask & W.rows) >> r & 1 && W.own) {
-        const int e = L.rec[W.w * R + r][W.lane];
-        T *tr = a.traces + otr + (l - 1);
-        if (e > 0) {
-#pragma clang loop unroll(disable)
-          for (int k = 0; k < e >> 8; k++) tr[(int64_t)nts * L.col[(e & 255) - 1 + k]] = G.p[r];
-        } else if (e < 0) {
-          const int j = W.j0 + r;
-          const int u = find_point(a.pt.rrow, a.pt.urec_cell, a.pt.nrows, s, j, (int64_t)j * nx + W.i);
-#pragma clang loop unroll(disable)
-          for (int k = a.pt.urec_ptr[u]; k < a.pt.urec_ptr[u + 1]; k++)
-            tr[(int64_t)nts * a.pt.urec_list[k]] = G.p[r];
-        }
-      }
+      if (!ADJ && (W.rmask & W.rows) >> r & 1 && W.own)
+        level_record<T, R>(a, L, W, nts, r, a.traces + otr + (l - 1), G.p[r]);
     }
   };
   auto fresh = [&] {
