@@ -2632,10 +2632,15 @@ class El2dEngine final : public Engine {
   // them and starts first.  A corner's wave has at least 3 rows (a chunk steps
   // the stresses of 4 more), which gives an interior one 16 (12 in the adjoint);
   // chunks grow from there until the waves of the batch are resident at once,
-  // up to 40 (24) rows.  us per step with 16 / 24 / 40 / 56 rows, 1500 x 600, 12
-  // shots, float32: forward 102 / 95 / 88 / 91, adjoint 268 / 267 / 280 / 290;
+  // up to 40 rows (56); where that takes more, they go in several rounds of
+  // chunks of 40 (24) rows.  us per step with 16 / 24 / 40 / 56 rows, 1500 x 600,
+  // 12 shots, float32: forward 102 / 95 / 88 / 91, adjoint 268 / 267 / 280 / 290;
   // with the same 40 rows everywhere and in grid order 101 and 306.  813 x 407, 4
   // shots, forward: 22 with 16 rows, 25 with 40, 27 with 5 rows everywhere.
+  // Adjoint, float64 (one wave per SIMD), in one round against two of 24 rows:
+  // 124 x 101, 28 shots 36 / 54; 813 x 407, 4 shots 67 / 79; 1500 x 600, 2 shots 85
+  // / 96; float32, 1500 x 600, 4 shots 92 / 99.  (The forward ends at 40: longer
+  // chunks gather more sources' taps in a wave.)
   void choose_rows(int nshots, const int *nsrc, const swx_elastic_shot_desc *shots) {
     static constexpr double COST[2][2] = {{1.0, 2.3}, {1.5, 2.9}};      // [x strip][z strip]
     const int lo = std::max(3, h_ + 2), za = lo + 2, zb = std::min(nz_ - 2, nz_ - h_ - 2) - 1;
@@ -2665,13 +2670,17 @@ class El2dEngine final : public Engine {
                                {inner ? za : 0, inner ? zb : 0, 0}};
       int nxs = 0;
       for (int bx = 0; bx < nbx; bx++) nxs += xs(bx);
-      const int most = pin ? std::clamp(std::atoi(pin), 1, ER_ROWS) : adj ? 24 : 40;
-      int ch = pin ? most : adj ? 12 : 16;
-      for (; ch < most; ch++) {
+      const int several = adj ? 24 : 40, longest = adj ? ER_ROWS : 40;
+      int ch = pin ? std::clamp(std::atoi(pin), 1, ER_ROWS) : adj ? 12 : 16;
+      for (; !pin; ch++) {
         int64_t n = 0;
         for (const auto &r : range)
           n += (int64_t)nxs * chunks(ch, r[1] - r[0], 1, r[2]) + (int64_t)(nbx - nxs) * chunks(ch, r[1] - r[0], 0, r[2]);
         if (n * nshots <= (int64_t)per_cu * ER_W * cus) break;
+        if (ch == longest) {
+          ch = several;
+          break;
+        }
       }
       std::vector<int4> slow, rest;
       for (const auto &r : range)
