@@ -380,13 +380,13 @@ def alg_bytes(physics, n, halo, e, nts, S, variant=(0, 0)):
         else:
             # CD: r p^n, p^n-1, fact; w p^n+1 (4e); + w D (5e).  Adjoint with
             # the fused correlation: + r D, grad read-modify-write (7e).
-            if physics == "cd2d" and len(variant) > 1 and variant[1] > 22:
+            if physics == "cd2d" and _cd2d_levels(variant) > 1:
                 # n levels per launch: a launch reads p^n, p^n-1 and fact once
                 # (3e), writes the two last levels (2e) and the D of every
                 # stored level (1e); an adjoint launch also reads and writes
                 # the gradient (2e) and reads one history level per level.
                 # Launches end at multiples of S.
-                n = variant[1] % 10
+                n = _cd2d_levels(variant)
                 lf = sum(-(-(min((k + 1) * S, nt) - k * S) // n) for k in range(kl + 1))
                 lr = kl * -(-S // n)
                 fwd_b += (lf + lr) * (5 * e * N + strip) + (last + rep) * e * N
@@ -395,7 +395,8 @@ def alg_bytes(physics, n, halo, e, nts, S, variant=(0, 0)):
                 adj_n += lf
                 continue
             if physics == "cd2d" and len(variant) > 1 and variant[1] % 10 == 2:
-                # two levels per forward / replay launch: r p^n, p^n-1, fact
+                # two levels per forward / replay launch and one per adjoint
+                # launch, both levels written: r p^n, p^n-1, fact
                 # once per launch (3e), w each level (1e) and its D (1e);
                 # launches start at levels 1, 3, 5, ... of the forward and
                 # of every replayed segment
@@ -439,6 +440,12 @@ def alg_bytes(physics, n, halo, e, nts, S, variant=(0, 0)):
             for k in range(0, len(nts), ga):
                 adj_b += 3 * e * N * max(nts[k:k + ga])
     return {0: (fwd_b, fwd_n), 1: (adj_b, adj_n)}
+
+
+def _cd2d_levels(variant):
+    """Most levels per launch of a CD 2D plan, 0 if its variant does not say
+    (11 x levels: the same number in both directions)."""
+    return variant[1] // 11 if len(variant) > 1 and variant[1] % 11 == 0 else 0
 
 
 def kernel_names(physics, variant):
@@ -489,15 +496,12 @@ def kernel_names(physics, variant):
         return f"{k} (forward)", f"{k} (adjoint)"
     # [rows per thread or window shapes, levels per launch; each but the rows
     # 10 x adjoint + forward / replay]
-    if len(variant) > 1 and variant[1] > 22:
+    if _cd2d_levels(variant) > 1:
         shape = {0: "8, 8", 1: "4, 16", 2: "2, 16"}
         return (f"cd2d_stepn_kernel<float, {shape[variant[0] % 10]}, false> (forward)",
                 f"cd2d_stepn_kernel<float, {shape[variant[0] // 10]}, true> (adjoint)")
     k = f"cd2d_step_kernel<float, {variant[0] or 2}>"
-    two = variant[1] if len(variant) > 1 else 0
-    fwd = "cd2d_step2_kernel<float, false>" if two % 10 == 2 else k
-    adj = "cd2d_step2_kernel<float, true>" if two // 10 == 2 else k
-    return f"{fwd} (forward)", f"{adj} (adjoint)"
+    return f"{k} (forward)", f"{k} (adjoint)"
 
 
 def traffic_from_profiles(workload, kernel):
