@@ -301,15 +301,17 @@ __global__ __launch_bounds__(TX *TZ) void cd2d_step_kernel(Cd2dStepArgs<T> a) {
 // once.  Every cell update is spelled as in cd2d_cell, so the results are
 // bitwise those of n one-level launches.
 //
-// Bound by latency at small sizes (a launch of 8 levels of one 201 x 151 shot
-// takes 17 us: 5-7 us of loads, stores and launch, 1.3 us per level of barrier,
-// LDS round trip and the strip updates' chain) and by instruction issue at
-// large ones (about 20 vector instructions per cell and level, 1.5-1.8 times
-// the grid's cells).  us per level against the two-level LDS tiles this
-// replaces (one level per launch where that was faster):
-//   f32 201 x 151:        forward 5.1 -> 2.2, adjoint + replay   8.9 -> 3.7
-//   f32 1000 x 1000:      forward 7.9 -> 3.9, adjoint + replay  15.9 -> 7.2
-//   f64 12 x 397 x 253:   forward  15 -> 6.2, adjoint + replay    33 -> 13
+// Bound by latency: of the barrier, the LDS round trip and the strip updates'
+// chain of a level, and of a launch's loads and stores (one 201 x 151 shot:
+// 11.3 us per launch of 8 levels).  Counters, forward / adjoint: 1000 x 1000
+// float32 has 1.2 / 1.8 waves per SIMD, vector units issuing 0.22 of the time,
+// 1.5 / 2.5 TB/s; 4 x 2000 x 1000 has 3.0 / 3.2, 0.48 / 0.38 and 2.7 / 3.6 TB/s,
+// with 1.5-1.8 times the grid's cells stepped.  us per level against the
+// two-level LDS tiles this replaces (one level per launch where that was
+// faster):
+//   f32 201 x 151:        forward 5.1 -> 1.8, adjoint + replay   8.9 -> 3.2
+//   f32 1000 x 1000:      forward 7.9 -> 3.5, adjoint + replay  15.9 -> 7.6
+//   f64 12 x 397 x 253:   forward  15 -> 6.0, adjoint + replay    33 -> 15
 
 template <typename T>
 struct Cd2dStepNArgs {

@@ -600,10 +600,11 @@ __global__ __launch_bounds__(TX *TY) void cd3d_step_kernel(Cd3dArgs<T> a) {
 // float64 47 / 28 and 49 / 39; 300 x 280 x 200 float32 199 / 123 and 217 / 184;
 // 600 x 600 x 400 float32 1009 / 812 (4.2 TB/s of the 24 bytes per cell that
 // it cannot do without) and 1307 / 1315.  What bounds the march at 300 x 280 x
-// 200 (counters of its form without the LDS exchange): 0.5 of the wave cycles wait on memory at 4 waves per SIMD, the address
-// units are busy 0.65 of the time (rows start at any alignment, so that a
-// window touches three cache lines instead of two), and a quarter of the cells
-// have strips to step besides.
+// 200 (counters, forward with history / adjoint): 3.4 / 2.9 waves per SIMD that
+// wait for memory half of their cycles (rows start at any alignment, so that a
+// window touches three cache lines instead of two), 3.8 / 4.1 TB/s, vector
+// units issuing 0.34 / 0.30 of the time; at 600 x 600 x 400, 8 shots 5.2 / 5.3
+// TB/s, 0.85 of a triad's rate, 1.14 times the bytes of the owned cells.
 // Expressions are those of cd3d_step_kernel: results are bitwise the same.
 constexpr int RM_W = 2;      // rows (waves) per block
 
@@ -1186,11 +1187,12 @@ class Cd3dEngine final : public Engine {
   }
 
   // The row march, unless its 32-bit byte offsets do not reach over a shot's
-  // field (from 4 GiB on).  It is the faster one at every size: us per step,
-  // row march / best tile shape, forward with history and adjoint, 600 x 600 x 400 float32
-  // 812 / 1009 and 1315 / 1307, 400 x 400 x 300 float64 575 / 755 and 950 / 930,
-  // 300 x 280 x 200 float32 123 / 199 and 184 / 217, 129 x 117 x 91 float64
-  // 28 / 47 and 39 / 49.
+  // field (from 4 GiB on).  us per step, row march / best tile shape, forward
+  // with history and adjoint: 600 x 600 x 400 float32 812 / 1009 and 1315 / 1307,
+  // 400 x 400 x 300 float64 575 / 755 and 950 / 930, 300 x 280 x 200 float32 123 /
+  // 199 and 184 / 217, 129 x 117 x 91 float64 28 / 47 and 39 / 49.  (The adjoint
+  // gives up 1 and 2% at the two largest; a gradient takes one shape for both
+  // directions and its forward and replayed steps gain 20% and more.)
   // Planes per chunk: as few as still let every block of the grid be resident
   // at once, from 6 on; grids that need more than 12 take several
   // rounds anyway, and 12 is the best for them (8: more planes loaded twice,

@@ -867,13 +867,17 @@ __global__ __launch_bounds__(NB) void vd2d_fwd2_kernel(Vd2dArgs<T> a) {
 // values of the n levels are staged in LDS once.  Cell updates are spelled as
 // in vd2d_fwd_general_tile: results are bitwise those of n single steps.
 //
-// Bound by latency on small grids (701 x 403 float32: 19 us for 5 levels, 9.7 us
-// for one of the tile steps) and by instruction issue on large ones, where the
-// windows step 2.1 times the owned cells (96 rows, 4 levels): 1000 x
-// 700, 8 shots float32 49 -> 33 us per level; 2000 x 800, 32 shots 349 -> 270.
+// Bound by latency on small grids (701 x 403 float32: 18 us for 5 levels, 9.7 us
+// for one of the tile steps; 1.5 waves per SIMD) and by what the windows step
+// twice on large ones, 2.1 times the owned cells (96 rows, 4 levels): 1000 x
+// 700, 8 shots float32 49 -> 32 us per level; 2000 x 800, 32 shots 349 -> 254.
+// Counters there (64 shots), forward / adjoint: vector units issue 0.56 / 0.36
+// of the time at 3.5 / 1.8 waves per SIMD, 2.7 / 3.3 TB/s, 1.31 / 1.47 times the
+// bytes of the owned cells.
 // The adjoint keeps the three gradients of its cells in registers too and
 // reads one history level per level: 701 x 403 10.9 -> 5.1 us, 2000 x 800, 32
-// shots 585 -> 530 (8 x 8 rows; 601 with 4 x 16, where six registers spill).
+// shots 585 -> 474 (8 x 8 rows; 4 x 16, where six registers spill, takes 1.13
+// times as long).
 template <typename T, int R, int NW>
 struct Vd2dNLds : LevelPoints<T, NW * R> {
   T vz[3][NW][TX];             // rows R-2, R-1 and 0 of vz

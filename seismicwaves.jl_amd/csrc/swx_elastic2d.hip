@@ -1624,12 +1624,14 @@ __global__ void el_record_kernel(const T *u, int64_t N, TapView<T> r0, TapView<T
 // for a tile) it loads a row of u once per wave and recomputes 6 of 64 columns
 // and 4 rows per chunk.  us per step, tile / row march: 813 x 407, 4 shots,
 // float32, forward 45 / 22; 1500 x 600, 12 shots, float32, forward 130 / 88 and
-// adjoint 346 / 267; 331 x 257, 3 shots, float64, forward 34 / 19, adjoint 29 /
-// 28.  What bounds it: at 1500 x 600 memory (24 and 88 bytes per cell of fields,
-// history and gradients and 20 of the model, which the shots share in the last
-// cache: 5.4 and 4.4 TB/s with them); on small grids the corners' waves, which
-// issue three times the instructions of an interior one per row, and in double
-// precision the adjoint's registers (one wave per SIMD).
+// adjoint 346 / 267; 331 x 257, 3 shots, float64, forward 34 / 15, adjoint 29 /
+// 28.  What bounds it: at 1500 x 600 memory (16 shots, counters: 6.1 and 6.4 TB/s,
+// the rate of a triad, 1.24 and 1.42 times the bytes of the owned cells; 3.0
+// and 2.6 waves per SIMD, vector units issuing 0.27 and 0.20 of the time); on
+// small grids the latency of the corners' waves, which issue three times the
+// instructions of an interior one per row (331 x 257, 3 shots, float64: 0.3 and
+// 0.4 waves per SIMD), and in the double-precision adjoint of larger ones the
+// registers (one wave per SIMD).
 constexpr int ER_OWN = 58, ER_W = 4;      // columns per window, waves per block
 constexpr int ER_ROWS = 56;               // most rows per chunk (64 lanes hold the coefficients of the rows loaded)
 constexpr int ER_TAPS = 256;              // most moment-tensor taps per wave (two sources of 8 x 8 taps per stress grid)
