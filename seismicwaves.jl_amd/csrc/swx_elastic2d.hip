@@ -1647,25 +1647,27 @@ struct ElRow {
 // stresses), then f1 (shear)
 template <typename T>
 struct ElTaps {
-  uint64_t cols[2][64];                   // of a family and row of the chunk: columns with taps
-  int start[2][64], end[2];               // its first tap; end of a family's
-  uint64_t several;                       // rows with more than one tap on a cell
-  int key[ER_TAPS];                       // 64 * row of the chunk + lane
+  uint64_t cols[2][64];                   // of a family and row of the chunk: columns with taps,
+  int start[2][64];                       // its first cell
+  int first[ER_TAPS + 1];                 // first tap of a cell; their number after the last one
   T c0[ER_TAPS], c1[ER_TAPS], f[ER_TAPS];
 };
 
 // Taps of family t (SHEAR: f1), its entries [e0, e1) on rows jr .. jr+63, in
-// the columns X0 .. X0+63, listed in L from tap n on.  A source's wave is the
-// last one of a step on a small grid, so that its list is built from three
-// loads in a row (place and point of an entry, its time function) and a row
-// of the march finds a lane's tap by counting columns: 400 x 300, one source of
-// 8 x 8 taps per grid, float32, 12.6 us per replayed step, against 27.3 with a
-// search for each entry's cell and a walk along the taps of the row (the two
-// launches of el_stress_kernel and el_disp_kernel: about 17).
+// the columns X0 .. X0+63, listed in L from tap n and cell u on (both are
+// advanced).  A source's wave is the last one of a step on a small grid, so
+// that its list is built from three loads in a row (place and point of an
+// entry, its time function) and a row of the march finds a lane's taps by
+// counting columns, on cells with several of them too.  us per replayed step,
+// 400 x 300, float32, one source of 8 x 8 taps per grid / two of them two cells
+// apart: 13.4 / 14.9, against 27.2 / 42.5 with a search for each entry's cell and
+// a walk along the taps of the row (the two launches of el_stress_kernel and
+// el_disp_kernel: about 17).
 template <typename T, bool SHEAR>
-__device__ __forceinline__ int el_row_taps(const ElArgs<T> &a, const TapView<T> &t, int s, int nts, int jr, int X0,
-                                           int e0, int e1, ElTaps<T> &L, int n) {
+__device__ __forceinline__ void el_row_taps(const ElArgs<T> &a, const TapView<T> &t, int s, int nts, int jr, int X0,
+                                            int e0, int e1, ElTaps<T> &L, int &n, int &u) {
   const int lane = threadIdx.x & (TX - 1);
+  const uint64_t below = (uint64_t(1) << lane) - 1;
   const T *tf = a.tf + a.off_tf[s] + (a.it - 1);
   const T *M = a.mom + 3 * (int64_t)a.off_mom[s];
   int last = -1;                          // cell of the entry before
@@ -1675,42 +1677,42 @@ __device__ __forceinline__ int el_row_taps(const ElArgs<T> &a, const TapView<T> 
     const int p = t.epoint[e];
     const T x = t.ecoef[e];
     const int col = ij.x - X0, m = ij.y - jr, c = ij.y * a.nx + ij.x;
+    const int up = __shfl_up(c, 1);
     const bool in = eb + lane < e1 && col >= 0 && col < TX;
-    const uint64_t w = __ballot(in);
-    const int q = n + __builtin_popcountll(w & ((uint64_t(1) << lane) - 1));
-    const int up = __shfl_up(c, 1), before = lane ? up : last;
+    const bool head = in && c != (lane ? up : last);
+    const uint64_t w = __ballot(in), wh = __ballot(head);
+    const int q = n + __builtin_popcountll(w & below), v = u + __builtin_popcountll(wh & below);
     if (in && q < ER_TAPS) {
-      L.key[q] = m * TX + col;
       L.c0[q] = M[3 * p + (SHEAR ? 2 : 0)] * x;
       L.c1[q] = SHEAR ? T(0) : M[3 * p + 1] * x;
       L.f[q] = tf[(int64_t)nts * p];
-      atomicOr((unsigned long long *)&L.cols[SHEAR][m], 1ull << col);
-      atomicMin(&L.start[SHEAR][m], q);
-      if (c == before) atomicOr((unsigned long long *)&L.several, 1ull << m);
+      if (head) {
+        L.first[v] = q;
+        atomicOr((unsigned long long *)&L.cols[SHEAR][m], 1ull << col);
+        atomicMin(&L.start[SHEAR][m], v);
+      }
     }
     last = __shfl(c, TX - 1);
     n = min(n + __builtin_popcountll(w), ER_TAPS);
+    u = min(u + __builtin_popcountll(wh), ER_TAPS);
   }
-  return n;
 }
 
 // The lane's taps of row m: add(tap) in list order.
 template <typename T, typename F>
-__device__ __forceinline__ void el_row_add(const ElTaps<T> &L, int f, int m, bool several, int lane, F add) {
+__device__ __forceinline__ void el_row_add(const ElTaps<T> &L, int f, int m, int lane, F add) {
   const uint64_t w = L.cols[f][m];
-  const int t = L.start[f][m];
-  if (several) {
-    for (int k = t; k < L.end[f] && L.key[k] < (m + 1) * TX; k++)
-      if ((L.key[k] & (TX - 1)) == lane) add(k);
-  } else if (w >> lane & 1) {
-    add(t + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(w >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)w, 0)));
+  if (w >> lane & 1) {
+    const int u = L.start[f][m] +
+                  (int)__builtin_amdgcn_mbcnt_hi((unsigned)(w >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)w, 0));
+    for (int k = L.first[u]; k < L.first[u + 1]; k++) add(k);
   }
 }
 
 // XS: the window reaches a strip or a side; ZS: the chunk's rows do.
 template <typename T, bool XS, bool ZS, bool ADJ>
 __device__ __forceinline__ void el_row_march(const ElArgs<T> &a, int s, int nts, int X0, int Z0, int Z1, bool own,
-                                             const ElTaps<T> *L, uint64_t taps, uint64_t several) {
+                                             const ElTaps<T> *L, uint64_t taps) {
   constexpr unsigned E = sizeof(T);
   const int nx = a.nx, nz = a.nz, h = a.h;
   const int lane = threadIdx.x & (TX - 1), i = X0 + lane;
@@ -1906,12 +1908,11 @@ __device__ __forceinline__ void el_row_march(const ElArgs<T> &a, int s, int nts,
     T vxz = q.mh * (c1 + c2);
     if (!ADJ) {
       if (taps >> m & 1) {
-        const bool more = several >> m & 1;
-        el_row_add(*L, 0, m, more, lane, [&](int k) {
+        el_row_add(*L, 0, m, lane, [&](int k) {
           vxx += L->c0[k] * L->f[k];
           vzz += L->c1[k] * L->f[k];
         });
-        el_row_add(*L, 1, m, more, lane, [&](int k) { vxz += L->c0[k] * L->f[k]; });
+        el_row_add(*L, 1, m, lane, [&](int k) { vxz += L->c0[k] * L->f[k]; });
       }
     }
     if (XS || ZS) {
@@ -2063,7 +2064,7 @@ __global__ __launch_bounds__(TX *ER_W) void el_row_kernel(ElArgs<T> a) {
   const int nx = a.nx, nz = a.nz, h = a.h;
   const int bx = tile.x, X0 = bx * ER_OWN + 1, Z0 = tile.y, Z1 = tile.z;
   const bool own = X0 + lane <= nx && lane >= (bx ? 3 : 0) && lane < (bx < a.nbx_rows - 1 ? TX - 3 : TX);
-  uint64_t tap_rows = 0, several = 0;
+  uint64_t tap_rows = 0;
   if (!ADJ && a.kind == 1) {
     const int jr = Z0 - 2, j0 = max(jr, 1) - 1, j1 = min(Z1 + 1, nz);
     const int64_t o = (int64_t)s * (a.nrows + 1);
@@ -2073,13 +2074,13 @@ __global__ __launch_bounds__(TX *ER_W) void el_row_kernel(ElArgs<T> a) {
       const int e0 = a.f0.eptr[u0], e1 = a.f0.eptr[u1], g0 = a.f1.eptr[v0], g1 = a.f1.eptr[v1];
       L.cols[0][lane] = L.cols[1][lane] = 0;
       L.start[0][lane] = L.start[1][lane] = ER_TAPS;
-      L.several = 0;
       __builtin_amdgcn_wave_barrier();
-      L.end[0] = el_row_taps<T, false>(a, a.f0, s, nts, jr, X0, e0, e1, L, 0);
-      L.end[1] = el_row_taps<T, true>(a, a.f1, s, nts, jr, X0, g0, g1, L, L.end[0]);
+      int n = 0, u = 0;
+      el_row_taps<T, false>(a, a.f0, s, nts, jr, X0, e0, e1, L, n, u);
+      el_row_taps<T, true>(a, a.f1, s, nts, jr, X0, g0, g1, L, n, u);
+      L.first[u] = n;
       __builtin_amdgcn_wave_barrier();
       tap_rows = __ballot((L.cols[0][lane] | L.cols[1][lane]) != 0);
-      several = __ballot(L.several >> lane & 1);
     }
   }
   const bool corr = ADJ && a.corr_step > 0 && a.corr_step <= nts && a.corr_step <= a.corr_lim;
@@ -2088,8 +2089,8 @@ __global__ __launch_bounds__(TX *ER_W) void el_row_kernel(ElArgs<T> a) {
   const bool zs = Z0 - 2 < lo || Z1 + 1 > min(nz - 2, nz - h - 2);
   const ElTaps<T> *L = &taps[ADJ ? 0 : w];
   auto run = [&](auto xsc, auto zsc) {
-    if (ADJ && corr) el_row_march<T, xsc(), zsc(), true>(a, s, nts, X0, Z0, Z1, own, L, 0, 0);
-    else el_row_march<T, xsc(), zsc(), false>(a, s, nts, X0, Z0, Z1, own, L, tap_rows, several);
+    if (ADJ && corr) el_row_march<T, xsc(), zsc(), true>(a, s, nts, X0, Z0, Z1, own, L, 0);
+    else el_row_march<T, xsc(), zsc(), false>(a, s, nts, X0, Z0, Z1, own, L, tap_rows);
   };
   if (xs && zs) run(std::true_type{}, std::true_type{});
   else if (xs) run(std::true_type{}, std::false_type{});
