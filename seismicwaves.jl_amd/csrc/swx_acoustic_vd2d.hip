@@ -2503,6 +2503,12 @@ class Vd2dEngine final : public Engine {
   //   f64  331 x 257             17.2 /  12 /  10 / 9.1
   //   f64  1000 x 1000             47 /  38 /  41 /  53
   //   f64  1000 x 700, 8 shots    202 / 201 / 207 / 273
+  // Next to the two lines (910 and 1078 windows of 3 levels, 2660 and 3990 of 2;
+  // the second line lies a little before the last gain of two levels):
+  //   f64  600 x 500, 2 shots    35.2 / 27.5 / 27.3
+  //   f64  1000 x 700            36.5 / 30.0 / 31.5
+  //   f64  1000 x 700, 4 shots    110 / 105 / 107
+  //   f64  1000 x 700, 6 shots    158 / 154 / 156
   int choose_steps(const char *env, bool adj) const {
     if (const char *v = std::getenv(env)) {
       const int t = std::atoi(v);
